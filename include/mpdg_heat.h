@@ -137,14 +137,15 @@ int mpdg_heat_op_vmult_f32(const mpdg_heat_op *op, float *dst, const float *src,
 /* vmult that allocates nothing (no hipMalloc/hipFree, no allocating library call). No
    counterpart in the reference: it is for callers that cannot allocate device memory (code
    under HIP graph capture, tight serving loops, harnesses that forbid it). Same result as
-   mpdg_heat_op_vmult, bit for bit (same kernels). The apply's scratch -- the contributions to
-   the DoF rows where four columns of the launch meet -- is a fixed per-GPU array of 2^20
-   doubles (8 MiB) instead of the operator's lazily allocated buffer (entries needed: about
-   0.75 M for Q3 on 128^3 cells, 0.64 M for mapped Q3 on 96^3 cells, 0.27 M for Q4 on 96^3
-   cells); meshes that need more get MPDG_ERR_TOO_LARGE. FP64
-   operators only; a k(T) law on a mapped mesh needs one earlier mpdg_heat_op_vmult (which
-   sizes its rescaled metric), else MPDG_ERR_INVALID. All calls on one GPU share the array:
-   calls that overlap on one GPU race. */
+   mpdg_heat_op_vmult, bit for bit (same kernels). The apply's scratch is, for Q1..Q3, the
+   operator's own, allocated by mpdg_heat_op_create (MPDG_ERR_NOMEM when that had no room);
+   for Q4, a fixed per-GPU array of 2^20 doubles (8 MiB). Meshes beyond a fixed maximum get
+   MPDG_ERR_TOO_LARGE: more than 2^20 DoFs on the rows along x where four columns of cells
+   meet (about 0.75 M for Q3 on 128^3 cells, 0.64 M for mapped Q3 on 96^3 cells, 0.27 M for
+   Q4 on 96^3 cells; columns of 4 x 4, 3 x 2, 4 x 2, 4 x 3 cells in y, z for Q1..Q4, 2 x 2 for
+   mapped Q3). FP64 operators only; a k(T) law on a mapped mesh needs one earlier
+   mpdg_heat_op_vmult (which sizes its rescaled metric), else MPDG_ERR_INVALID. Q4 calls that
+   overlap on one GPU race, and so do overlapping calls of one operator. */
 int mpdg_heat_op_vmult_noalloc(const mpdg_heat_op *op, double *dst, const double *src, void *stream);
 /* compute_inverse_diagonal_from_matrixfree (heat_diffuse_operator.cpp:273-284):
    inv = |d| > 1e-10 ? 1/d : 1, constrained rows 1 */

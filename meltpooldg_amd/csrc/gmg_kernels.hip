@@ -47,14 +47,12 @@ __global__ __launch_bounds__(256) void coarse_matrix_kernel(CoarseTables t, int 
         const double b[3] = {t.G[qx][j0] * t.S[qy][j1] * t.S[qz][j2], t.S[qx][j0] * t.G[qy][j1] * t.S[qz][j2],
                              t.S[qx][j0] * t.S[qy][j1] * t.G[qz][j2]};
         if (metric) {
-          const int q = qx + n1 * (qy + n1 * qz);
-          const T *M = metric + cell * 7 * nloc + q;
-          const double g00 = M[nloc], g01 = M[2 * nloc], g11 = M[3 * nloc], g02 = M[4 * nloc], g12 = M[5 * nloc],
-                       g22 = M[6 * nloc];
+          auto M = [&](int comp) -> double { return metric[metric_at(n1, nc0, cell, comp, qx, qy, qz)]; };
+          const double g00 = M(1), g01 = M(2), g11 = M(3), g02 = M(4), g12 = M(5), g22 = M(6);
           const double gg = a[0] * (g00 * b[0] + g01 * b[1] + g02 * b[2]) +
                             a[1] * (g01 * b[0] + g11 * b[1] + g12 * b[2]) +
                             a[2] * (g02 * b[0] + g12 * b[1] + g22 * b[2]);
-          acc += c_mass * (double)M[0] * pI * pJ + kap * gg;
+          acc += c_mass * M(0) * pI * pJ + kap * gg;
         } else {
           const double W = t.w[qx] * t.w[qy] * t.w[qz];
           acc += W * (cm * pI * pJ + kap * (ks0 * a[0] * b[0] + ks1 * a[1] * b[1] + ks2 * a[2] * b[2]));

@@ -1,5 +1,5 @@
-// Matrix-free apply of the implicit heat operator J = c_m M + K_kappa on a
-// structured Q_k hex mesh, for CDNA4 (gfx950).
+// Matrix-free apply of the implicit heat operator J = c_m M + K_kappa on a structured Q4 hex mesh,
+// for CDNA4 (gfx950), and the dispatch over the degrees (Q1..Q3: heat_brick.hip).
 //
 // Replaces HeatDiffuseMultiPhaseOperator::tangent_cell_loop /
 // tangent_local_cell_operation (source/heat/heat_diffuse_operator.cpp:201-241,
@@ -30,45 +30,23 @@
 namespace mpdg {
 
 // cells of a chunk along x, y, z and wavefronts per workgroup (NW * (64 / N1) cells per chunk),
-// chosen by measurement of the apply on large meshes (Q2 64^3, Q3 128^3, Q4 96^3). Longer chunks
-// halve the scatter barriers per column and lengthen the coalesced x rows of the write-out; flat
-// columns (BZ = 1) add face rows on every z plane; one-, two- and eight-wavefront workgroups were
-// slower everywhere (one wavefront, Q3 4x2x2: 0.70 vs 0.64 ms; its barriers are free, but its
-// 2x2-cell columns share 36 % of their rows with neighbours). Q3 (FP64 per-qp): 4x4x4 0.694 ms, 16x2x2 0.652, 8x4x2 0.645, 8x2x4 0.667,
-// 16x4x1 0.878, 8x8x1 0.945; FP32 Q3 (4 wavefronts per SIMD with constant k): 16x2x2 is 1-1.5 %
-// faster than 8x4x2 for every conductivity mode, 8x2x4 equal, 4x4x4 9 % slower, 8x4x2 with 4x2x2-cell
-// wavefront boxes (40.3 KB of LDS: four workgroups per CU instead of three) within 2 %. Q2: 14x3x2 beats
-// 7x4x3 by 5 % (FP64) and 25 % (FP32). Q4: FP64 keeps 4x4x3 (the longer shapes are 1-4 % slower),
-// FP32 gains 11 % with 12x2x2.
+// chosen by measurement of the apply at Q4 96^3: FP64 4x4x3 (longer shapes 1-4 % slower), FP32 12x2x2
+// (11 % faster than 4x4x3).
 // WX x WY x WZ: how the chunk is split into the NW wavefronts' boxes of cells (each box holds
 // the 64 / N1 cells of one wavefront and has its own sub-brick of DoF sums, see ApplyGeom).
 template <int N1, typename Number> struct ChunkShape;
-template <typename Number> struct ChunkShape<2, Number> {
-  static constexpr int BX = 8, BY = 4, BZ = 4, NW = 4, WX = 1, WY = 1, WZ = 4;
-};
-template <typename Number> struct ChunkShape<3, Number> {
-  static constexpr int BX = 14, BY = 3, BZ = 2, NW = 4, WX = 2, WY = 1, WZ = 2;
-};
-template <> struct ChunkShape<4, double> { static constexpr int BX = 8, BY = 4, BZ = 2, NW = 4, WX = 1, WY = 2, WZ = 2; };
-template <> struct ChunkShape<4, float> { static constexpr int BX = 16, BY = 2, BZ = 2, NW = 4, WX = 1, WY = 2, WZ = 2; };
 template <> struct ChunkShape<5, double> { static constexpr int BX = 4, BY = 4, BZ = 3, NW = 4, WX = 1, WY = 4, WZ = 1; };
 template <> struct ChunkShape<5, float> { static constexpr int BX = 12, BY = 2, BZ = 2, NW = 4, WX = 1, WY = 2, WZ = 2; };
-// mapped cells (metric per point): FP64 Q3 runs 8 % faster with 16x2x2 than with the Cartesian
-// 8x4x2 (Q3 96^3, 1.02 vs 1.11 ms), where 8x4x2 stays 2 % ahead
-template <int N1, typename Number, bool MAPPED> struct ChunkShapeOf { using type = ChunkShape<N1, Number>; };
-template <> struct ChunkShapeOf<4, double, true> {
-  struct type { static constexpr int BX = 16, BY = 2, BZ = 2, NW = 4, WX = 1, WY = 2, WZ = 2; };
-};
 
 // Brick rows per batch of the write-out, whose LDS reads are all issued before any of its sums
 // (0: one row at a time, each read waited for in turn). Batches pay where the write-out's LDS
 // latency is exposed: the FP64 Q4 apply (one wavefront per SIMD) runs 6 % faster with batches
-// of 5 rows; at Q3 they change nothing in FP64 and cost FP32 its occupancy (spills).
+// of 5 rows.
 template <int N1, typename Number, bool MAPPED> struct WriteOutBatch { static constexpr int value = 0; };
 template <> struct WriteOutBatch<5, double, false> { static constexpr int value = 5; };
 
 template <int N1, typename Number = double, bool MAPPED = false> struct ApplyGeom {
-  using Shape = typename ChunkShapeOf<N1, Number, MAPPED>::type;
+  using Shape = ChunkShape<N1, Number>;
   static constexpr int K = N1 - 1;
   static constexpr int CPW = 64 / N1;                 // cells per wavefront
   static constexpr int NW = Shape::NW;                // wavefronts per workgroup
@@ -248,18 +226,6 @@ __device__ __forceinline__ int brick_parts(int p, int (&part)[2]) {
   }
 }
 
-template <typename Number>
-__device__ __forceinline__ Number law_kappa(int law, const Number *p, Number T) {
-  if (law == LAW_TANH) {
-    return p[0] * (Number(1) + p[1] * tanh((T - p[2]) / p[3]));
-  }
-  // mushy zone (liquid_solid): p = {k_liquid, k_solid, T_solidus, T_liquidus}
-  const Number inv = Number(1) / (p[3] - p[2]);
-  Number fs = (p[3] - T) * inv;
-  fs = fs < Number(0) ? Number(0) : (fs > Number(1) ? Number(1) : fs);
-  return p[0] + (p[1] - p[0]) * (Number(3) - Number(2) * fs) * fs * fs;
-}
-
 // Gather the z-plane l of a cell (read_dof_values with homogeneous Dirichlet rows zeroed).
 // Lanes without a cell read cell 0's plane (in bounds) and zero it afterwards, so the loads
 // carry no per-element branches.
@@ -325,14 +291,8 @@ __device__ __forceinline__ void load_kappa_qp(const Number *__restrict__ kappa, 
 
 // wavefronts per SIMD the register allocation targets (1 = the compiler's choice). Mapped
 // cells keep all three flux components and the metric live at the quadrature points and get
-// the full register file rather than spill. The FP32 Q3 apply with a constant conductivity
-// fits 128 VGPRs (2 spilled) and runs 4 % faster at 4 wavefronts than at 3; with per-point or
-// law conductivity the same limit spills 13-18 VGPRs.
+// the full register file rather than spill.
 template <int N1, typename Number, bool MAPPED, int KMODE> struct Occupancy { static constexpr int W = 1; };
-template <int KM> struct Occupancy<4, double, false, KM> { static constexpr int W = 2; };
-template <int KM> struct Occupancy<4, float, false, KM> { static constexpr int W = 3; };
-template <> struct Occupancy<4, float, false, KAPPA_CONST> { static constexpr int W = 4; };
-template <int KM> struct Occupancy<4, float, true, KM> { static constexpr int W = 2; };
 template <int KM> struct Occupancy<5, float, false, KM> { static constexpr int W = 2; };
 
 template <int N1, typename Number, int KMODE, bool MAPPED>
@@ -346,7 +306,7 @@ void heat_apply_kernel(const ApplyArgs<Number, N1> P,
   // the last x plane of the chunk, carried to the next one (two buffers by chunk parity, since
   // the write-out reads the previous chunk's carry while it writes its own). Sized at launch
   // rather than declared: with the size known, the compiler derives the occupancy from the
-  // LDS and schedules for it (at Q3 FP64 it then spills 29 VGPRs; this way it needs 230).
+  // LDS and schedules for it.
   extern __shared__ double dyn_lds[];
   double *const lds_raw = dyn_lds;
   double *const acc = dyn_lds + G::TBUF_DOUBLES;
@@ -765,19 +725,10 @@ size_t edge_elems_shape(const int *nc) {
   const long ny = (nc[1] + G::BY - 1) / G::BY, nz = (nc[2] + G::BZ - 1) / G::BZ;
   return (size_t)((ny - 1) * (nz - 1) * ((long)(N1 - 1) * nc[0] + 1));
 }
-template <int N1, typename Number>
-size_t edge_elems_n1(const int *nc, int mapped) {
-  const size_t c = edge_elems_shape<N1, Number, false>(nc), m = edge_elems_shape<N1, Number, true>(nc);
-  return mapped < 0 ? std::max(c, m) : (mapped ? m : c);
-}
-size_t apply_edge_elems(int degree, const int *nc, bool fp32, int mapped) {
-  switch (degree) {
-    case 1: return fp32 ? edge_elems_n1<2, float>(nc, mapped) : edge_elems_n1<2, double>(nc, mapped);
-    case 2: return fp32 ? edge_elems_n1<3, float>(nc, mapped) : edge_elems_n1<3, double>(nc, mapped);
-    case 3: return fp32 ? edge_elems_n1<4, float>(nc, mapped) : edge_elems_n1<4, double>(nc, mapped);
-    case 4: return fp32 ? edge_elems_n1<5, float>(nc, mapped) : edge_elems_n1<5, double>(nc, mapped);
-    default: return 0;
-  }
+size_t apply_edge_elems(int degree, const int *nc, bool fp32) {
+  if (degree >= 1 && degree <= 3) return brick_scratch_elems(degree, nc);
+  if (degree != 4) return 0;
+  return fp32 ? edge_elems_shape<5, float, false>(nc) : edge_elems_shape<5, double, false>(nc);
 }
 
 // LDS beyond 64 KiB per workgroup has to be allowed per kernel before its first launch
@@ -852,25 +803,15 @@ int launch_apply_shape(const OperatorData<Number> &op, const Number *src, Number
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }
 
-template <int N1, typename Number>
-int launch_apply_n1(const OperatorData<Number> &op_in, const Number *src, Number *dst, hipStream_t stream,
-                    hipEvent_t kernel_start, hipEvent_t kernel_end) {
+template <typename Number>
+int launch_apply(const OperatorData<Number> &op_in, const Number *src, Number *dst, hipStream_t stream,
+                 hipEvent_t kernel_start, hipEvent_t kernel_end) {
   const OperatorData<Number> op = kernel_view(op_in);
   if (op.metric == nullptr && op_in.metric != nullptr) return MPDG_ERR_INVALID;  // metric_k not computed
-  if (op.metric) return launch_apply_shape<N1, Number, true>(op, src, dst, stream, kernel_start, kernel_end);
-  return launch_apply_shape<N1, Number, false>(op, src, dst, stream, kernel_start, kernel_end);
-}
-
-template <typename Number>
-int launch_apply(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
-                 hipEvent_t kernel_start, hipEvent_t kernel_end) {
-  switch (op.degree) {
-    case 1: return launch_apply_n1<2, Number>(op, src, dst, stream, kernel_start, kernel_end);
-    case 2: return launch_apply_n1<3, Number>(op, src, dst, stream, kernel_start, kernel_end);
-    case 3: return launch_apply_n1<4, Number>(op, src, dst, stream, kernel_start, kernel_end);
-    case 4: return launch_apply_n1<5, Number>(op, src, dst, stream, kernel_start, kernel_end);
-    default: return MPDG_ERR_INVALID;
-  }
+  if (op.degree >= 1 && op.degree <= 3) return launch_brick<Number>(op, src, dst, stream, kernel_start, kernel_end);
+  if (op.degree != 4) return MPDG_ERR_INVALID;
+  if (op.metric) return launch_apply_shape<5, Number, true>(op, src, dst, stream, kernel_start, kernel_end);
+  return launch_apply_shape<5, Number, false>(op, src, dst, stream, kernel_start, kernel_end);
 }
 
 template int launch_apply<double>(const OperatorData<double> &, const double *, double *, hipStream_t, hipEvent_t,

@@ -29,15 +29,6 @@ AuxTables<Number> make_aux_tables(int k) {
   return t;
 }
 
-template <typename Number>
-__device__ __forceinline__ Number law_value(int law, const Number *p, Number T) {
-  if (law == LAW_TANH) return p[0] * (Number(1) + p[1] * tanh((T - p[2]) / p[3]));
-  const Number inv = Number(1) / (p[3] - p[2]);
-  Number fs = (p[3] - T) * inv;
-  fs = fs < Number(0) ? Number(0) : (fs > Number(1) ? Number(1) : fs);
-  return p[0] + (p[1] - p[0]) * (Number(3) - Number(2) * fs) * fs * fs;
-}
-
 // Cell-local tensor kernels. A 256-thread workgroup holds kCellsPerBlock<N1> cells with N1^2
 // threads per cell, one per line of the cell's N1^3 tensor; a contraction with a 1D matrix
 // along each direction is one sweep in registers and one transpose through LDS, so a cell
@@ -112,7 +103,7 @@ __global__ __launch_bounds__(256) void kappa_law_kernel(AuxTables<Number> t, int
       Number s = Number(0);
 #pragma unroll
       for (int l = 0; l < N1; ++l) s += t.S[q][l] * u[l];
-      const Number k = law_value<Number>(law, p, s);
+      const Number k = law_kappa<Number>(law, p, s);
       if (kq && active) kq[cell * NQ + q * L2 + r] = k;
       part += t.w[q] * k;
     }
@@ -267,7 +258,7 @@ __global__ __launch_bounds__(256) void diagonal_kernel(AuxTables<Number> t, int 
         Number c = Number(0);
         if (active) {
           if (MAPPED) {
-            const Number m = metric[(cell * 7 + comp[term]) * NQ + qz * L2 + r];
+            const Number m = metric[metric_at(N1, nc0, cell, comp[term], b, a, qz)];
             c = term == 0 ? cm * m : (term >= 4 ? Number(2) : Number(1)) * kk[qz] * m;
           } else {
             const Number W = t.w[qz] * t.w[a] * t.w[b];
@@ -628,8 +619,10 @@ __global__ __launch_bounds__(256) void metric_kernel(AuxTables<double> t, int n1
   const int nq = n1 * n1 * n1, K = n1 - 1;
   const long gid = (long)blockIdx.x * 256 + threadIdx.x;
   if (gid >= ncells * nq) return;
-  const long cell = gid / nq;
-  const int q = gid - cell * nq;
+  // consecutive threads: consecutive cells of a row, so that the stores of a component are contiguous
+  const long row = gid / ((long)nc0 * nq);
+  const int in_row = (int)(gid - row * nc0 * nq), q = in_row / nc0;
+  const long cell = row * nc0 + in_row % nc0;
   const int qx = q % n1, qy = (q / n1) % n1, qz = q / (n1 * n1);
   const int cx = cell % nc0, cy = (cell / nc0) % nc1, cz = cell / ((long)nc0 * nc1);
   double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -661,14 +654,14 @@ __global__ __launch_bounds__(256) void metric_kernel(AuxTables<double> t, int n1
   B[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
   const double jxw = fabs(det) * t.w[qx] * t.w[qy] * t.w[qz];
   auto g = [&](int a, int b) { return jxw * (B[a][0] * B[b][0] + B[a][1] * B[b][1] + B[a][2] * B[b][2]); };
-  Number *M = metric + cell * 7 * nq + q;
-  M[0] = (Number)jxw;
-  M[nq] = (Number)g(0, 0);
-  M[2 * nq] = (Number)g(0, 1);
-  M[3 * nq] = (Number)g(1, 1);
-  M[4 * nq] = (Number)g(0, 2);
-  M[5 * nq] = (Number)g(1, 2);
-  M[6 * nq] = (Number)g(2, 2);
+  auto M = [&](int comp) -> Number & { return metric[metric_at(n1, nc0, cell, comp, qx, qy, qz)]; };
+  M(0) = (Number)jxw;
+  M(1) = (Number)g(0, 0);
+  M(2) = (Number)g(0, 1);
+  M(3) = (Number)g(1, 1);
+  M(4) = (Number)g(0, 2);
+  M(5) = (Number)g(1, 2);
+  M(6) = (Number)g(2, 2);
 }
 
 template <typename Number>
@@ -679,23 +672,31 @@ int launch_metric(const OperatorData<Number> &op, const double *coords, Number *
                      n1, op.nc[0], op.nc[1], op.n_cells, op.nd[0], op.nd[1], op.n_dofs, coords, metric);
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }
-// metric_k[c][0][q] = metric[c][0][q] (JxW), metric_k[c][i][q] = kq[c][q] metric[c][i][q] (i = 1..6)
+// metric_k: component 0 (JxW) as it is, components 1..6 times the point's conductivity kq[cell][q]
 template <typename Number>
 __global__ __launch_bounds__(256) void scale_metric_kernel(const Number *__restrict__ metric, const Number *__restrict__ kq,
-                                                           Number *__restrict__ out, long ncells, int nq) {
-  const long n = ncells * 7 * nq;
-  for (long g = (long)blockIdx.x * 256 + threadIdx.x; g < n; g += (long)gridDim.x * 256) {
-    const long c = g / (7 * nq);
-    const int r = g - c * 7 * nq, comp = r / nq, q = r - comp * nq;
-    out[g] = comp == 0 ? metric[g] : kq[c * nq + q] * metric[g];
+                                                           Number *__restrict__ out, long ncells, int n1, int nc0) {
+  // consecutive threads: consecutive cells of a row (as the metric lies)
+  const int nq = n1 * n1 * n1;
+  const long n = ncells * nq;
+  for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < n; t += (long)gridDim.x * 256) {
+    const long row = t / ((long)nc0 * nq);
+    const int in_row = (int)(t - row * nc0 * nq), q = in_row / nc0;
+    const long c = row * nc0 + in_row % nc0;
+    const int qx = q % n1, qy = (q / n1) % n1, qz = q / (n1 * n1);
+    const Number k = kq[c * nq + q];
+    for (int comp = 0; comp < 7; ++comp) {
+      const long g = metric_at(n1, nc0, c, comp, qx, qy, qz);
+      out[g] = comp == 0 ? metric[g] : k * metric[g];
+    }
   }
 }
 template <typename Number>
 int launch_scale_metric(const OperatorData<Number> &op, const Number *kq, Number *metric_k, hipStream_t s) {
-  const int n1 = op.degree + 1, nq = n1 * n1 * n1;
-  const long n = op.n_cells * 7 * nq;
+  const int n1 = op.degree + 1;
+  const long n = op.n_cells * n1 * n1 * n1;
   hipLaunchKernelGGL(scale_metric_kernel<Number>, dim3(std::min<long>((n + 255) / 256, 16384)), dim3(256), 0, s,
-                     op.metric, kq, metric_k, op.n_cells, nq);
+                     op.metric, kq, metric_k, op.n_cells, n1, op.nc[0]);
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }
 template int launch_scale_metric<double>(const OperatorData<double> &, const double *, double *, hipStream_t);

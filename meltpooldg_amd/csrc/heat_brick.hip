@@ -1,0 +1,956 @@
+// Matrix-free apply of the implicit heat operator J = c_m M + K_kappa for Q1..Q3 on CDNA4
+// (gfx950): HeatDiffuseMultiPhaseOperator::tangent_cell_loop / tangent_local_cell_operation
+// (source/heat/heat_diffuse_operator.cpp:201-241, :957-1086). Q4 runs the column kernel of
+// heat_apply.hip (its five z planes do not fit the four lane rows used here).
+//
+// Work decomposition
+//   * A workgroup of four wavefronts owns a brick of 16 x SEG x ZC cells (ZC = 4, Q1: 8). A
+//     wavefront holds one pencil of 16 cells along x per step and marches along y.
+//   * Lane = 16 (z plane of the cell) + (cell along x); the lane's registers hold the plane's
+//     N1 x N1 DoFs [y][x]. Q1 puts two cells' planes into the four lane rows, Q2 leaves one row
+//     idle.
+//   * Sum factorisation without a change of layout: x and y sweeps are register-local; the z
+//     sweeps contract over the lane rows. In FP64 that is v_mfma_f64_4x4x4_4b (B and D share the
+//     layout lane = 16 k + column, so a z sweep is one MFMA per register with the 1D table as A; it
+//     runs at the rate of v_fma_f64 and saves the LDS transposes around a sweep on the VALU); in FP32
+//     the forward pair of sweeps is one v_mfma_f32_16x16x4 per register whose rows 4 g + r hold row g
+//     of table r, and the backward pair transposes y registers against lane rows with
+//     v_permlane32/16_swap. Conductivity per point: twelve sweeps (collocated gradients on the Gauss
+//     points). One conductivity per Cartesian cell: seven sweeps with 1D mass and stiffness matrices.
+//   * Sums over cells, in FP64 at every precision and in a fixed order: along y the top row of
+//     a cell stays in registers for the next step; along x the last column moves one lane up
+//     (DPP row_shr:1); along z the top plane goes through LDS to the next pencil (one workgroup
+//     barrier per step).
+//   * A brick stores its DoFs except its upper x, y, z planes; those are shared with the next
+//     brick, which owns them, and go to a scratch array per class (planes, edges, corners).
+//     brick_fixup_kernel adds the classes to dst in a fixed order: no atomics and no zeroed
+//     rows, and vmult is bitwise repeatable.
+//
+// What bounds it: at Q3 FP64 with k per point, HBM (2.5 GB moved of 2.0 GB that the apply cannot do
+// without, 870 VALU instructions per 64 lanes and step) -- Q3 128^3, whole vmult: 0.663 ms for the column
+// kernel with LDS transposes, scatter and atomics it replaces, 0.566 ms here; elsewhere the VALU (Q3 128^3,
+// constant k: FP64 0.62 -> 0.43 ms, FP32 0.42 -> 0.28 ms; Q2 64^3 FP32 35.7 -> 25.5 us; Q3 75 x 62 x 49 FP32
+// 83.8 -> 50.5 us; mapped Q3 96^3 FP64, bound by the stored metric, 1.08 -> 0.82 ms).
+#include "kernels.hpp"
+
+namespace mpdg {
+
+namespace {
+
+constexpr int kNX = 16;  // cells of a pencil along x (lanes of a DPP row)
+constexpr int kNW = 4;   // wavefronts of a workgroup
+
+template <int N1> struct BrickShape {
+  static constexpr int K = N1 - 1;
+  static constexpr int ZPW = N1 == 2 ? 2 : 1;  // cells along z per wavefront
+  static constexpr int ZC = kNW * ZPW;         // cells along z per brick
+};
+
+// A brick is cells[0] x cells[1] x cells[2] cells: pencils of kNX cells side by side along x, done one
+// after the other, steps along y, pencils along z. Shared-plane classes: bit 0 upper x plane, bit 1
+// upper y plane, bit 2 upper z plane.
+struct BrickGrid {
+  int nb[3];       // bricks
+  int cells[3];    // cells of a full brick
+  long off[8];     // scratch offset of each class (off[0] unused)
+  long total;      // scratch entries
+};
+constexpr int kMaxSteps = 16, kMaxPencils = 2;
+
+// Steps along y and pencils along x per brick. Long bricks share fewer planes and amortise the
+// table set-up; short ones give the chip enough wavefronts: about 2048 workgroups while a brick is
+// shorter than 16 steps (Q2 64^3 FP32: 25.5 us; 1024: 29, 4096: 33; Q3 64^3 per cell FP32: 43 us against 48
+// and 49), then two pencils along x where more than 1024 remain (the x planes' fix-up is strided:
+// Q3 128^3 FP64 per point 619 us against 634 with one, 643 with four, whose LDS halves the occupancy).
+// The rule depends on the mesh only, so every apply of a mesh sums in the same order.
+BrickGrid brick_grid(int k, const int *nc) {
+  BrickGrid g;
+  const int zc = k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC;
+  const int px = (nc[0] + kNX - 1) / kNX;
+  g.cells[2] = zc;
+  g.nb[2] = (nc[2] + zc - 1) / zc;
+  const long steps = (long)px * g.nb[2] * nc[1];  // workgroup steps of the whole apply
+  g.cells[1] = (int)std::min<long>({kMaxSteps, std::max<long>(1, steps / 2048), nc[1]});
+  g.nb[1] = (nc[1] + g.cells[1] - 1) / g.cells[1];
+  const int xb = (int)std::min<long>({kMaxPencils, std::max<long>(1, (long)px * g.nb[1] * g.nb[2] / 512), px});
+  g.cells[0] = kNX * xb;
+  g.nb[0] = (px + xb - 1) / xb;
+  const long nd[3] = {(long)k * nc[0] + 1, (long)k * nc[1] + 1, (long)k * nc[2] + 1};
+  long o = 0;
+  g.off[0] = 0;
+  for (int c = 1; c < 8; ++c) {
+    g.off[c] = o;
+    long n = 1;
+    for (int d = 0; d < 3; ++d) n *= (c >> d & 1) ? g.nb[d] - 1 : nd[d];
+    o += n;
+  }
+  g.total = o;
+  return g;
+}
+
+template <typename Number, int N1>
+struct BrickArgs {
+  Half1D<Number, N1, false> S;            // shape values at the Gauss points
+  Half1D<Number, N1, true> D, Dy, G;      // collocation derivative (Dy: times ky/kx), basis derivative
+  Half1D<Number, N1, true> Gz;            // basis derivative times kz/kx
+  Half1D<Number, N1, false> M1, K1;       // 1D mass and stiffness matrices of the unit cell
+  Number w[(N1 + 1) / 2];  // Gauss weights (symmetric)
+  int nc[3], nd[3];
+  long n_cells;
+  BrickGrid g;
+  int dmask, law;
+  Number cm, kx, ky, kz, kappa;  // V c_m, k_d = V/h_d^2 (mapped cells: 1)
+  Number law_p[4];
+  const Number *kappa_arr, *T, *metric;
+  Number *scratch;
+};
+
+// x sweep (second index): out[j][q] = sum_i M(q, i) in[j][i]; y sweep (first index) likewise
+template <int N1, bool TR, bool ADD, typename Number, typename Mat>
+__device__ __forceinline__ void sweep_x(const Mat &M, const Number (&in)[N1][N1], Number (&out)[N1][N1]) {
+#pragma unroll
+  for (int j = 0; j < N1; ++j)
+#pragma unroll
+    for (int q = 0; q < N1; ++q) {
+      Number a = ADD ? out[j][q] : Number(0);
+#pragma unroll
+      for (int i = 0; i < N1; ++i) a = fma(TR ? M(i, q) : M(q, i), in[j][i], a);
+      out[j][q] = a;
+    }
+}
+template <int N1, bool TR, bool ADD, typename Number, typename Mat>
+__device__ __forceinline__ void sweep_y(const Mat &M, const Number (&in)[N1][N1], Number (&out)[N1][N1]) {
+#pragma unroll
+  for (int i = 0; i < N1; ++i)
+#pragma unroll
+    for (int q = 0; q < N1; ++q) {
+      Number a = ADD ? out[q][i] : Number(0);
+#pragma unroll
+      for (int j = 0; j < N1; ++j) a = fma(TR ? M(j, q) : M(q, j), in[j][i], a);
+      out[q][i] = a;
+    }
+}
+
+using f32x4 = float __attribute__((ext_vector_type(4)));
+
+// entry (row, col) of a table for a lane-dependent place; 0 outside (Q2's idle row)
+template <int N1, typename Number, typename Mat>
+__device__ __forceinline__ Number table_entry(const Mat &M, int row, int col) {
+  Number v = 0;
+#pragma unroll
+  for (int a = 0; a < N1; ++a)
+#pragma unroll
+    for (int b = 0; b < N1; ++b) v = (row == a && col == b) ? M(a, b) : v;
+  return v;
+}
+
+__device__ __forceinline__ void swap32(float &a, float &b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const unsigned x = r[0], y = r[1];  // (a bit cast of a subscript would read element 0)
+  a = __uint_as_float(x);
+  b = __uint_as_float(y);
+}
+__device__ __forceinline__ void swap16(float &a, float &b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const unsigned x = r[0], y = r[1];
+  a = __uint_as_float(x);
+  b = __uint_as_float(y);
+}
+__device__ __forceinline__ void swap16(double &a, double &b) {
+  float al = __uint_as_float((unsigned)__double2loint(a)), ah = __uint_as_float((unsigned)__double2hiint(a));
+  float bl = __uint_as_float((unsigned)__double2loint(b)), bh = __uint_as_float((unsigned)__double2hiint(b));
+  swap16(al, bl);
+  swap16(ah, bh);
+  a = __hiloint2double((int)__float_as_uint(ah), (int)__float_as_uint(al));
+  b = __hiloint2double((int)__float_as_uint(bh), (int)__float_as_uint(bl));
+}
+// registers <-> lane rows: afterwards register j of lane row r holds what register r of lane row
+// j held (Q1: within each pair of lane rows)
+template <int N1, typename Number> __device__ __forceinline__ void row_transpose(Number (&r)[4]) {
+  if constexpr (N1 == 2) {
+    swap16(r[0], r[1]);
+  } else {
+    swap32(r[0], r[2]);
+    swap32(r[1], r[3]);
+    swap16(r[0], r[1]);
+    swap16(r[2], r[3]);
+  }
+}
+
+// The lane's entries of the A operands of the z sweeps (see the file's head): forward tables F0 and
+// F1 (values and derivative, or mass and stiffness), backward ones S^T and G_z^T.
+template <int N1, typename Number> struct ZTables {  // Q1: transposed sweeps only
+  template <typename Args, typename T0, typename T1>
+  __device__ __forceinline__ ZTables(const Args &, const T0 &, const T1 &, int) {}
+};
+template <int N1> struct ZTablesF64 {
+  double f0, f1, st, gt;
+  template <typename Args, typename T0, typename T1>
+  __device__ __forceinline__ ZTablesF64(const Args &P, const T0 &F0, const T1 &F1, int lane) {
+    const int i = lane & 3, k = lane >> 4;  // A[i][k]
+    f0 = table_entry<N1, double>(F0, i, k);
+    f1 = table_entry<N1, double>(F1, i, k);
+    st = table_entry<N1, double>(P.S, k, i);
+    gt = table_entry<N1, double>(P.Gz, k, i);
+  }
+};
+template <int N1> struct ZTablesF32 {
+  float f01;
+  template <typename Args, typename T0, typename T1>
+  __device__ __forceinline__ ZTablesF32(const Args &, const T0 &F0, const T1 &F1, int lane) {
+    const int row = (lane & 15) >> 2, r = lane & 3, k = lane >> 4;  // A[4 row + r][k] = table r, entry (row, k)
+    const float a = table_entry<N1, float>(F0, row, k), b = table_entry<N1, float>(F1, row, k);
+    f01 = r > 1 ? 0.0f : (r == 0 ? a : b);
+  }
+};
+template <> struct ZTables<3, double> : ZTablesF64<3> { using ZTablesF64<3>::ZTablesF64; };
+template <> struct ZTables<4, double> : ZTablesF64<4> { using ZTablesF64<4>::ZTablesF64; };
+template <> struct ZTables<3, float> : ZTablesF32<3> { using ZTablesF32<3>::ZTablesF32; };
+template <> struct ZTables<4, float> : ZTablesF32<4> { using ZTablesF32<4>::ZTablesF32; };
+
+// v = F0 t along z, and g = F1 t when SECOND
+template <int N1, bool SECOND, typename Number, typename T0, typename T1>
+__device__ __forceinline__ void z_forward(const T0 &F0, const T1 &F1, const ZTables<N1, Number> &z, const Number (&t)[N1][N1],
+                                          Number (&v)[N1][N1], Number (&g)[N1][N1]) {
+  if constexpr (N1 == 2) {
+    // pairs of lane rows hold different cells: sweeps on the transposed pairs, so that nothing of one
+    // cell is multiplied into another
+#pragma unroll
+    for (int i = 0; i < N1; ++i) {
+      Number a[4] = {t[0][i], t[1][i], 0, 0}, s[4] = {0, 0, 0, 0}, d[4] = {0, 0, 0, 0};
+      row_transpose<N1>(a);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        s[q] = fma(F0(q, 0), a[0], F0(q, 1) * a[1]);
+        d[q] = fma(F1(q, 0), a[0], F1(q, 1) * a[1]);
+      }
+      row_transpose<N1>(s);
+      if (SECOND) row_transpose<N1>(d);
+#pragma unroll
+      for (int j = 0; j < N1; ++j) {
+        v[j][i] = s[j];
+        if (SECOND) g[j][i] = d[j];
+      }
+    }
+  } else if constexpr (sizeof(Number) == 8) {
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        const double x = t[j][i];
+        v[j][i] = __builtin_amdgcn_mfma_f64_4x4x4f64(z.f0, x, 0.0, 0, 0, 0);
+        if (SECOND) g[j][i] = __builtin_amdgcn_mfma_f64_4x4x4f64(z.f1, x, 0.0, 0, 0, 0);
+      }
+  } else {
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        const f32x4 r = __builtin_amdgcn_mfma_f32_16x16x4f32(z.f01, t[j][i], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        v[j][i] = r[0];
+        if (SECOND) g[j][i] = r[1];
+      }
+  }
+}
+
+// out = S_z^T e + G_z^T f (the z table of the way back carries the direction's factor)
+template <int N1, typename Args, typename Number>
+__device__ __forceinline__ void z_backward(const Args &P, const ZTables<N1, Number> &z, const Number (&e)[N1][N1],
+                                           const Number (&f)[N1][N1], Number (&out)[N1][N1]) {
+  if constexpr (N1 > 2 && sizeof(Number) == 8) {
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        const double a = __builtin_amdgcn_mfma_f64_4x4x4f64(z.gt, f[j][i], 0.0, 0, 0, 0);
+        out[j][i] = __builtin_amdgcn_mfma_f64_4x4x4f64(z.st, e[j][i], a, 0, 0, 0);
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N1; ++i) {
+      Number a[4] = {0, 0, 0, 0}, b[4] = {0, 0, 0, 0}, o[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int j = 0; j < N1; ++j) {
+        a[j] = e[j][i];
+        b[j] = f[j][i];
+      }
+      row_transpose<N1>(a);
+      row_transpose<N1>(b);
+#pragma unroll
+      for (int q = 0; q < N1; ++q) {
+        Number s = 0;
+#pragma unroll
+        for (int k = 0; k < N1; ++k) s = fma(P.Gz(k, q), b[k], s);
+#pragma unroll
+        for (int k = 0; k < N1; ++k) s = fma(P.S(k, q), a[k], s);
+        o[q] = s;
+      }
+      row_transpose<N1>(o);
+#pragma unroll
+      for (int j = 0; j < N1; ++j) out[j][i] = o[j];
+    }
+  }
+}
+
+// value of the previous lane in the row of 16; the first lane gets `first`
+__device__ __forceinline__ double from_previous_cell(double x, double first) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(x), 0x111, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(x), 0x111, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// orders the LDS accesses of a wavefront's lanes
+__device__ __forceinline__ void lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Wavefronts per SIMD the register allocation targets: as many as fit without spills (Q3 FP64 needs
+// 226 VGPRs with per-point conductivity and 168 with one per cell, Q3 FP32 129 and 116; mapped cells
+// hold three fluxes: 195 and 129). Fewer wavefronts were slower even where the next step's source was
+// loaded ahead, and with three or four the loads need no such registers.
+template <int N1, typename Number, bool MAPPED, int KMODE> struct BrickOccupancy { static constexpr int W = 4; };
+template <bool M, int KM> struct BrickOccupancy<3, double, M, KM> { static constexpr int W = 3; };
+template <bool M, int KM> struct BrickOccupancy<4, double, M, KM> { static constexpr int W = 2; };
+template <> struct BrickOccupancy<4, double, false, KAPPA_CONST> { static constexpr int W = 3; };
+template <> struct BrickOccupancy<4, double, false, KAPPA_CELL> { static constexpr int W = 3; };
+template <int KM> struct BrickOccupancy<4, float, true, KM> { static constexpr int W = 3; };
+template <> struct BrickOccupancy<4, float, false, KAPPA_QP> { static constexpr int W = 3; };
+
+// what a lane is, in one register (tested where it is needed: as loop invariants the tests would
+// occupy two scalar registers each, and the 1D tables need those)
+constexpr int F_TOP = 1;     // its lane row holds its cell's upper z plane
+constexpr int F_LOW = 2;     // ... the lowest z plane, with a pencil below in the brick
+constexpr int F_STORE = 4;   // ... a plane of the mesh that this wavefront stores
+constexpr int F_HZ = 8;      // ... the brick's upper z plane, owned by the next brick
+constexpr int F_LAST = 16;   // the last lane of its row
+__device__ __forceinline__ int opaque(int f) {
+  asm volatile("" : "+v"(f));
+  return f;
+}
+
+// The kernel's arguments read anew where they are used: kept in scalar registers over the whole
+// loop, the mesh's sizes and offsets push the 1D tables out of them (150 v_readlane per step)
+template <typename Args> __device__ __forceinline__ const __attribute__((address_space(4))) Args &fresh_args() {
+  auto p = (const __attribute__((address_space(4))) Args *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+
+template <int N1, typename Number, int KMODE, bool MAPPED>
+__global__ __launch_bounds__(64 * kNW) __attribute__((amdgpu_waves_per_eu(BrickOccupancy<N1, Number, MAPPED, KMODE>::W)))
+void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__ src, Number *__restrict__ dst) {
+  using B = BrickShape<N1>;
+  constexpr int K = B::K, NQ = N1 * N1 * N1, W = K * kNX;
+  // Q3: per-point conductivities go through LDS. 16 cells' values are contiguous in memory and are
+  // loaded 1 KB per instruction; read in place, a lane's own N1^2 values would cost one L1 line per
+  // lane and load (0.12 ms of the Q3 128^3 apply)
+  constexpr bool STAGE = KMODE == KAPPA_QP && N1 == 4 && !MAPPED;
+  constexpr int NV = 16 / (int)sizeof(Number), CH = N1 * N1 / NV, PER = 4 * CH, NLD = STAGE ? kNX * PER / 64 : 1;
+  __shared__ double top[2][B::ZC][K][N1][kNX];      // top planes of the pencils' cells, by step parity
+  __shared__ double yrow[kNW][kMaxPencils][N1][64]; // top rows of the previous y step's cells
+  __shared__ Number srow[kNW][kMaxPencils][N1][64]; // their source rows, the next step's lowest
+  __shared__ double xcol[kNW][N1][4];               // last x column of the previous pencil
+  // per wavefront: staged conductivities, then the rows of results, to be stored with consecutive
+  // lanes on consecutive addresses
+  constexpr int STAGE_N = STAGE ? NQ * kNX : 0, TILE_N = K > 1 ? 4 * (64 / W) * W : 1;
+  __shared__ __attribute__((aligned(16))) Number buf[kNW][STAGE_N > TILE_N ? STAGE_N : TILE_N];
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row = lane >> 4, c = lane & 15;
+  const int l = N1 == 2 ? row & 1 : row;                  // z plane of the cell
+  const int zc = N1 == 2 ? 2 * wave + (row >> 1) : wave;  // cell along z in the brick
+  // consecutive workgroups run on different XCDs; give each XCD a contiguous range of bricks
+  const int nbr = gridDim.x, xcd = blockIdx.x & 7;
+  int b = xcd * (nbr >> 3) + min(xcd, nbr & 7) + (blockIdx.x >> 3);
+  const int bx = b % P.g.nb[0];
+  b /= P.g.nb[0];
+  const int by = b % P.g.nb[1], bz = b / P.g.nb[1];
+  const int cz = bz * B::ZC + zc, cy0 = by * P.g.cells[1], cx0 = bx * P.g.cells[0];
+  const int cy_end = min(cy0 + P.g.cells[1], P.nc[1]), cx_end = min(cx0 + P.g.cells[0], P.nc[0]);
+  const int iz = K * cz + l;
+  const long sy = P.nd[0], sz = (long)P.nd[0] * P.nd[1];
+  // a conductivity that is constant on a Cartesian cell: the cell's operator is a sum of products of
+  // 1D mass and stiffness matrices, seven sweeps instead of twelve
+  constexpr bool TENSOR = !MAPPED && (KMODE == KAPPA_CONST || KMODE == KAPPA_CELL);
+  const ZTables<N1, Number> zt = [&] {
+    if constexpr (TENSOR) return ZTables<N1, Number>(P, P.M1, P.K1, lane);
+    else return ZTables<N1, Number>(P, P.S, P.G, lane);
+  }();
+  Number wz = 0;
+#pragma unroll
+  for (int a = 0; a < N1; ++a) wz = l == a ? P.w[a < N1 - 1 - a ? a : N1 - 1 - a] : wz;
+  int flags = 0;
+  {
+    const bool on = cz < P.nc[2] && l <= K, last_z = cz == P.nc[2] - 1;
+    if (l == K) flags |= F_TOP;
+    if (l == 0 && zc > 0) flags |= F_LOW;
+    if (on && (l < K || zc == B::ZC - 1 || last_z)) flags |= F_STORE;
+    if (l == K && !last_z) flags |= F_HZ;
+    if (c == kNX - 1) flags |= F_LAST;
+  }
+  // Lanes without a cell work on the mesh's last cell in their direction: in bounds, and nothing of
+  // theirs reaches another lane's cell (sums pass upwards in x and z only). Q2's idle lane row
+  // holds zeros.
+  const long zoff = sz * (K * min(cz, P.nc[2] - 1) + min(l, K));
+
+  // constrained planes that touch the pencil at (cxb, cy): zero the DoFs on them
+  auto constrain = [&](int cxb, int cy, auto &u) {
+    const auto &A = fresh_args<BrickArgs<Number, N1>>();
+    int m = A.dmask;
+    if (m) {
+      if (cxb > 0) m &= ~1;
+      if (cxb + kNX < A.nc[0]) m &= ~2;
+      if (cy > 0) m &= ~4;
+      if (cy + 1 < A.nc[1]) m &= ~8;
+    }
+    if (m) {
+      const int cx = cxb + opaque(c), z = opaque(iz);
+      const bool con_z = ((m & 16) && z == 0) || ((m & 32) && z == A.nd[2] - 1);
+#pragma unroll
+      for (int j = 0; j < N1; ++j)
+#pragma unroll
+        for (int i = 0; i < N1; ++i)
+          if (con_z || ((m & 4) && j == 0) || ((m & 8) && j == K) || ((m & 1) && i == 0 && cx == 0) ||
+              ((m & 2) && i == K && cx == A.nc[0] - 1))
+            u[j][i] = 0;
+    }
+  };
+  // the plane's rows of the pencil's cells
+  auto load_rows = [&](const Number *field, int cxb, int cy, bool lowest, Number (&u)[N1][N1]) {
+    const Number *p = field + (zoff + K * min(cxb + c, P.nc[0] - 1)) + sy * ((long)K * cy);
+#pragma unroll
+    for (int i = 0; i < N1; ++i) u[0][i] = lowest ? p[i] : Number(0);
+#pragma unroll
+    for (int j = 1; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) u[j][i] = p[i + sy * j];
+    if (N1 == 3) {
+#pragma unroll
+      for (int j = 0; j < N1; ++j)
+#pragma unroll
+        for (int i = 0; i < N1; ++i) u[j][i] = row < 3 ? u[j][i] : Number(0);
+    }
+  };
+  int parity = 0;
+  for (int cy = cy0; cy < cy_end; ++cy) {
+    const bool last = cy + 1 == cy_end;  // the brick's top row is complete too
+    int pen = 0;
+    for (int cxb = cx0; cxb < cx_end; cxb += kNX, ++pen, parity ^= 1) {
+      const long cell = min(cxb + c, P.nc[0] - 1) + (long)P.nc[0] * (cy + (long)P.nc[1] * min(cz, P.nc[2] - 1));
+      Number u[N1][N1];
+      load_rows(src, cxb, cy, cy == cy0, u);
+      if (cy > cy0) {
+#pragma unroll
+        for (int i = 0; i < N1; ++i) u[0][i] = srow[wave][pen][i][lane];
+      }
+      if (!last) {
+#pragma unroll
+        for (int i = 0; i < N1; ++i) srow[wave][pen][i][lane] = u[K][i];
+      }
+      constrain(cxb, cy, u);
+
+      // ---- conductivity at the points of this lane's plane qz = l ----
+      const auto &A = fresh_args<BrickArgs<Number, N1>>();
+      using Vec = Number __attribute__((ext_vector_type(NV)));
+      Number kq[N1][N1];
+      Vec kraw[NLD];
+      Number kc = P.kappa;
+      if (KMODE == KAPPA_CELL) kc = A.kappa_arr[cell];
+      if constexpr (STAGE) {
+        const long first = cxb + (long)A.nc[0] * (cy + (long)A.nc[1] * min(bz * B::ZC + wave, A.nc[2] - 1));
+        const Vec *p = reinterpret_cast<const Vec *>(A.kappa_arr) + first * (NQ / NV);
+        // (a ragged row's last pencil reads into the next row's cells; the array's end is clamped)
+        const long left = (A.n_cells - first) * (NQ / NV);
+        if (left >= 64 * NLD) {
+#pragma unroll
+          for (int m = 0; m < NLD; ++m) kraw[m] = __builtin_nontemporal_load(p + 64 * m + lane);
+        } else {
+#pragma unroll
+          for (int m = 0; m < NLD; ++m) kraw[m] = p[min((long)(64 * m + lane), left - 1)];
+        }
+      } else if (KMODE == KAPPA_QP) {
+        const Number *p = A.kappa_arr + cell * NQ + N1 * N1 * min(l, K);
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) kq[j][i] = p[N1 * j + i];
+      }
+      if (KMODE == KAPPA_LAW) {
+        Number a[N1][N1], t[N1][N1];
+        load_rows(P.T, cxb, cy, true, a);
+        sweep_x<N1, false, false>(P.S, a, t);
+        sweep_y<N1, false, false>(P.S, t, a);
+        z_forward<N1, false>(P.S, P.G, zt, a, t, t);
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) kq[j][i] = law_kappa<Number>(P.law, P.law_p, t[j][i]);
+      }
+      Number v[N1][N1];
+      if constexpr (TENSOR) {
+        // J u = M_x [M_y (c_m M_z + k k_z K_z) + k k_y K_y M_z] u + k k_x K_x M_y M_z u
+        Number mz[N1][N1], p[N1][N1];
+        z_forward<N1, true>(P.M1, P.K1, zt, u, mz, p);
+        if (N1 == 3 && KMODE == KAPPA_CELL) kc = row < 3 ? kc : Number(0);
+        const Number kx = kc * P.kx, ky = kc * P.ky, kz = kc * P.kz;
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) p[j][i] = fma(P.cm, mz[j][i], kz * p[j][i]);
+        Number s[N1][N1];
+        sweep_y<N1, false, false>(P.M1, mz, u);
+        sweep_y<N1, false, false>(P.M1, p, s);
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) {
+            mz[j][i] *= ky;
+            u[j][i] *= kx;
+          }
+        sweep_y<N1, false, true>(P.K1, mz, s);
+        sweep_x<N1, false, false>(P.M1, s, v);
+        sweep_x<N1, false, true>(P.K1, u, v);
+      } else {
+        // ---- to the points: v = values, gz = z derivative ----
+        Number gz[N1][N1], e[N1][N1];
+        {
+          Number t[N1][N1];
+          sweep_x<N1, false, false>(P.S, u, t);
+          sweep_y<N1, false, false>(P.S, t, u);
+          z_forward<N1, true>(P.S, P.G, zt, u, v, gz);
+        }
+        // ---- at the points (heat_diffuse_operator.cpp:1029-1077): e = c_m W v + D_x^T f_x + D_y^T f_y,
+        //      gz becomes f_z ----
+        if (MAPPED) {
+          Number gx[N1][N1], gy[N1][N1];
+          sweep_x<N1, false, false>(P.D, v, gx);
+          sweep_y<N1, false, false>(P.D, v, gy);
+          const long pencil = cxb / kNX + (long)((P.nc[0] + kNX - 1) / kNX) * (cy + (long)P.nc[1] * min(cz, P.nc[2] - 1));
+          const Number *M = P.metric + (pencil * 7 * NQ + min(l, K)) * kNX + min(c, P.nc[0] - 1 - cxb);  // (metric_at)
+          const bool idle = N1 == 3 && row == 3;
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) {
+              const Number *m = M + (N1 * j + i) * N1 * kNX;
+              constexpr int C1 = NQ * kNX;
+              const Number g00 = m[C1], g01 = m[2 * C1], g11 = m[3 * C1], g02 = m[4 * C1], g12 = m[5 * C1], g22 = m[6 * C1];
+              const Number x = gx[j][i], y = gy[j][i], z = gz[j][i];
+              e[j][i] = P.cm * m[0] * v[j][i];
+              gx[j][i] = kc * (g00 * x + g01 * y + g02 * z);
+              gy[j][i] = kc * (g01 * x + g11 * y + g12 * z);
+              gz[j][i] = kc * (g02 * x + g12 * y + g22 * z);
+              if (idle) e[j][i] = gx[j][i] = gy[j][i] = gz[j][i] = Number(0);
+            }
+          sweep_x<N1, true, true>(P.D, gx, e);
+          sweep_y<N1, true, true>(P.Dy, gy, e);
+        } else {
+          if constexpr (STAGE) {
+            // the 16-byte chunks of a 128-byte line are permuted by the cell's index, so that all lanes'
+            // reads of chunk p spread over the banks
+            Number *kb = buf[wave];
+#pragma unroll
+            for (int m = 0; m < NLD; ++m) {
+              const int slot = 64 * m + lane, cc = slot / PER, ch = slot % PER;
+              *reinterpret_cast<Vec *>(kb + (PER * cc + (ch ^ (cc & 7))) * NV) = kraw[m];
+            }
+            lds_fence();
+#pragma unroll
+            for (int p = 0; p < CH; ++p) {
+              const Vec t = *reinterpret_cast<const Vec *>(kb + (PER * c + ((CH * row + p) ^ (c & 7))) * NV);
+#pragma unroll
+              for (int a = 0; a < NV; ++a) kq[(p * NV + a) / N1][(p * NV + a) % N1] = t[a];
+            }
+            lds_fence();
+          }
+          // weights of the lane's points: products of the few distinct 1D weights
+          constexpr int H = (N1 + 1) / 2;
+          const Number wk = wz * P.kx;
+          const Number wm = wz * P.cm;
+          Number wks[H][H], wms[H][H];
+#pragma unroll
+          for (int a = 0; a < H; ++a)
+#pragma unroll
+            for (int d = 0; d <= a; ++d) {
+              wks[a][d] = wks[d][a] = (P.w[a] * P.w[d]) * wk;
+              wms[a][d] = wms[d][a] = (P.w[a] * P.w[d]) * wm;
+            }
+          auto half = [](int i) { return i < N1 - 1 - i ? i : N1 - 1 - i; };
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) {
+              const Number w = wks[half(j)][half(i)];
+              kq[j][i] = w * kq[j][i];
+              if (N1 == 3 && row == 3) kq[j][i] = Number(0);
+              gz[j][i] *= kq[j][i];
+            }
+          // x derivative and flux row by row, with the mass term
+#pragma unroll
+          for (int j = 0; j < N1; ++j) {
+            Number f[N1];
+#pragma unroll
+            for (int q = 0; q < N1; ++q) {
+              Number g = 0;
+#pragma unroll
+              for (int i = 0; i < N1; ++i) g = fma(P.D(q, i), v[j][i], g);
+              f[q] = kq[j][q] * g;
+            }
+#pragma unroll
+            for (int i = 0; i < N1; ++i) {
+              Number a = wms[half(j)][half(i)] * v[j][i];
+#pragma unroll
+              for (int q = 0; q < N1; ++q) a = fma(P.D(q, i), f[q], a);
+              e[j][i] = a;
+            }
+          }
+          // y derivative and flux column by column
+#pragma unroll
+          for (int i = 0; i < N1; ++i) {
+            Number f[N1];
+#pragma unroll
+            for (int q = 0; q < N1; ++q) {
+              Number g = 0;
+#pragma unroll
+              for (int j = 0; j < N1; ++j) g = fma(P.D(q, j), v[j][i], g);
+              f[q] = kq[q][i] * g;
+            }
+#pragma unroll
+            for (int j = 0; j < N1; ++j) {
+              Number a = e[j][i];
+#pragma unroll
+              for (int q = 0; q < N1; ++q) a = fma(P.Dy(q, j), f[q], a);
+              e[j][i] = a;
+            }
+          }
+        }
+        // ---- back to the DoFs ----
+        z_backward<N1>(P, zt, e, gz, v);
+        sweep_y<N1, true, false>(P.S, v, e);
+        sweep_x<N1, true, false>(P.S, e, v);
+      }
+      // ---- sums over the brick's cells ----
+      const int f = opaque(flags);
+      double r[N1][N1];
+#pragma unroll
+      for (int j = 0; j < N1; ++j)
+#pragma unroll
+        for (int i = 0; i < N1; ++i) r[j][i] = (double)v[j][i];
+      double(&yr)[N1][64] = yrow[wave][pen];
+      if (cy > cy0) {
+#pragma unroll
+        for (int i = 0; i < N1; ++i) r[0][i] += yr[i][lane];
+      }
+      if (!last) {
+#pragma unroll
+        for (int i = 0; i < N1; ++i) yr[i][lane] = r[K][i];
+      }
+#pragma unroll
+      for (int j = 0; j < N1; ++j) {
+        if (j == K && !last) continue;
+        r[j][0] += from_previous_cell(r[j][K], pen > 0 ? xcol[wave][j][row] : 0.0);
+      }
+      if (cxb + kNX < cx_end && (f & F_LAST)) {
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+          if (j < K || last) xcol[wave][j][row] = r[j][K];
+      }
+      double(&tp)[B::ZC][K][N1][kNX] = top[parity];
+      if (f & F_TOP) {
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) tp[zc][j][i][c] = r[j][i];
+      }
+      __syncthreads();
+      if (f & F_LOW) {
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) r[j][i] += tp[zc - 1][j][i][c];
+      }
+      if (last) {  // the top row takes another round
+        __syncthreads();
+        if (f & F_TOP) {
+#pragma unroll
+          for (int i = 0; i < N1; ++i) tp[zc][0][i][c] = r[K][i];
+        }
+        __syncthreads();
+        if (f & F_LOW) {
+#pragma unroll
+          for (int i = 0; i < N1; ++i) r[K][i] += tp[zc - 1][0][i][c];
+        }
+      }
+      const auto &Z = fresh_args<BrickArgs<Number, N1>>();
+      const bool hy = cy != Z.nc[1] - 1;  // the top row is not the mesh's
+      constrain(cxb, cy, r);
+
+      // ---- store rows 0..K-1, and the top row after the last step: to dst, or to the class of the
+      //      brick's upper y / z plane ----
+      if constexpr (K == 1) {
+        // the lanes already hold consecutive columns
+        const int cx = cxb + c;
+        if ((f & F_STORE) && cx < Z.nc[0]) {
+          const bool hz = f & F_HZ;
+          Number *o = (hz ? Z.scratch + Z.g.off[4] + (long)bz * sz : dst + sz * iz) + cx;
+          o[sy * cy] = (Number)r[0][0];
+          if (last) {
+            Number *t = !hy ? o + sy * (cy + 1)
+                            : Z.scratch + (hz ? Z.g.off[6] + ((long)by + (long)(Z.g.nb[1] - 1) * bz) * sy
+                                              : Z.g.off[2] + ((long)by + (long)(Z.g.nb[1] - 1) * iz) * sy) + cx;
+            *t = (Number)r[1][0];
+          }
+        }
+      } else {
+        constexpr int RPI = 64 / W;    // rows stored at a time
+        Number *const tl = buf[wave];  // [lane row][j of RPI][x]
+        const int x = lane % W, jr = lane / W, czw = bz * B::ZC + wave;
+        if (czw < Z.nc[2]) {
+          const long at = sy * ((long)K * cy) + K * cxb;  // uniform
+          const int mine = x + (int)sy * jr;
+          const bool st = jr < RPI && x < K * (cx_end - cxb);
+          Number *o = dst + (sz * (K * czw) + at) + mine;
+          const bool end = czw == Z.nc[2] - 1;
+          Number *oz = end ? o + sz * K : Z.scratch + (Z.g.off[4] + (long)bz * sz + at) + mine;
+          const Number *t = tl + lane;
+#pragma unroll
+          for (int j = 0; j < K; j += RPI) {
+#pragma unroll
+            for (int k = j; k < j + RPI; ++k)
+#pragma unroll
+              for (int i = 0; i < K; ++i) tl[(row * RPI + k - j) * W + K * c + i] = (Number)r[k][i];
+            lds_fence();
+            if (st) {
+#pragma unroll
+              for (int rw = 0; rw < K; ++rw) o[sz * rw + sy * j] = t[rw * RPI * W];
+              if (end || wave == kNW - 1) oz[sy * j] = t[K * RPI * W];
+            }
+            lds_fence();
+          }
+          if (last) {
+#pragma unroll
+            for (int i = 0; i < K; ++i) tl[row * W + K * c + i] = (Number)r[K][i];
+            lds_fence();
+#pragma unroll
+            for (int rw = 0; rw < N1; ++rw) {
+              const int z = K * czw + rw;
+              const bool up = rw == K && czw != Z.nc[2] - 1;
+              if (up && wave != kNW - 1) continue;
+              Number *p;
+              if (hy)
+                p = Z.scratch + (up ? Z.g.off[6] + ((long)by + (long)(Z.g.nb[1] - 1) * bz) * sy
+                                    : Z.g.off[2] + ((long)by + (long)(Z.g.nb[1] - 1) * z) * sy);
+              else
+                p = (up ? Z.scratch + Z.g.off[4] + (long)bz * sz : dst + sz * z) + sy * ((long)K * cy + K);
+              if (jr == 0 && x < K * (cx_end - cxb)) p[K * cxb + x] = tl[rw * W + x];
+            }
+            lds_fence();
+          }
+        }
+      }
+      // ---- column K of the brick's last cells: to dst at the mesh's end, else to the x classes ----
+      if (cxb + kNX >= cx_end) {
+        const int cx = cxb + c;
+        if ((f & F_STORE) && cx == cx_end - 1) {
+          const bool hx = cx_end != Z.nc[0], hz = f & F_HZ;
+          const long ny1 = Z.g.nb[1] - 1, nz1 = Z.g.nb[2] - 1;
+#pragma unroll
+          for (int j = 0; j < N1; ++j) {
+            if (j == K && !last) continue;
+            const bool y = j == K && hy;
+            const int iy = K * cy + j;
+            Number *o;
+            if (hx) {
+              if (y) o = Z.scratch + (hz ? Z.g.off[7] + (bx * ny1 + by) * nz1 + bz : Z.g.off[3] + (bx * ny1 + by) * Z.nd[2] + iz);
+              else o = Z.scratch + (hz ? Z.g.off[5] + (bx * nz1 + bz) * Z.nd[1] + iy : Z.g.off[1] + ((long)bx * Z.nd[2] + iz) * Z.nd[1] + iy);
+            } else {
+              if (y) o = Z.scratch + (hz ? Z.g.off[6] + (by + ny1 * bz) * sy : Z.g.off[2] + (by + ny1 * iz) * sy);
+              else o = (hz ? Z.scratch + Z.g.off[4] + (long)bz * sz : dst + sz * iz) + sy * iy;
+              o += K * cx + K;
+            }
+            *o = (Number)r[j][K];
+          }
+        }
+      }
+    }
+  }
+}
+
+// dst += the classes of the planes bricks share, in class order (sums in FP64). A wavefront takes up
+// to 64 kFixup DoFs of a line: of an x row of the shared z planes, then of the shared y planes (rows
+// off the z planes), then of a y line of the shared x planes (off both). All its loads are issued
+// before the sums and stores.
+constexpr int kFixup = 4;
+template <typename Number>
+__global__ __launch_bounds__(256) void brick_fixup_kernel(Number *__restrict__ dst, const Number *__restrict__ scratch,
+                                                          BrickGrid g, int K, int nd0, int nd1, int nd2, int parts) {
+  const int lane = threadIdx.x & 63;
+  long line = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int i0 = (int)(line % parts) * (64 * kFixup) + lane;
+  line /= parts;
+  const long nz = (long)(g.nb[2] - 1) * nd1, ny = (long)(g.nb[1] - 1) * nd2, nx = (long)(g.nb[0] - 1) * nd2;
+  const int px = K * g.cells[0], py = K * g.cells[1], pz = K * g.cells[2];
+  const long sy = nd0, sz = (long)nd0 * nd1;
+  // the shared plane a coordinate lies on (-1: none): the multiples of p inside the mesh
+  auto plane = [](int i, int p, int nb) { return i > 0 && i % p == 0 && i / p < nb ? i / p - 1 : -1; };
+  int iy = -1, iz = -1, hy = -1, hz = -1;
+  if (line < nz) {
+    hz = (int)(line / nd1);
+    iy = (int)(line - (long)hz * nd1);
+    iz = pz * (hz + 1);
+    hy = plane(iy, py, g.nb[1]);
+  } else if ((line -= nz) < ny) {
+    iz = (int)(line / (g.nb[1] - 1));
+    hy = (int)(line - (long)iz * (g.nb[1] - 1));
+    iy = py * (hy + 1);
+    if (plane(iz, pz, g.nb[2]) >= 0) return;
+  } else if ((line -= ny) < nx) {
+    const int hx = (int)(line / nd2);
+    iz = (int)(line - (long)hx * nd2);
+    if (plane(iz, pz, g.nb[2]) >= 0) return;
+    const Number *s = scratch + g.off[1] + line * nd1;
+    Number *d = dst + (long)px * (hx + 1) + sz * iz;
+    Number a[kFixup], b[kFixup];
+#pragma unroll
+    for (int t = 0; t < kFixup; ++t) {
+      const int i = min(i0 + 64 * t, nd1 - 1);
+      a[t] = d[sy * i];
+      b[t] = s[i];
+    }
+#pragma unroll
+    for (int t = 0; t < kFixup; ++t) {
+      const int i = i0 + 64 * t;
+      if (i < nd1 && plane(i, py, g.nb[1]) < 0) d[sy * i] = (Number)((double)a[t] + (double)b[t]);
+    }
+    return;
+  } else {
+    return;
+  }
+  Number *d = dst + sy * iy + sz * iz;
+  const Number *cy = scratch + g.off[2] + (hy + (long)(g.nb[1] - 1) * iz) * nd0;
+  const Number *cz = scratch + g.off[4] + ((long)hz * nd1 + iy) * nd0;
+  const Number *cyz = scratch + g.off[6] + (hy + (long)(g.nb[1] - 1) * hz) * nd0;
+  Number a[kFixup], b[kFixup], e[kFixup], f[kFixup];
+#pragma unroll
+  for (int t = 0; t < kFixup; ++t) {
+    const int ix = min(i0 + 64 * t, nd0 - 1);
+    a[t] = d[ix];
+    b[t] = hy >= 0 ? cy[ix] : Number(0);
+    e[t] = hz >= 0 ? cz[ix] : Number(0);
+    f[t] = hy >= 0 && hz >= 0 ? cyz[ix] : Number(0);
+  }
+#pragma unroll
+  for (int t = 0; t < kFixup; ++t) {
+    const int ix = i0 + 64 * t;
+    if (ix >= nd0) continue;
+    const int hx = plane(ix, px, g.nb[0]);
+    double s = (double)a[t];
+    if (hx >= 0) s += (double)scratch[g.off[1] + ((long)hx * nd2 + iz) * nd1 + iy];
+    s += (double)b[t];
+    if (hx >= 0 && hy >= 0) s += (double)scratch[g.off[3] + ((long)hx * (g.nb[1] - 1) + hy) * nd2 + iz];
+    s += (double)e[t];
+    if (hx >= 0 && hz >= 0) s += (double)scratch[g.off[5] + ((long)hx * (g.nb[2] - 1) + hz) * nd1 + iy];
+    s += (double)f[t];
+    if (hx >= 0 && hy >= 0 && hz >= 0)
+      s += (double)scratch[g.off[7] + ((long)hx * (g.nb[1] - 1) + hy) * (g.nb[2] - 1) + hz];
+    d[ix] = (Number)s;
+  }
+}
+
+template <int N1, typename Number>
+int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
+                    hipEvent_t kernel_start, hipEvent_t kernel_end) {
+  BrickArgs<Number, N1> A;
+  const FE1D &fe = fe1d(N1 - 1);
+  const bool mapped = op.metric != nullptr;
+  const double vol = mapped ? 1.0 : op.h[0] * op.h[1] * op.h[2];
+  double Dy[kMaxN1][kMaxN1], Gz[kMaxN1][kMaxN1];
+  const double ry = mapped ? 1.0 : (op.h[0] * op.h[0]) / (op.h[1] * op.h[1]);
+  const double rz = mapped ? 1.0 : (op.h[0] * op.h[0]) / (op.h[2] * op.h[2]);
+  for (int q = 0; q < N1; ++q)
+    for (int i = 0; i < N1; ++i) {
+      Dy[q][i] = fe.D[q][i] * ry;
+      Gz[q][i] = fe.G[q][i] * rz;
+    }
+  A.S.set(fe.S);
+  A.D.set(fe.D);
+  A.G.set(fe.G);
+  A.Dy.set(Dy);
+  A.Gz.set(Gz);
+  for (int a = 0; 2 * a < N1; ++a) A.w[a] = (Number)fe.qw[a];
+  for (int d = 0; d < 3; ++d) {
+    A.nc[d] = op.nc[d];
+    A.nd[d] = op.nd[d];
+  }
+  A.n_cells = op.n_cells;
+  A.g = brick_grid(N1 - 1, op.nc);
+  A.dmask = op.dmask;
+  A.law = op.law;
+  A.cm = (Number)(op.c_mass * vol);
+  A.kx = (Number)(mapped ? 1.0 : vol / (op.h[0] * op.h[0]));
+  A.ky = (Number)(mapped ? 1.0 : vol / (op.h[1] * op.h[1]));
+  A.kz = (Number)(mapped ? 1.0 : vol / (op.h[2] * op.h[2]));
+  double M1[kMaxN1][kMaxN1] = {}, K1[kMaxN1][kMaxN1] = {};
+  for (int i = 0; i < N1; ++i)
+    for (int j = 0; j < N1; ++j)
+      for (int q = 0; q < N1; ++q) {
+        M1[i][j] += fe.S[q][i] * fe.qw[q] * fe.S[q][j];
+        K1[i][j] += fe.G[q][i] * fe.qw[q] * fe.G[q][j];
+      }
+  A.M1.set(M1);
+  A.K1.set(K1);
+  A.kappa = (Number)op.kappa;
+  for (int i = 0; i < 4; ++i) A.law_p[i] = (Number)op.law_p[i];
+  A.kappa_arr = op.kappa_arr;
+  A.T = op.T;
+  A.metric = op.metric;
+  A.scratch = op.edge;
+  if (A.g.total > 0 && (op.edge == nullptr || (size_t)A.g.total > op.edge_elems)) return MPDG_ERR_INVALID;
+  const dim3 grid((unsigned)((long)A.g.nb[0] * A.g.nb[1] * A.g.nb[2])), block(64 * kNW);
+  if (kernel_start) (void)hipEventRecord(kernel_start, stream);
+#define MPDG_BRICK(KM, MP) hipLaunchKernelGGL((heat_brick_kernel<N1, Number, KM, MP>), grid, block, 0, stream, A, src, dst)
+  if (mapped) {
+    switch (op.kappa_mode) {
+      case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, true); break;
+      case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, true); break;
+      default: return MPDG_ERR_INVALID;  // per-qp conductivity on mapped meshes runs through metric_k
+    }
+  } else {
+    switch (op.kappa_mode) {
+      case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, false); break;
+      case KAPPA_QP: MPDG_BRICK(KAPPA_QP, false); break;
+      case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, false); break;
+      case KAPPA_LAW: MPDG_BRICK(KAPPA_LAW, false); break;
+      default: return MPDG_ERR_INVALID;
+    }
+  }
+#undef MPDG_BRICK
+  if (kernel_end) (void)hipEventRecord(kernel_end, stream);
+  const long lines = (long)(A.g.nb[2] - 1) * op.nd[1] + (long)(A.g.nb[1] - 1) * op.nd[2] + (long)(A.g.nb[0] - 1) * op.nd[2];
+  const int longest = A.g.nb[0] > 1 ? std::max(op.nd[0], op.nd[1]) : op.nd[0];
+  const int parts = (longest + 64 * kFixup - 1) / (64 * kFixup);
+  if (lines > 0)
+    hipLaunchKernelGGL(brick_fixup_kernel<Number>, dim3((unsigned)((lines * parts + 3) / 4)), dim3(256), 0, stream, dst,
+                       op.edge, A.g, N1 - 1, op.nd[0], op.nd[1], op.nd[2], parts);
+  return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
+}
+
+}  // namespace
+
+size_t brick_scratch_elems(int degree, const int *nc) { return (size_t)brick_grid(degree, nc).total; }
+
+template <typename Number>
+int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
+                 hipEvent_t kernel_start, hipEvent_t kernel_end) {
+  switch (op.degree) {
+    case 1: return launch_brick_n1<2, Number>(op, src, dst, stream, kernel_start, kernel_end);
+    case 2: return launch_brick_n1<3, Number>(op, src, dst, stream, kernel_start, kernel_end);
+    case 3: return launch_brick_n1<4, Number>(op, src, dst, stream, kernel_start, kernel_end);
+    default: return MPDG_ERR_INVALID;
+  }
+}
+template int launch_brick<double>(const OperatorData<double> &, const double *, double *, hipStream_t, hipEvent_t, hipEvent_t);
+template int launch_brick<float>(const OperatorData<float> &, const float *, float *, hipStream_t, hipEvent_t, hipEvent_t);
+
+}  // namespace mpdg

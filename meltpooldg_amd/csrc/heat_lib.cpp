@@ -24,11 +24,11 @@ inline int dev_ok() { return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ER
 int mpdg_heat_op::ensure_edge() const {
   const size_t n = apply_edge_elems(d64.degree, d64.nc, precision == MPDG_FP32);
   if (precision == MPDG_FP64) {
-    MPDG_TRY(edge64.resize_zeroed(n));
+    MPDG_TRY(d64.degree < 4 ? edge64.resize(n) : edge64.resize_zeroed(n));
     d64.edge = edge64.get();
     d64.edge_elems = n;
   } else {
-    MPDG_TRY(edge32.resize_zeroed(n));
+    MPDG_TRY(d64.degree < 4 ? edge32.resize(n) : edge32.resize_zeroed(n));
     d32.edge = edge32.get();
     d32.edge_elems = n;
   }
@@ -61,13 +61,13 @@ int mpdg_heat_op::refresh_metric_k(hipStream_t s) const {
   const size_t nq = (size_t)d64.n_cells * n1 * n1 * n1;
   if (precision == MPDG_FP64) {
     MPDG_TRY(kq.resize(nq));
-    MPDG_TRY(metric64_k.resize(nq * 7));
+    MPDG_TRY(metric64_k.resize(metric_elems(n1, d64.nc)));
     MPDG_TRY(launch_kappa_qp<double>(d64, kq.get(), s));
     MPDG_TRY(launch_scale_metric<double>(d64, kq.get(), metric64_k.get(), s));
     d64.metric_k = metric64_k.get();
   } else {
     MPDG_TRY(kq32.resize(nq));
-    MPDG_TRY(metric32_k.resize(nq * 7));
+    MPDG_TRY(metric32_k.resize(metric_elems(n1, d64.nc)));
     MPDG_TRY(launch_kappa_qp<float>(d32, kq32.get(), s));
     MPDG_TRY(launch_scale_metric<float>(d32, kq32.get(), metric32_k.get(), s));
     d32.metric_k = metric32_k.get();
@@ -164,7 +164,7 @@ int mpdg_heat_op::create_rhs(double *dst, const double *T, const double *T_old, 
       const int n1 = d64.degree + 1;
       const size_t nq = (size_t)d64.n_cells * n1 * n1 * n1;
       MPDG_TRY(kq.resize(nq));
-      MPDG_TRY(metric64_k.resize(nq * 7));
+      MPDG_TRY(metric64_k.resize(metric_elems(n1, d64.nc)));
       MPDG_TRY(launch_kappa_qp<double>(jt, kq.get(), s));
       MPDG_TRY(launch_scale_metric<double>(jt, kq.get(), metric64_k.get(), s));
       jt.metric_k = metric64_k.get();
@@ -548,7 +548,7 @@ struct GMGPrecond : mpdg_precond {
     }
     for (auto &L : lev) {
       const int n1 = L->od.degree + 1;
-      MPDG_TRY(L->metric.resize((size_t)L->od.n_cells * 7 * n1 * n1 * n1));
+      MPDG_TRY(L->metric.resize(metric_elems(n1, L->od.nc)));
       MPDG_TRY(launch_metric<T>(L->od, L->coords.get(), L->metric.get(), nullptr));
       L->od.metric = L->metric.get();
       L->od.coords = L->coords.get();
@@ -591,7 +591,7 @@ struct GMGPrecond : mpdg_precond {
       const int n1 = top.od.degree + 1;
       const size_t nq = (size_t)top.od.n_cells * n1 * n1 * n1;
       MPDG_TRY(top.kq_scratch.resize(nq));
-      MPDG_TRY(top.metric_k.resize(nq * 7));
+      MPDG_TRY(top.metric_k.resize(metric_elems(n1, top.od.nc)));
       MPDG_TRY(launch_kappa_qp<T>(top.od, top.kq_scratch.get(), s));
       MPDG_TRY(launch_scale_metric<T>(top.od, top.kq_scratch.get(), top.metric_k.get(), s));
       top.od.metric_k = top.metric_k.get();
@@ -1150,6 +1150,9 @@ int mpdg_heat_op_create(const mpdg_heat_desc *desc, mpdg_heat_op **out) {
   op->d32.set_mesh(desc->degree, desc->n_cells, desc->extent);
   op->d64.dmask = op->d32.dmask = desc->dirichlet_faces & 63;
   op->d64.c_mass = op->d32.c_mass = desc->rho_cp;  // dt = 1 until reset_time_increment
+  // the apply's scratch, so that mpdg_heat_op_vmult_noalloc finds it; where there is no room (or no
+  // device yet) the first apply tries again and reports the error
+  if (op->precision == MPDG_FP64 && desc->degree < 4 && op->ensure_edge() != MPDG_OK) (void)hipGetLastError();
   *out = op;
   return MPDG_OK;
 }
@@ -1217,7 +1220,7 @@ int mpdg_heat_op_set_robin(mpdg_heat_op *op, int mask, double alpha, double T_in
 int mpdg_heat_op_set_mapping(mpdg_heat_op *op, const double *coords) {
   if (!op || !coords) return MPDG_ERR_INVALID;
   const int n1 = op->d64.degree + 1;
-  const size_t nm = (size_t)op->d64.n_cells * 7 * n1 * n1 * n1;
+  const size_t nm = metric_elems(n1, op->d64.nc);
   op->coords = coords;
   op->d64.coords = op->d32.coords = coords;
   if (op->precision == MPDG_FP64) {
@@ -1312,10 +1315,10 @@ int mpdg_heat_op_vmult(const mpdg_heat_op *op, double *dst, const double *src, v
 // ---------------------------------------------------------------------------
 // vmult without allocation (mpdg_heat_op_vmult_noalloc)
 // ---------------------------------------------------------------------------
-// The apply's only scratch is the edge buffer (rows where four columns meet). Here it lives
-// in a fixed device array of kNoAllocScratchDoubles doubles (8 MiB), one copy per GPU, held
-// until the process ends. Every call on a GPU uses that GPU's copy: calls that overlap on one
-// GPU (other streams, other threads) race.
+// Q1..Q3: the operator's own scratch, allocated when it is created. Q4: the apply's scratch (rows
+// where four columns meet) lives in a fixed device array of kNoAllocScratchDoubles doubles (8 MiB), one
+// copy per GPU, held until the process ends. Every Q4 call on a GPU uses that GPU's copy: calls that
+// overlap on one GPU (other streams, other threads) race.
 constexpr size_t kNoAllocScratchDoubles = size_t(1) << 20;
 static __device__ __align__(256) double scratch[kNoAllocScratchDoubles];
 
@@ -1341,6 +1344,15 @@ int scratch_address(double **out) {
 }
 }  // namespace
 
+// The measure of a mesh that the fixed maximum of vmult_noalloc is compared with: DoF rows along x
+// where four columns of BY x BZ cells meet.
+static size_t noalloc_measure(int degree, const int *nc, bool mapped) {
+  static const int by[5] = {0, 4, 3, 4, 4}, bz[5] = {0, 4, 2, 2, 3};
+  const int y = mapped && degree == 3 ? 2 : by[degree];
+  const long rows = (long)((nc[1] + y - 1) / y - 1) * ((nc[2] + bz[degree] - 1) / bz[degree] - 1);
+  return (size_t)(rows * ((long)degree * nc[0] + 1));
+}
+
 int mpdg_heat_op_vmult_noalloc(const mpdg_heat_op *op, double *dst, const double *src, void *stream) {
   if (!op || !dst || !src || op->precision != MPDG_FP64) return MPDG_ERR_INVALID;
   hipStream_t s = S(stream);
@@ -1354,11 +1366,19 @@ int mpdg_heat_op_vmult_noalloc(const mpdg_heat_op *op, double *dst, const double
       // already exist at their size (an earlier vmult made them), so that nothing is allocated
       const int n1 = op->d64.degree + 1;
       const size_t nq = (size_t)op->d64.n_cells * n1 * n1 * n1;
-      if (op->kq.n != nq || op->metric64_k.n != nq * 7) return MPDG_ERR_INVALID;
+      if (op->kq.n != nq || op->metric64_k.n != metric_elems(n1, op->d64.nc)) return MPDG_ERR_INVALID;
       MPDG_TRY(op->refresh_metric_k(s));
     }
-    const size_t need = apply_edge_elems(op->d64.degree, op->d64.nc, false, op->d64.metric ? 1 : 0);
-    if (need > kNoAllocScratchDoubles) return MPDG_ERR_TOO_LARGE;
+    if (noalloc_measure(op->d64.degree, op->d64.nc, op->d64.metric != nullptr) > kNoAllocScratchDoubles)
+      return MPDG_ERR_TOO_LARGE;
+    if (op->d64.degree < 4) {
+      // the operator's scratch, allocated when it was created
+      if (op->d64.edge_elems != apply_edge_elems(op->d64.degree, op->d64.nc, false)) return MPDG_ERR_NOMEM;
+      MPDG_TRY(launch_apply<double>(op->d64, src, dst, s));
+      if (op->d64.robin_mask) MPDG_TRY(launch_boundary(op->d64, 0, nullptr, dst, src, op->T_robin, s));
+      return MPDG_OK;
+    }
+    const size_t need = apply_edge_elems(op->d64.degree, op->d64.nc, false);
     double *scr = nullptr;
     MPDG_TRY(scratch_address(&scr));
     OperatorData<double> od = op->d64;

@@ -14,6 +14,18 @@ namespace mpdg {
 enum KappaMode { KAPPA_CONST = MPDG_KAPPA_CONST, KAPPA_QP = MPDG_KAPPA_QP, KAPPA_CELL = MPDG_KAPPA_CELL, KAPPA_LAW = MPDG_KAPPA_LAW };
 enum LawId { LAW_TANH = MPDG_LAW_TANH, LAW_MUSHY = MPDG_LAW_MUSHY };
 
+template <typename Number>
+__device__ __forceinline__ Number law_kappa(int law, const Number *p, Number T) {
+  if (law == LAW_TANH) {
+    return p[0] * (Number(1) + p[1] * tanh((T - p[2]) / p[3]));
+  }
+  // mushy zone (liquid_solid): p = {k_liquid, k_solid, T_solidus, T_liquidus}
+  const Number inv = Number(1) / (p[3] - p[2]);
+  Number fs = (p[3] - T) * inv;
+  fs = fs < Number(0) ? Number(0) : (fs > Number(1) ? Number(1) : fs);
+  return p[0] + (p[1] - p[0]) * (Number(3) - Number(2) * fs) * fs * fs;
+}
+
 // Everything a level operator needs on the device (pointers are device memory).
 template <typename Number>
 struct OperatorData {
@@ -34,14 +46,15 @@ struct OperatorData {
   int robin_mask = 0;
   double alpha = 0, emissivity = 0, T_inf_conv = 0, T_inf_rad = 0;
   const double *T_robin = nullptr;  // temperature for the radiation linearisation (FP64)
-  // mapped geometry: per quadrature point [cell][7][q]: JxW, then G = JxW J^-1 J^-T as (00, 01, 11, 02, 12, 22)
+  // mapped geometry, 7 values per quadrature point (placed by metric_at): JxW, then G = JxW J^-1 J^-T as
+  // (00, 01, 11, 02, 12, 22)
   const Number *metric = nullptr;
   // metric with the conductivity folded in (kappa_q G), used for per-qp / k(T) conductivity on mapped meshes
   const Number *metric_k = nullptr;
   const double *coords = nullptr;   // mapping node coordinates (X block, Y block, Z block), FP64
-  // apply scratch: contributions of the upper z-layer of columns to the DoF rows where four
-  // columns meet, summed into dst after the cell kernel so that vmult is bitwise reproducible
-  // (apply_edge_elems Number entries, all zero between applies)
+  // apply scratch (apply_edge_elems Number entries): contributions to DoFs that workgroups share, summed
+  // into dst after the cell kernel so that vmult is bitwise reproducible. Q4: the rows where four
+  // columns meet, all zero between applies; Q1..Q3: the bricks' upper planes, written by every apply
   Number *edge = nullptr;
   size_t edge_elems = 0;
   void set_mesh(int k, const int *ncells, const double *ext) {
@@ -56,6 +69,21 @@ struct OperatorData {
     n_cells = (long)nc[0] * nc[1] * nc[2];
   }
 };
+
+// Where component comp of quadrature point q = (qx, qy, qz) of a cell's metric lies. Q1..Q3:
+// [pencil of 16 cells along x][comp][qy][qx][qz][cell of the pencil], so that each load of the apply's
+// wavefront (lane = 16 qz + cell) is contiguous (Q3 96^3 FP64 apply: 0.88 ms; 2.4 ms with [cell][comp][q],
+// where every lane reads its own line); Q4, whose kernel gives a lane consecutive qx: [cell][comp][q].
+__host__ __device__ __forceinline__ long metric_at(int n1, int nc0, long cell, int comp, int qx, int qy, int qz) {
+  const int nq = n1 * n1 * n1;
+  if (n1 == 5) return (cell * 7 + comp) * nq + qx + n1 * (qy + n1 * qz);
+  const long row = cell / nc0, cx = cell - row * nc0, pencil = row * ((nc0 + 15) / 16) + cx / 16;
+  return ((pencil * 7 + comp) * nq + (qy * n1 + qx) * n1 + qz) * 16 + cx % 16;
+}
+inline size_t metric_elems(int n1, const int *nc) {
+  const size_t cells_x = n1 == 5 ? nc[0] : (nc[0] + 15) / 16 * 16;
+  return cells_x * nc[1] * nc[2] * 7 * n1 * n1 * n1;
+}
 
 // A 1D N1 x N1 table stored by its symmetry about the cell centre (Gauss-Lobatto nodes and
 // Gauss points are symmetric): T[N1-1-q][N1-1-i] = T[q][i] (ANTI = false, shape values) or
@@ -122,10 +150,14 @@ void fill_apply_args(const OperatorData<Number> &op, ApplyArgs<Number, N1> &A) {
 template <typename Number>
 int launch_apply(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                  hipEvent_t kernel_start = nullptr, hipEvent_t kernel_end = nullptr);
-// entries of OperatorData::edge the apply of a mesh of degree k and n_cells cells needs with
-// the Cartesian (mapped = 0) or mapped (1) chunk shape, or the larger of the two (mapped = -1);
-// 0 when no DoF row is shared by four columns
-size_t apply_edge_elems(int degree, const int *n_cells, bool fp32, int mapped = -1);
+// entries of OperatorData::edge the apply of a mesh of degree k and n_cells cells needs
+size_t apply_edge_elems(int degree, const int *n_cells, bool fp32);
+
+// heat_brick.hip: the apply for Q1..Q3 and the scratch entries (OperatorData::edge) it needs
+template <typename Number>
+int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
+                 hipEvent_t kernel_start, hipEvent_t kernel_end);
+size_t brick_scratch_elems(int degree, const int *n_cells);
 
 // heat_aux.hip: diagonal, boundary faces, residual, norms, conductivity
 // diag = the operator's diagonal (cells only; constrained rows 1); scratch: 2 n_cells (k+1)^3 values

@@ -435,3 +435,55 @@ def test_node_coordinates_match_the_oracle_mapping(cuda, degree, nc, amp):
     X = M.node_coordinates(degree, nc, L, mapping_amplitude=amp).cpu().numpy()
     ref = orc.coords if amp else np.concatenate(orc.node_coords())
     assert np.max(np.abs(X - ref)) < 1e-14
+
+
+# edges of the apply's bricks: pencils of 16 cells along x (one, two, an odd number; ragged), 4 cells
+# along z (Q1: 8), one or several steps along y and pencils per brick, one brick in a direction
+BRICK_CASES = [(1, (1, 1, 1), "const", 0, 0), (1, (15, 2, 8), "cell", 0, 0b100001), (1, (17, 3, 9), "qp", 0, 0),
+               (2, (16, 4, 4), "cell", 0, 0b001100), (2, (33, 5, 5), "qp", 1, 0), (2, (31, 6, 3), "law", 0, 0b010010),
+               (3, (16, 3, 4), "qp", 0, 0), (3, (47, 2, 5), "cell", 1, 0b111111), (3, (1, 9, 7), "qp", 1, 0b000100),
+               (3, (33, 40, 140), "qp", 0, 0b100000), (2, (70, 65, 60), "const", 1, 0), (1, (40, 90, 120), "law", 0, 0)]
+
+
+@pytest.mark.parametrize("degree,nc,mode,precision,dmask", BRICK_CASES)
+def test_vmult_at_brick_edges(cuda, degree, nc, mode, precision, dmask):
+    torch = cuda
+    orc, gop, _ = make_pair(torch, degree, nc, mode=mode, precision=precision, dirichlet=dmask, seed=21)
+    x = np.random.default_rng(22).uniform(-1.0, 1.0, orc.n_dofs)
+    xd = torch.tensor(x, dtype=torch.float64 if precision == 0 else torch.float32, device="cuda")
+    yd = torch.full_like(xd, float("nan"))  # every entry is written
+    gop.vmult(yd, xd)
+    torch.cuda.synchronize()
+    assert rel_err(yd.cpu().numpy(), orc.vmult(xd.cpu().numpy().astype(np.float64))) < (1e-12 if precision == 0 else 1e-5)
+
+
+@pytest.mark.parametrize("degree,nc,mode", [(1, (18, 5, 9), "const"), (2, (17, 4, 5), "cell"), (3, (33, 3, 4), "const")])
+def test_mapped_vmult_and_diagonal_at_brick_edges(cuda, degree, nc, mode):
+    torch = cuda
+    orc, gop, _ = make_pair(torch, degree, nc, mode=mode, mapped=0.05, seed=23)
+    x = np.random.default_rng(24).uniform(-1.0, 1.0, orc.n_dofs)
+    yd = torch.full((orc.n_dofs,), float("nan"), dtype=torch.float64, device="cuda")
+    gop.vmult(yd, torch.tensor(x, device="cuda"))
+    d = torch.empty_like(yd)
+    gop.compute_diagonal(d)
+    torch.cuda.synchronize()
+    assert rel_err(yd.cpu().numpy(), orc.vmult(x)) < 1e-12
+    assert rel_err(d.cpu().numpy(), orc.diagonal()) < 1e-12
+
+
+def test_nonfinite_sources_stay_in_the_cells_that_hold_them(cuda):
+    """A NaN in one DoF reaches the DoFs of the cells that hold it and no others (nothing of one cell is
+    multiplied into another, as by the idle or paired lanes of a matrix instruction)."""
+    torch = cuda
+    for degree in (1, 2, 3):
+        nc = (18, 5, 9)
+        _, gop, _ = make_pair(torch, degree, nc, mode="qp", seed=25)
+        nd = [degree * n + 1 for n in nc]
+        x = torch.zeros(nd[2], nd[1], nd[0], dtype=torch.float64, device="cuda")
+        at = (degree * 4, degree * 2, degree * 15)  # z, y, x: a vertex of eight cells
+        x[at] = float("nan")
+        y = torch.empty_like(x)
+        gop.vmult(y.view(-1), x.view(-1))
+        want = torch.zeros_like(x, dtype=torch.bool)
+        want[tuple(slice(a - degree, a + degree + 1) for a in at)] = True
+        assert torch.equal(torch.isnan(y), want)
