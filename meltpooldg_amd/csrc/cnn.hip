@@ -31,18 +31,51 @@ __device__ __forceinline__ float bf16_to_f32(unsigned short h) { return __uint_a
 // four consecutive bf16 values (8-byte aligned) as the MFMA operand, in one 8-byte load
 __device__ __forceinline__ bf16x4 load4(const unsigned short *p) { return *reinterpret_cast<const bf16x4 *>(p); }
 
+// A brick of voxels per workgroup, one wavefront per z plane: its voxels and their neighbours are staged
+// in LDS as they lie in memory (32 bytes per voxel; zero outside the grid).
+constexpr int kBrX = 16, kBrY = 4, kBrZ = 4;
+constexpr int kBrIn = (kBrX + 2) * (kBrY + 2) * (kBrZ + 2), kBrOut = kBrX * kBrY * kBrZ;
+struct Bricks {
+  int nx, ny, nz, bx, by, bz;
+  __host__ __device__ Bricks(int x, int y, int z)
+      : nx(x), ny(y), nz(z), bx((x + kBrX - 1) / kBrX), by((y + kBrY - 1) / kBrY), bz((z + kBrZ - 1) / kBrZ) {}
+  __host__ __device__ long count() const { return (long)bx * by * bz; }
+  __device__ void origin(long b, int &x0, int &y0, int &z0) const {
+    x0 = (int)(b % bx) * kBrX;
+    y0 = (int)((b / bx) % by) * kBrY;
+    z0 = (int)(b / ((long)bx * by)) * kBrZ;
+  }
+};
+// SX x SY x SZ voxels from (x0, y0, z0), 16 bytes (half the channels of a voxel) per thread and turn
+template <int SX, int SY, int SZ>
+__device__ __forceinline__ void stage_voxels(const Bricks &B, const unsigned short *__restrict__ in, unsigned short *s,
+                                             int x0, int y0, int z0) {
+#pragma unroll
+  for (int k = 0; k < (2 * SX * SY * SZ + 255) / 256; ++k) {
+    const int i = (int)threadIdx.x + 256 * k;
+    if (i >= 2 * SX * SY * SZ) break;
+    const int v = i >> 1, x = x0 + v % SX, y = y0 + (v / SX) % SY, z = z0 + v / (SX * SY);
+    uint4 d = make_uint4(0, 0, 0, 0);
+    if (x >= 0 && x < B.nx && y >= 0 && y < B.ny && z >= 0 && z < B.nz)
+      d = reinterpret_cast<const uint4 *>(in)[2 * (x + (long)B.nx * (y + (long)B.ny * z)) + (i & 1)];
+    reinterpret_cast<uint4 *>(s)[i] = d;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // forward / data-gradient convolution: out[v][co] = act(bias[co] + sum_tap,ci W[tap][co][ci] in[v+off(tap)][ci])
 // mode 0: linear, 1: ReLU, 2: multiply by the ReLU mask of `mask` (backward: g * (a > 0))
+// A wavefront's operands of one dz (rows y-1..y+4, three x offsets: 18 LDS reads) serve its four rows'
+// 36 products; the taps accumulate in the order of t whatever the brick. Bound: latency of staging and
+// of the first weights (65^3 voxels: 26.8 us with 27 bounds-checked global loads per 16 voxels, 21 us here).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void conv3_kernel(const unsigned short *__restrict__ in,
                                                     unsigned short *__restrict__ out,
                                                     const unsigned short *__restrict__ W, const float *__restrict__ bias,
                                                     int nx, int ny, int nz, int mode,
                                                     const unsigned short *__restrict__ mask) {
-  const int lane = threadIdx.x & 63;
-  const int wave = (blockIdx.x * 256 + threadIdx.x) >> 6;
-  const int nwaves = (gridDim.x * 256) >> 6;
+  __shared__ __attribute__((aligned(16))) unsigned short s_in[16 * kBrIn];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = lane & 15, kg = lane >> 4;
   bf16x4 a[27];
 #pragma unroll
@@ -50,31 +83,37 @@ __global__ __launch_bounds__(256) void conv3_kernel(const unsigned short *__rest
   float bv[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) bv[i] = bias ? bias[4 * kg + i] : 0.0f;
-  // tiles of 16 consecutive voxels in the lexicographic order (a tile may wrap into the next x
-  // row: every lane finds its own neighbours), so no lanes idle at the ends of short x rows
-  const long nvox = (long)nx * ny * nz;
-  const long ntiles = (nvox + 15) >> 4;
-  const int sy = 16 * nx, sz = 16 * nx * ny;  // element strides of y and z neighbours (grids < 2^26 voxels)
-  for (long tile = wave; tile < ntiles; tile += nwaves) {
-    const long v = tile * 16 + n;
-    const long vc = v < nvox ? v : nvox - 1;
-    const int x = (int)(vc % nx), y = (int)((vc / nx) % ny), z = (int)(vc / ((long)nx * ny));
-    // which neighbours exist; a missing one is read at the voxel itself and replaced by zero,
-    // so the 27 loads carry no branches and only one address add each
-    const bool xl = x > 0, xh = x < nx - 1, yl = y > 0, yh = y < ny - 1, zl = z > 0, zh = z < nz - 1;
-    const unsigned short *c = in + vc * 16 + 4 * kg;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const Bricks B(nx, ny, nz);
+  for (long brick = blockIdx.x; brick < B.count(); brick += gridDim.x) {
+    int x0, y0, z0;
+    B.origin(brick, x0, y0, z0);
+    __syncthreads();  // the previous brick's reads
+    stage_voxels<kBrX + 2, kBrY + 2, kBrZ + 2>(B, in, s_in, x0 - 1, y0 - 1, z0 - 1);
+    __syncthreads();
+    const int x = x0 + n, z = z0 + wave;
+    f32x4 acc[kBrY];
 #pragma unroll
-    for (int t = 0; t < 27; ++t) {
-      const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-      const bool ok = (dx < 0 ? xl : (dx > 0 ? xh : true)) && (dy < 0 ? yl : (dy > 0 ? yh : true)) &&
-                      (dz < 0 ? zl : (dz > 0 ? zh : true));
-      const int off = 16 * dx + sy * dy + sz * dz;
-      bf16x4 b = load4(c + (ok ? off : 0));
-      if (!ok) b = bf16x4{0, 0, 0, 0};
-      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[t], b, acc, 0, 0, 0);
+    for (int y = 0; y < kBrY; ++y) acc[y] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dz = 0; dz < 3; ++dz) {
+      bf16x4 b[kBrY + 2][3];
+#pragma unroll
+      for (int r = 0; r < kBrY + 2; ++r)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+          b[r][dx] = load4(s_in + (((wave + dz) * (kBrY + 2) + r) * (kBrX + 2) + n + dx) * 16 + 4 * kg);
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+          for (int y = 0; y < kBrY; ++y)
+            acc[y] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[dx + 3 * dy + 9 * dz], b[y + dy][dx], acc[y], 0, 0, 0);
     }
-    if (v < nvox) {
+#pragma unroll
+    for (int y = 0; y < kBrY; ++y) {
+      if (x >= nx || y0 + y >= ny || z >= nz) continue;
+      const long v = x + (long)nx * (y0 + y + (long)ny * z);
       unsigned short o[4];
       uint2 mk = make_uint2(0, 0);
       if (mode == 2) mk = *reinterpret_cast<const uint2 *>(mask + v * 16 + 4 * kg);
@@ -82,7 +121,7 @@ __global__ __launch_bounds__(256) void conv3_kernel(const unsigned short *__rest
                                     (unsigned short)(mk.y & 0xffff), (unsigned short)(mk.y >> 16)};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float r = acc[i] + bv[i];
+        float r = acc[y][i] + bv[i];
         if (mode == 1) r = r > 0.f ? r : 0.f;
         if (mode == 2) r = bf16_to_f32(mv[i]) > 0.f ? r : 0.f;
         o[i] = f32_to_bf16(r);
@@ -95,72 +134,105 @@ __global__ __launch_bounds__(256) void conv3_kernel(const unsigned short *__rest
 
 // ---------------------------------------------------------------------------
 // weight gradient: dW[tap][co][ci] = sum_v g[v][co] in[v+off(tap)][ci], db[co] = sum_v g[v][co]
-// (g = gradient of the layer's pre-activation). MFMA with the voxels as the
-// contraction: A (M = co, K = voxel): lane holds g[v = x0+4(l/16)+j][co = l%16];
-// B (K = voxel, N = ci): lane holds in[v+off][ci = l%16]. Every wavefront walks its own tiles
-// in a fixed order and stores its partial sums to part[wavefront][27*256 + 16] (no two lanes of a
-// wavefront share an entry); wgrad_reduce sums the wavefronts' partials in a fixed order, so the
+// (g = gradient of the layer's pre-activation). MFMA with the voxels as the contraction:
+// A (M = co, K = voxel): lane holds g[v = x0+4(l/16)+j][co = l%16]; B (K = voxel, N = ci): lane holds
+// in[v+off][ci = l%16], i.e. both transposed against the channel-last arrays. A workgroup stages a brick
+// of 16 x 4 x 4 voxels (and its neighbours in `in`, zero outside the grid) in LDS as it lies in memory
+// and reads the operands with ds_read_b64_tr_b16, which transposes 4 x 16 elements per 16 lanes; a read
+// of `in` serves up to three taps. Persistent workgroups sum their bricks in registers, then their four
+// wavefronts in LDS, and store one partial each; wgrad_reduce sums those in a fixed order, so the
 // gradient is bitwise repeatable.
+// Bound: staging (a 28.9 KB brick per 16 x 4 x 4 voxels). 65^3 voxels, per layer: 273 us with 2-byte loads
+// of each operand value from global memory and 240 us for the reduction of 1024 partials by 28 workgroups;
+// 24 and 11 us here.
 // ---------------------------------------------------------------------------
+constexpr int kWgN = 27 * 256 + 16;  // gradient entries of a layer
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+__device__ __forceinline__ bf16x4 load_transposed(unsigned short *tile, int lane) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4 *)(tile + 4 * lane));
+}
 __global__ __launch_bounds__(256) void wgrad_kernel(const unsigned short *__restrict__ g,
                                                     const unsigned short *__restrict__ in, int nx, int ny, int nz,
                                                     float *__restrict__ part) {
-  const int lane = threadIdx.x & 63;
-  const int wave = (blockIdx.x * 256 + threadIdx.x) >> 6;
-  const int nwaves = (gridDim.x * 256) >> 6;
-  const int n = lane & 15, kg = lane >> 4;
-  f32x4 acc[27];
+  constexpr int STAGE = 16 * (kBrIn + kBrOut) * 2, LDS = STAGE > 4 * kWgN ? STAGE : 4 * kWgN;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[LDS];
+  unsigned short *const s_in = reinterpret_cast<unsigned short *>(lds), *const s_g = s_in + 16 * kBrIn;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  f32x4 acc[27], bacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int t = 0; t < 27; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.f;
-  const int tx = (nx + 15) >> 4;
-  const long ntiles = (long)tx * ny * nz;
-  for (long tile = wave; tile < ntiles; tile += nwaves) {
-    const int x0 = (int)(tile % tx) * 16, y = (int)((tile / tx) % ny), z = (int)(tile / ((long)tx * ny));
-    bf16x4 a;
+  const bf16x4 ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
+  const Bricks B(nx, ny, nz);
+  for (long brick = blockIdx.x; brick < B.count(); brick += gridDim.x) {
+    int x0, y0, z0;
+    B.origin(brick, x0, y0, z0);
+    __syncthreads();  // the previous brick's reads
+    stage_voxels<kBrX + 2, kBrY + 2, kBrZ + 2>(B, in, s_in, x0 - 1, y0 - 1, z0 - 1);
+    stage_voxels<kBrX, kBrY, kBrZ>(B, g, s_g, x0, y0, z0);
+    __syncthreads();
+    bf16x4 a[kBrY];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int x = x0 + 4 * kg + j;
-      short val = 0;
-      if (x < nx) val = (short)g[((long)x + (long)nx * (y + (long)ny * z)) * 16 + n];
-      a[j] = val;
-      bsum += bf16_to_f32((unsigned short)val);
+    for (int y = 0; y < kBrY; ++y) {
+      a[y] = load_transposed(s_g + ((wave * kBrY + y) * kBrX) * 16, lane);
+      bacc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[y], ones, bacc, 0, 0, 0);
     }
 #pragma unroll
-    for (int t = 0; t < 27; ++t) {
-      const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-      const int ys = y + dy, zs = z + dz;
-      bf16x4 b = {0, 0, 0, 0};
-      if (ys >= 0 && ys < ny && zs >= 0 && zs < nz) {
+    for (int dz = 0; dz < 3; ++dz)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int x = x0 + 4 * kg + j, xs = x + dx;
-          if (x < nx && xs >= 0 && xs < nx) b[j] = (short)in[((long)xs + (long)nx * (ys + (long)ny * zs)) * 16 + n];
+      for (int r = 0; r < kBrY + 2; ++r)  // row y + dy of `in`
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          const bf16x4 b = load_transposed(s_in + (((wave + dz) * (kBrY + 2) + r) * (kBrX + 2) + dx) * 16, lane);
+#pragma unroll
+          for (int dy = 0; dy < 3; ++dy)
+            if (r - dy >= 0 && r - dy < kBrY) {
+              const int t = dx + 3 * dy + 9 * dz;
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[r - dy], b, acc[t], 0, 0, 0);
+            }
         }
-      }
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
-    }
   }
-  // D[m = co = 4 kg + i][n = ci]
-  float *mine = part + (long)wave * (27 * 256 + 16);
+  // the wavefronts' sums, in their order; D[m = co = 4 kg + i][n = ci]
+  float *const sum = reinterpret_cast<float *>(lds);
+  const int n = lane & 15, kg = lane >> 4;
+  for (int w = 0; w < 4; ++w) {
+    __syncthreads();
+    if (w != wave) continue;
 #pragma unroll
-  for (int t = 0; t < 27; ++t)
+    for (int t = 0; t < 27; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) mine[t * 256 + (4 * kg + i) * 16 + n] = acc[t][i];
-  // bias: lanes with the same co (= n here, since a holds g[.][co = n]) summed over kg
-  bsum += __shfl_xor(bsum, 16);
-  bsum += __shfl_xor(bsum, 32);
-  if (kg == 0) mine[27 * 256 + n] = bsum;
+      for (int i = 0; i < 4; ++i) {
+        float &o = sum[t * 256 + (4 * kg + i) * 16 + n];
+        o = w == 0 ? acc[t][i] : o + acc[t][i];
+      }
+    if (n == 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float &o = sum[27 * 256 + 4 * kg + i];
+        o = w == 0 ? bacc[i] : o + bacc[i];
+      }
+  }
+  __syncthreads();
+  float *mine = part + (long)blockIdx.x * kWgN;
+  for (int i = tid; i < kWgN; i += 256) mine[i] = sum[i];
 }
 
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restrict__ part, int nparts,
-                                                           float *__restrict__ dW, float *__restrict__ db) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= 27 * 256 + 16) return;
+// 64 entries per workgroup, 16 threads per entry (partials g, g + 16, ...), then a fixed-order tree
+__global__ __launch_bounds__(1024) void wgrad_reduce_kernel(const float *__restrict__ part, int nparts,
+                                                            float *__restrict__ dW, float *__restrict__ db) {
+  __shared__ float sh[16][64];
+  const int o = threadIdx.x & 63, grp = threadIdx.x >> 6, i = blockIdx.x * 64 + o;
   float s = 0.f;
-  for (int b = 0; b < nparts; ++b) s += part[(long)b * (27 * 256 + 16) + i];
-  if (i < 27 * 256) dW[i] = s;
-  else db[i - 27 * 256] = s;
+  if (i < kWgN)
+    for (int b = grp; b < nparts; b += 16) s += part[(long)b * kWgN + i];
+  sh[grp][o] = s;
+  for (int h = 8; h > 0; h >>= 1) {
+    __syncthreads();
+    if (grp < h) sh[grp][o] += sh[grp + h][o];
+  }
+  if (grp == 0 && i < kWgN) {
+    if (i < 27 * 256) dW[i] = sh[0][o];
+    else db[i - 27 * 256] = sh[0][o];
+  }
 }
 
 // bf16 weights for the forward pass (W[tap][co][ci], channel counts padded to 16)
@@ -389,24 +461,20 @@ __global__ __launch_bounds__(256) void scale3_kernel(CnnFields F, int n0, int n1
 // workgroups of the statistics pass: one per 1024 points (each ends with a device-scope release
 // and a counter atomic, which dominate on the network's small grids), at most kStatsBlocks
 static inline int stats_blocks(long n) { return (int)std::max<long>(1, std::min<long>(kStatsBlocks, (n + 1023) / 1024)); }
-static inline int cnn_grid(long ntiles) {
-  return (int)std::max<long>(1, std::min<long>((ntiles + 3) / 4, 2048));
-}
-
 int cnn_conv(const unsigned short *in, unsigned short *out, const unsigned short *W, const float *bias, const int *dims,
              int mode, const unsigned short *mask, hipStream_t s) {
-  const long ntiles = ((long)dims[0] * dims[1] * dims[2] + 15) / 16;
-  if ((long)dims[0] * dims[1] * dims[2] >= (1L << 26)) return MPDG_ERR_INVALID;  // 32-bit neighbour offsets
-  hipLaunchKernelGGL(conv3_kernel, dim3(cnn_grid(ntiles)), dim3(256), 0, s, in, out, W, bias, dims[0], dims[1],
+  if ((long)dims[0] * dims[1] * dims[2] >= (1L << 26)) return MPDG_ERR_INVALID;  // the network's grid limit
+  const int nb = (int)std::min<long>(2048, Bricks(dims[0], dims[1], dims[2]).count());
+  hipLaunchKernelGGL(conv3_kernel, dim3(nb), dim3(256), 0, s, in, out, W, bias, dims[0], dims[1],
                      dims[2], mode, mask);
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }
 
 int cnn_wgrad(const unsigned short *g, const unsigned short *in, const int *dims, float *part, int nblocks, float *dW,
               float *db, hipStream_t s) {
-  hipLaunchKernelGGL(wgrad_kernel, dim3(nblocks), dim3(256), 0, s, g, in, dims[0], dims[1], dims[2], part);
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((27 * 256 + 16 + 255) / 256), dim3(256), 0, s, part, 4 * nblocks, dW,
-                     db);
+  const int nb = (int)std::min<long>(nblocks, Bricks(dims[0], dims[1], dims[2]).count());
+  hipLaunchKernelGGL(wgrad_kernel, dim3(nb), dim3(256), 0, s, g, in, dims[0], dims[1], dims[2], part);
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((kWgN + 63) / 64), dim3(1024), 0, s, part, nb, dW, db);
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }
 

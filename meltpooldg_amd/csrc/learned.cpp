@@ -37,7 +37,7 @@ namespace {
 constexpr int kLayers = 4;
 constexpr int kCin[kLayers] = {4, 16, 16, 16};
 constexpr int kCout[kLayers] = {16, 16, 16, 1};
-constexpr int kWgradBlocks = 256;
+constexpr int kWgradBlocks = 512;
 inline hipStream_t S(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 // deterministic Gaussian numbers (splitmix64 + Box-Muller)
@@ -122,7 +122,7 @@ struct mpdg_learned {
     for (int l = 0; l <= kLayers; ++l) MPDG_TRY(act[l].resize((size_t)n * 16));
     MPDG_TRY(g0.resize((size_t)n * 16));
     MPDG_TRY(g1.resize((size_t)n * 16));
-    MPDG_TRY(part.resize((size_t)kWgradBlocks * 4 * (27 * 256 + 16)));  // one slot per wavefront
+    MPDG_TRY(part.resize((size_t)kWgradBlocks * (27 * 256 + 16)));  // one slot per workgroup
     MPDG_TRY(stats.resize(4));
     MPDG_TRY(spart.resize(4 * 1024));
     MPDG_TRY(scount.resize(1));

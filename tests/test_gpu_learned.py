@@ -41,6 +41,27 @@ def test_forward_matches_oracle(cuda, shape, degree, rho):
     assert np.linalg.norm(got - exp) <= 2e-2 * np.linalg.norm(exp)
 
 
+# edges of the 16 x 4 x 4 voxel bricks of the convolution and of the weight gradient, and more bricks than
+# the weight gradient's 512 workgroups; tolerances as in test_gradients_match_oracle
+@pytest.mark.parametrize("shape", [(2, 2, 2), (4, 4, 16), (5, 5, 17), (3, 9, 15), (8, 3, 33), (65, 57, 33)])
+def test_gradients_at_brick_edges(cuda, shape):
+    torch = cuda
+    import meltpooldg_amd as M
+    Tnm1, Tn, q, z, Tnp1 = sample(shape, seed=4)
+    net, _ = make_net(M, shape, qscale=0.5)
+    w = init(5).astype(np.float32)
+    net.set_weights(w)
+    loss, g = net.gradients(*[to_dev(torch, a) for a in (Tnm1, Tn, q, z, Tnp1)])
+    ref_loss, ref = N.loss_and_gradients(w, Tnm1, Tn, q, z, Tnp1, qscale=0.5, bf=True)
+    assert abs(loss - ref_loss) <= 2e-2 * ref_loss
+    o = 0
+    for ci, co in zip(N.CIN, N.COUT):
+        n = co * ci * 27 + co
+        a, b = g[o:o + n].astype(np.float64), ref[o:o + n]
+        o += n
+        assert np.linalg.norm(a - b) <= 5e-2 * np.linalg.norm(b)
+
+
 @pytest.mark.parametrize("shape,degree,rho", [((6, 7, 18), 1, 1), ((17, 13, 9), 2, 2), ((9, 17, 17), 4, 2),
                                               ((13, 25, 13), 3, 4)])
 def test_gradients_match_oracle(cuda, shape, degree, rho):
