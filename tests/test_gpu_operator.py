@@ -487,3 +487,39 @@ def test_nonfinite_sources_stay_in_the_cells_that_hold_them(cuda):
         want = torch.zeros_like(x, dtype=torch.bool)
         want[tuple(slice(a - degree, a + degree + 1) for a in at)] = True
         assert torch.equal(torch.isnan(y), want)
+
+
+# edges of the boundary kernel's tiles of face cells (16, 8, 5, 4 per direction for Q1..Q4): one tile, a
+# remainder of one cell, several tiles; all six faces, constrained faces among them
+@pytest.mark.parametrize("degree,nc,dmask", [(1, (17, 16, 33), 0), (2, (9, 8, 1), 0b000001), (2, (16, 17, 7), 0),
+                                             (3, (5, 6, 11), 0b100000), (4, (4, 5, 9), 0)])
+def test_robin_at_tile_edges(cuda, degree, nc, dmask):
+    torch = cuda
+    import meltpooldg_amd as M
+    rng = np.random.default_rng(41)
+    orc0 = O.Operator(degree, nc)
+    T = 1000.0 + 50.0 * rng.uniform(-1, 1, orc0.n_dofs)
+    orc = O.Operator(degree, nc, c_mass=3.6e2, kappa=0.5, T=T, dirichlet_mask=dmask, robin_mask=63, alpha=2500.0,
+                     emissivity=0.98, T_inf_conv=300.0, T_inf_rad=310.0)
+    gop = M.HeatDiffuseMultiPhaseOperator(degree, nc, rho_cp=3.6, dirichlet_faces=dmask)
+    gop.reset_time_increment(1e-2)
+    gop.set_conductivity_constant(0.5)
+    Td = torch.tensor(T, device="cuda")
+    gop.set_robin(63, alpha=2500.0, T_inf_conv=300.0, emissivity=0.98, T_inf_rad=310.0, T=Td)
+    x = rng.uniform(-1, 1, orc.n_dofs)
+    y, d, r = (torch.zeros(orc.n_dofs, dtype=torch.float64, device="cuda") for _ in range(3))
+    gop.vmult(y, torch.tensor(x, device="cuda"))
+    gop.compute_inverse_diagonal_from_matrixfree(d)
+    T_old = T - rng.uniform(0, 1, orc.n_dofs)
+    Tod = torch.tensor(T_old, device="cuda")
+    gop.create_rhs(r, Td, Tod)
+    # the faces' part of the residual (the cells' part takes T as zero on constrained DoFs, the oracle as given)
+    gop.set_robin(0)
+    cells = torch.zeros_like(r)
+    gop.create_rhs(cells, Td, Tod)
+    torch.cuda.synchronize()
+    orc_cells = O.Operator(degree, nc, c_mass=3.6e2, kappa=0.5, T=T, dirichlet_mask=dmask)
+    ref = orc.create_rhs(np.zeros(orc.n_dofs), T, T_old) - orc_cells.create_rhs(np.zeros(orc.n_dofs), T, T_old)
+    assert rel_err(y.cpu().numpy(), orc.vmult(x)) < 1e-12
+    assert rel_err(d.cpu().numpy(), orc.inverse_diagonal()) < 1e-12
+    assert rel_err((r - cells).cpu().numpy(), ref) < 1e-11
