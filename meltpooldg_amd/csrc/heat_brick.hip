@@ -103,6 +103,9 @@ struct BrickArgs {
   Number law_p[4];
   const Number *kappa_arr, *T, *metric;
   Number *scratch;
+  // residual: the mass term acts on fa src + fb T_old + fc q
+  Number fa, fb, fc;
+  const Number *T_old, *q;
 };
 
 // x sweep (second index): out[j][q] = sum_i M(q, i) in[j][i]; y sweep (first index) likewise
@@ -338,7 +341,8 @@ template <typename Args> __device__ __forceinline__ const __attribute__((address
   return *p;
 }
 
-template <int N1, typename Number, int KMODE, bool MAPPED>
+// RES: dst -= the residual's cell part (see launch_brick_residual) instead of dst = J src
+template <int N1, typename Number, int KMODE, bool MAPPED, bool RES = false>
 __global__ __launch_bounds__(64 * kNW) __attribute__((amdgpu_waves_per_eu(BrickOccupancy<N1, Number, MAPPED, KMODE>::W)))
 void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__ src, Number *__restrict__ dst) {
   using B = BrickShape<N1>;
@@ -448,10 +452,35 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
 #pragma unroll
         for (int i = 0; i < N1; ++i) srow[wave][pen][i][lane] = u[K][i];
       }
-      constrain(cxb, cy, u);
-
       // ---- conductivity at the points of this lane's plane qz = l ----
       const auto &A = fresh_args<BrickArgs<Number, N1>>();
+      Number w[N1][N1];  // RES: what the mass term is applied to
+      if constexpr (RES) {
+        Number t[N1][N1];
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) w[j][i] = A.fa * u[j][i];
+        if (A.fb != Number(0)) {
+          load_rows(A.T_old, cxb, cy, true, t);
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) w[j][i] = fma(A.fb, t[j][i], w[j][i]);
+        }
+        if (A.q) {
+          load_rows(A.q, cxb, cy, true, t);
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) w[j][i] = fma(A.fc, t[j][i], w[j][i]);
+        }
+        constrain(cxb, cy, w);
+      }
+      // the law is evaluated at the source as it is; interpolated below, before the constraints
+      constexpr bool LAW_OF_SRC = RES && KMODE == KAPPA_LAW;
+      if constexpr (!LAW_OF_SRC) constrain(cxb, cy, u);
+
       using Vec = Number __attribute__((ext_vector_type(NV)));
       Number kq[N1][N1];
       Vec kraw[NLD];
@@ -476,9 +505,9 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
 #pragma unroll
           for (int i = 0; i < N1; ++i) kq[j][i] = p[N1 * j + i];
       }
-      if (KMODE == KAPPA_LAW) {
+      if constexpr (KMODE == KAPPA_LAW && !LAW_OF_SRC) {
         Number a[N1][N1], t[N1][N1];
-        load_rows(P.T, cxb, cy, true, a);
+        load_rows(A.T, cxb, cy, true, a);
         sweep_x<N1, false, false>(P.S, a, t);
         sweep_y<N1, false, false>(P.S, t, a);
         z_forward<N1, false>(P.S, P.G, zt, a, t, t);
@@ -492,12 +521,13 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
         // J u = M_x [M_y (c_m M_z + k k_z K_z) + k k_y K_y M_z] u + k k_x K_x M_y M_z u
         Number mz[N1][N1], p[N1][N1];
         z_forward<N1, true>(P.M1, P.K1, zt, u, mz, p);
+        if constexpr (RES) z_forward<N1, false>(P.M1, P.K1, zt, w, w, w);
         if (N1 == 3 && KMODE == KAPPA_CELL) kc = row < 3 ? kc : Number(0);
         const Number kx = kc * P.kx, ky = kc * P.ky, kz = kc * P.kz;
 #pragma unroll
         for (int j = 0; j < N1; ++j)
 #pragma unroll
-          for (int i = 0; i < N1; ++i) p[j][i] = fma(P.cm, mz[j][i], kz * p[j][i]);
+          for (int i = 0; i < N1; ++i) p[j][i] = fma(P.cm, RES ? w[j][i] : mz[j][i], kz * p[j][i]);
         Number s[N1][N1];
         sweep_y<N1, false, false>(P.M1, mz, u);
         sweep_y<N1, false, false>(P.M1, p, s);
@@ -514,15 +544,32 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
       } else {
         // ---- to the points: v = values, gz = z derivative ----
         Number gz[N1][N1], e[N1][N1];
-        {
+        auto to_points = [&](Number (&x)[N1][N1]) {
           Number t[N1][N1];
-          sweep_x<N1, false, false>(P.S, u, t);
-          sweep_y<N1, false, false>(P.S, t, u);
-          z_forward<N1, true>(P.S, P.G, zt, u, v, gz);
+          sweep_x<N1, false, false>(P.S, x, t);
+          sweep_y<N1, false, false>(P.S, t, x);
+        };
+        to_points(u);
+        z_forward<N1, true>(P.S, P.G, zt, u, v, gz);
+        if constexpr (LAW_OF_SRC) {
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) kq[j][i] = law_kappa<Number>(P.law, P.law_p, v[j][i]);
+          if (A.dmask) {
+            load_rows(src, cxb, cy, true, u);
+            constrain(cxb, cy, u);
+            to_points(u);
+            z_forward<N1, true>(P.S, P.G, zt, u, v, gz);
+          }
+        }
+        if constexpr (RES) {
+          to_points(w);
+          z_forward<N1, false>(P.S, P.G, zt, w, w, w);
         }
         // ---- at the points (heat_diffuse_operator.cpp:1029-1077): e = c_m W v + D_x^T f_x + D_y^T f_y,
         //      gz becomes f_z ----
-        if (MAPPED) {
+        if constexpr (MAPPED) {
           Number gx[N1][N1], gy[N1][N1];
           sweep_x<N1, false, false>(P.D, v, gx);
           sweep_y<N1, false, false>(P.D, v, gy);
@@ -599,7 +646,7 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
             }
 #pragma unroll
             for (int i = 0; i < N1; ++i) {
-              Number a = wms[half(j)][half(i)] * v[j][i];
+              Number a = wms[half(j)][half(i)] * (RES ? w[j][i] : v[j][i]);
 #pragma unroll
               for (int q = 0; q < N1; ++q) a = fma(P.D(q, i), f[q], a);
               e[j][i] = a;
@@ -684,6 +731,14 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
       }
       const auto &Z = fresh_args<BrickArgs<Number, N1>>();
       const bool hy = cy != Z.nc[1] - 1;  // the top row is not the mesh's
+      if constexpr (RES) {
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) r[j][i] = -r[j][i];
+      }
+      // dst = x, or dst += x (RES); the classes are always stored
+      auto put = [&](Number *p, Number x, bool owner) { *p = RES && owner ? *p + x : x; };
       constrain(cxb, cy, r);
 
       // ---- store rows 0..K-1, and the top row after the last step: to dst, or to the class of the
@@ -694,12 +749,12 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
         if ((f & F_STORE) && cx < Z.nc[0]) {
           const bool hz = f & F_HZ;
           Number *o = (hz ? Z.scratch + Z.g.off[4] + (long)bz * sz : dst + sz * iz) + cx;
-          o[sy * cy] = (Number)r[0][0];
+          put(o + sy * cy, (Number)r[0][0], !hz);
           if (last) {
             Number *t = !hy ? o + sy * (cy + 1)
                             : Z.scratch + (hz ? Z.g.off[6] + ((long)by + (long)(Z.g.nb[1] - 1) * bz) * sy
                                               : Z.g.off[2] + ((long)by + (long)(Z.g.nb[1] - 1) * iz) * sy) + cx;
-            *t = (Number)r[1][0];
+            put(t, (Number)r[1][0], !hz && !hy);
           }
         }
       } else {
@@ -723,8 +778,8 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
             lds_fence();
             if (st) {
 #pragma unroll
-              for (int rw = 0; rw < K; ++rw) o[sz * rw + sy * j] = t[rw * RPI * W];
-              if (end || wave == kNW - 1) oz[sy * j] = t[K * RPI * W];
+              for (int rw = 0; rw < K; ++rw) put(o + sz * rw + sy * j, t[rw * RPI * W], true);
+              if (end || wave == kNW - 1) put(oz + sy * j, t[K * RPI * W], end);
             }
             lds_fence();
           }
@@ -743,7 +798,7 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
                                     : Z.g.off[2] + ((long)by + (long)(Z.g.nb[1] - 1) * z) * sy);
               else
                 p = (up ? Z.scratch + Z.g.off[4] + (long)bz * sz : dst + sz * z) + sy * ((long)K * cy + K);
-              if (jr == 0 && x < K * (cx_end - cxb)) p[K * cxb + x] = tl[rw * W + x];
+              if (jr == 0 && x < K * (cx_end - cxb)) put(p + K * cxb + x, tl[rw * W + x], !hy && !up);
             }
             lds_fence();
           }
@@ -769,7 +824,7 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
               else o = (hz ? Z.scratch + Z.g.off[4] + (long)bz * sz : dst + sz * iz) + sy * iy;
               o += K * cx + K;
             }
-            *o = (Number)r[j][K];
+            put(o, (Number)r[j][K], !hx && !y && !hz);
           }
         }
       }
@@ -859,25 +914,29 @@ __global__ __launch_bounds__(256) void brick_fixup_kernel(Number *__restrict__ d
 }
 
 template <int N1, typename Number>
-int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
-                    hipEvent_t kernel_start, hipEvent_t kernel_end) {
-  BrickArgs<Number, N1> A;
-  const FE1D &fe = fe1d(N1 - 1);
+int fill_brick_args(const OperatorData<Number> &op, BrickArgs<Number, N1> &A) {
   const bool mapped = op.metric != nullptr;
+  const FE1D &fe = fe1d(N1 - 1);
   const double vol = mapped ? 1.0 : op.h[0] * op.h[1] * op.h[2];
-  double Dy[kMaxN1][kMaxN1], Gz[kMaxN1][kMaxN1];
+  double Dy[kMaxN1][kMaxN1], Gz[kMaxN1][kMaxN1], M1[kMaxN1][kMaxN1] = {}, K1[kMaxN1][kMaxN1] = {};
   const double ry = mapped ? 1.0 : (op.h[0] * op.h[0]) / (op.h[1] * op.h[1]);
   const double rz = mapped ? 1.0 : (op.h[0] * op.h[0]) / (op.h[2] * op.h[2]);
   for (int q = 0; q < N1; ++q)
     for (int i = 0; i < N1; ++i) {
       Dy[q][i] = fe.D[q][i] * ry;
       Gz[q][i] = fe.G[q][i] * rz;
+      for (int j = 0; j < N1; ++j) {
+        M1[i][j] += fe.S[q][i] * fe.qw[q] * fe.S[q][j];
+        K1[i][j] += fe.G[q][i] * fe.qw[q] * fe.G[q][j];
+      }
     }
   A.S.set(fe.S);
   A.D.set(fe.D);
   A.G.set(fe.G);
   A.Dy.set(Dy);
   A.Gz.set(Gz);
+  A.M1.set(M1);
+  A.K1.set(K1);
   for (int a = 0; 2 * a < N1; ++a) A.w[a] = (Number)fe.qw[a];
   for (int d = 0; d < 3; ++d) {
     A.nc[d] = op.nc[d];
@@ -891,50 +950,80 @@ int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *d
   A.kx = (Number)(mapped ? 1.0 : vol / (op.h[0] * op.h[0]));
   A.ky = (Number)(mapped ? 1.0 : vol / (op.h[1] * op.h[1]));
   A.kz = (Number)(mapped ? 1.0 : vol / (op.h[2] * op.h[2]));
-  double M1[kMaxN1][kMaxN1] = {}, K1[kMaxN1][kMaxN1] = {};
-  for (int i = 0; i < N1; ++i)
-    for (int j = 0; j < N1; ++j)
-      for (int q = 0; q < N1; ++q) {
-        M1[i][j] += fe.S[q][i] * fe.qw[q] * fe.S[q][j];
-        K1[i][j] += fe.G[q][i] * fe.qw[q] * fe.G[q][j];
-      }
-  A.M1.set(M1);
-  A.K1.set(K1);
   A.kappa = (Number)op.kappa;
   for (int i = 0; i < 4; ++i) A.law_p[i] = (Number)op.law_p[i];
   A.kappa_arr = op.kappa_arr;
   A.T = op.T;
   A.metric = op.metric;
   A.scratch = op.edge;
-  if (A.g.total > 0 && (op.edge == nullptr || (size_t)A.g.total > op.edge_elems)) return MPDG_ERR_INVALID;
-  const dim3 grid((unsigned)((long)A.g.nb[0] * A.g.nb[1] * A.g.nb[2])), block(64 * kNW);
+  A.T_old = A.q = nullptr;
+  A.fa = A.fb = A.fc = Number(0);
+  return A.g.total > 0 && (op.edge == nullptr || (size_t)A.g.total > op.edge_elems) ? MPDG_ERR_INVALID : MPDG_OK;
+}
+
+template <int N1, typename Number>
+int finish_brick(const BrickArgs<Number, N1> &A, Number *dst, hipStream_t stream) {
+  const long lines = (long)(A.g.nb[2] - 1) * A.nd[1] + (long)(A.g.nb[1] - 1) * A.nd[2] + (long)(A.g.nb[0] - 1) * A.nd[2];
+  const int longest = A.g.nb[0] > 1 ? std::max(A.nd[0], A.nd[1]) : A.nd[0];
+  const int parts = (longest + 64 * kFixup - 1) / (64 * kFixup);
+  if (lines > 0)
+    hipLaunchKernelGGL(brick_fixup_kernel<Number>, dim3((unsigned)((lines * parts + 3) / 4)), dim3(256), 0, stream, dst,
+                       A.scratch, A.g, N1 - 1, A.nd[0], A.nd[1], A.nd[2], parts);
+  return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
+}
+template <int N1, typename Number> dim3 brick_blocks(const BrickArgs<Number, N1> &A) {
+  return dim3((unsigned)((long)A.g.nb[0] * A.g.nb[1] * A.g.nb[2]));
+}
+#define MPDG_BRICK(KM, MP, RES_) \
+  hipLaunchKernelGGL((heat_brick_kernel<N1, Number, KM, MP, RES_>), brick_blocks(A), dim3(64 * kNW), 0, stream, A, src, dst)
+
+template <int N1, typename Number>
+int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
+                    hipEvent_t kernel_start, hipEvent_t kernel_end) {
+  BrickArgs<Number, N1> A;
+  if (const int rc = fill_brick_args(op, A)) return rc;
   if (kernel_start) (void)hipEventRecord(kernel_start, stream);
-#define MPDG_BRICK(KM, MP) hipLaunchKernelGGL((heat_brick_kernel<N1, Number, KM, MP>), grid, block, 0, stream, A, src, dst)
-  if (mapped) {
+  if (op.metric) {
     switch (op.kappa_mode) {
-      case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, true); break;
-      case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, true); break;
+      case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, true, false); break;
+      case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, true, false); break;
       default: return MPDG_ERR_INVALID;  // per-qp conductivity on mapped meshes runs through metric_k
     }
   } else {
     switch (op.kappa_mode) {
-      case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, false); break;
-      case KAPPA_QP: MPDG_BRICK(KAPPA_QP, false); break;
-      case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, false); break;
-      case KAPPA_LAW: MPDG_BRICK(KAPPA_LAW, false); break;
+      case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, false, false); break;
+      case KAPPA_QP: MPDG_BRICK(KAPPA_QP, false, false); break;
+      case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, false, false); break;
+      case KAPPA_LAW: MPDG_BRICK(KAPPA_LAW, false, false); break;
       default: return MPDG_ERR_INVALID;
     }
   }
-#undef MPDG_BRICK
   if (kernel_end) (void)hipEventRecord(kernel_end, stream);
-  const long lines = (long)(A.g.nb[2] - 1) * op.nd[1] + (long)(A.g.nb[1] - 1) * op.nd[2] + (long)(A.g.nb[0] - 1) * op.nd[2];
-  const int longest = A.g.nb[0] > 1 ? std::max(op.nd[0], op.nd[1]) : op.nd[0];
-  const int parts = (longest + 64 * kFixup - 1) / (64 * kFixup);
-  if (lines > 0)
-    hipLaunchKernelGGL(brick_fixup_kernel<Number>, dim3((unsigned)((lines * parts + 3) / 4)), dim3(256), 0, stream, dst,
-                       op.edge, A.g, N1 - 1, op.nd[0], op.nd[1], op.nd[2], parts);
-  return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
+  return finish_brick(A, dst, stream);
 }
+
+template <int N1>
+int launch_brick_residual_n1(const OperatorData<double> &op, const double *src, const double *T_old, const double *q, double a,
+                             double b, double c, double *dst, hipStream_t stream) {
+  using Number = double;
+  BrickArgs<Number, N1> A;
+  if (const int rc = fill_brick_args(op, A)) return rc;
+  A.fa = a;
+  A.fb = b;
+  A.fc = c;
+  A.T_old = T_old;
+  A.q = q;
+  switch (op.kappa_mode) {
+    case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, false, true); break;
+    case KAPPA_QP: MPDG_BRICK(KAPPA_QP, false, true); break;
+    case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, false, true); break;
+    case KAPPA_LAW: MPDG_BRICK(KAPPA_LAW, false, true); break;
+    default: return MPDG_ERR_INVALID;
+  }
+  return finish_brick(A, dst, stream);
+}
+
+#undef MPDG_BRICK
 
 }  // namespace
 
@@ -953,4 +1042,14 @@ int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst,
 template int launch_brick<double>(const OperatorData<double> &, const double *, double *, hipStream_t, hipEvent_t, hipEvent_t);
 template int launch_brick<float>(const OperatorData<float> &, const float *, float *, hipStream_t, hipEvent_t, hipEvent_t);
 
+int launch_brick_residual(const OperatorData<double> &op, const double *T, const double *T_old, const double *q, double a,
+                          double b, double c, double *dst, hipStream_t stream) {
+  if (op.metric) return MPDG_ERR_INVALID;
+  switch (op.degree) {
+    case 1: return launch_brick_residual_n1<2>(op, T, T_old, q, a, b, c, dst, stream);
+    case 2: return launch_brick_residual_n1<3>(op, T, T_old, q, a, b, c, dst, stream);
+    case 3: return launch_brick_residual_n1<4>(op, T, T_old, q, a, b, c, dst, stream);
+    default: return MPDG_ERR_INVALID;
+  }
+}
 }  // namespace mpdg

@@ -125,10 +125,23 @@ int mpdg_heat_op::create_rhs(double *dst, const double *T, const double *T_old, 
     MPDG_TRY(launch_tangent_residual(d64, dt, mat, vel, vfield, T, T_old, q, dst, s));
     return launch_boundary(d64, 2, flux, dst, nullptr, T, s);
   }
+  MPDG_TRY(ensure_edge());
   const long n = d64.n_dofs;
+  auto apart = [&](const double *p) { return p == nullptr || p + n <= dst || dst + n <= p; };
+  if (d64.degree < 4 && !d64.metric && apart(T) && apart(T_old) && apart(q)) {
+    // one pass over the cells (Q2 64^3 with a law: 154 us as two applies and the vector passes below)
+    OperatorData<double> od = d64;
+    if (T_zero) {  // only the mass term; the pass reads T_old as its field
+      od.kappa_mode = KAPPA_CONST;
+      od.kappa = 0.0;
+      MPDG_TRY(launch_brick_residual(od, T_old, nullptr, q, -1.0, 0.0, -1.0 / od.c_mass, dst, s));
+    } else {
+      MPDG_TRY(launch_brick_residual(od, T, T_old, q, 1.0, -1.0, -1.0 / od.c_mass, dst, s));
+    }
+    return launch_boundary(d64, 2, flux, dst, nullptr, T, s);
+  }
   MPDG_TRY(tmp1.resize(n));
   MPDG_TRY(tmp2.resize(n));
-  MPDG_TRY(ensure_edge());
   if (T_zero && !tangent) {
     // dst += c_m M (T_old + q / c_m) + boundary terms at T = 0 (K T vanishes)
     OperatorData<double> mass = d64;

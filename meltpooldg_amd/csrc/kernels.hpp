@@ -158,6 +158,11 @@ template <typename Number>
 int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                  hipEvent_t kernel_start, hipEvent_t kernel_end);
 size_t brick_scratch_elems(int degree, const int *n_cells);
+// Q1..Q3, Cartesian cells: dst -= c_m M (a T + b T_old + c q) + K_k T in one pass (T_old is not read when
+// b = 0, q when null); constrained DoFs count as zero and are left alone, a conductivity law is evaluated at
+// T as given. dst must not overlap the inputs.
+int launch_brick_residual(const OperatorData<double> &op, const double *T, const double *T_old, const double *q, double a,
+                          double b, double c, double *dst, hipStream_t stream);
 
 // heat_aux.hip: diagonal, boundary faces, residual, norms, conductivity
 // diag = the operator's diagonal (cells only; constrained rows 1); scratch: 2 n_cells (k+1)^3 values

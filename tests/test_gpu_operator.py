@@ -471,6 +471,28 @@ def test_mapped_vmult_and_diagonal_at_brick_edges(cuda, degree, nc, mode):
     assert rel_err(d.cpu().numpy(), orc.diagonal()) < 1e-12
 
 
+@pytest.mark.parametrize("with_q", [True, False])
+@pytest.mark.parametrize("degree,nc,mode,dmask", [(d, nc, m, b) for d, nc, m, p, b in BRICK_CASES if p == 0] +
+                         [(1, (17, 3, 9), "law", 0b100001), (2, (17, 9, 5), "qp", 0b010000), (2, (18, 5, 5), "law", 0),
+                          (3, (18, 5, 5), "law", 0b001011), (3, (17, 17, 6), "const", 0)])
+def test_residual_in_one_pass_agrees_with_its_parts(cuda, degree, nc, mode, dmask, with_q):
+    """create_rhs in one pass over the cells, and as applies and vector updates (which a dst that is also an
+    input still takes): equal up to the order of summation (some hundred terms), relative to the sums."""
+    torch = cuda
+    _, gop, data = make_pair(torch, degree, nc, mode=mode, dirichlet=dmask, seed=31)
+    g = torch.Generator(device="cuda").manual_seed(32)
+    rand = lambda: torch.rand(gop.n_dofs, dtype=torch.float64, device="cuda", generator=g)  # noqa: E731
+    T = data["T"] if mode == "law" else rand()
+    T_old = T + 0.1 * rand()
+    q = 1e-3 * rand() if with_q else None
+    base = q if with_q else T_old
+    one, parts = base.clone(), base.clone()
+    gop.create_rhs(one, T, T_old, q)
+    gop.create_rhs(parts, T, T_old if with_q else parts, parts if with_q else None)
+    scale = float((parts - base).abs().max()) + 1e-3 * float(base.abs().max())
+    assert scale > 0 and float((one - parts).abs().max()) < 1e-12 * scale
+
+
 def test_nonfinite_sources_stay_in_the_cells_that_hold_them(cuda):
     """A NaN in one DoF reaches the DoFs of the cells that hold it and no others (nothing of one cell is
     multiplied into another, as by the idle or paired lanes of a matrix instruction)."""
