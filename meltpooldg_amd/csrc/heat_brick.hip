@@ -31,7 +31,7 @@
 // kernel with LDS transposes, scatter and atomics it replaces, 0.566 ms here; elsewhere the VALU (Q3 128^3,
 // constant k: FP64 0.62 -> 0.43 ms, FP32 0.42 -> 0.28 ms; Q2 64^3 FP32 35.7 -> 25.5 us; Q3 75 x 62 x 49 FP32
 // 83.8 -> 50.5 us; mapped Q3 96^3 FP64, bound by the stored metric, 1.08 -> 0.82 ms).
-#include "kernels.hpp"
+#include "tangent.hpp"
 
 namespace mpdg {
 
@@ -106,6 +106,10 @@ struct BrickArgs {
   // residual: the mass term acts on fa src + fb T_old + fc q
   Number fa, fb, fc;
   const Number *T_old, *q;
+  // the full Newton tangent: whether it has the solidification terms; convection: 0 none, 1 with the constant
+  // velocity vh (over the cell sizes), 2 with a velocity field
+  int conv, solid;
+  Number vh[3];
 };
 
 // x sweep (second index): out[j][q] = sum_i M(q, i) in[j][i]; y sweep (first index) likewise
@@ -309,6 +313,9 @@ __device__ __forceinline__ void lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+constexpr int KAPPA_TANGENT = 4;   // the full Newton tangent's coefficients instead of a conductivity
+constexpr int TANGENT_DIAGONAL = 5;  // ... and its diagonal: no source is read
+
 // Wavefronts per SIMD the register allocation targets: as many as fit without spills (Q3 FP64 needs
 // 226 VGPRs with per-point conductivity and 168 with one per cell, Q3 FP32 129 and 116; mapped cells
 // hold three fluxes: 195 and 129). Fewer wavefronts were slower even where the next step's source was
@@ -318,6 +325,8 @@ template <bool M, int KM> struct BrickOccupancy<3, double, M, KM> { static const
 template <bool M, int KM> struct BrickOccupancy<4, double, M, KM> { static constexpr int W = 2; };
 template <> struct BrickOccupancy<4, double, false, KAPPA_CONST> { static constexpr int W = 3; };
 template <> struct BrickOccupancy<4, double, false, KAPPA_CELL> { static constexpr int W = 3; };
+// (more loads of its eight coefficients in flight: Q3 50 x 40 x 30 142 -> 124 us)
+template <> struct BrickOccupancy<4, double, false, KAPPA_TANGENT> { static constexpr int W = 1; };
 template <int KM> struct BrickOccupancy<4, float, true, KM> { static constexpr int W = 3; };
 template <> struct BrickOccupancy<4, float, false, KAPPA_QP> { static constexpr int W = 3; };
 
@@ -340,6 +349,7 @@ template <typename Args> __device__ __forceinline__ const __attribute__((address
   asm volatile("" : "+s"(p));
   return *p;
 }
+
 
 // RES: dst -= the residual's cell part (see launch_brick_residual) instead of dst = J src
 template <int N1, typename Number, int KMODE, bool MAPPED, bool RES = false>
@@ -436,19 +446,25 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
         for (int i = 0; i < N1; ++i) u[j][i] = row < 3 ? u[j][i] : Number(0);
     }
   };
+  // the lane's first point in the arrays with ncomp values per point (point_data_at)
+  auto point_data = [&](const auto &A, int ncomp, int cxb, int cy) {
+    const long pencil = cxb / kNX + (long)((A.nc[0] + kNX - 1) / kNX) * (cy + (long)A.nc[1] * min(cz, A.nc[2] - 1));
+    return A.metric + (pencil * ncomp * NQ + min(l, K)) * kNX + min(c, A.nc[0] - 1 - cxb);
+  };
   int parity = 0;
   for (int cy = cy0; cy < cy_end; ++cy) {
     const bool last = cy + 1 == cy_end;  // the brick's top row is complete too
     int pen = 0;
     for (int cxb = cx0; cxb < cx_end; cxb += kNX, ++pen, parity ^= 1) {
       const long cell = min(cxb + c, P.nc[0] - 1) + (long)P.nc[0] * (cy + (long)P.nc[1] * min(cz, P.nc[2] - 1));
+      constexpr bool DIAGONAL = KMODE == TANGENT_DIAGONAL;
       Number u[N1][N1];
-      load_rows(src, cxb, cy, cy == cy0, u);
-      if (cy > cy0) {
+      if constexpr (!DIAGONAL) load_rows(src, cxb, cy, cy == cy0, u);
+      if (!DIAGONAL && cy > cy0) {
 #pragma unroll
         for (int i = 0; i < N1; ++i) u[0][i] = srow[wave][pen][i][lane];
       }
-      if (!last) {
+      if (!DIAGONAL && !last) {
 #pragma unroll
         for (int i = 0; i < N1; ++i) srow[wave][pen][i][lane] = u[K][i];
       }
@@ -479,7 +495,7 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
       }
       // the law is evaluated at the source as it is; interpolated below, before the constraints
       constexpr bool LAW_OF_SRC = RES && KMODE == KAPPA_LAW;
-      if constexpr (!LAW_OF_SRC) constrain(cxb, cy, u);
+      if constexpr (!LAW_OF_SRC && !DIAGONAL) constrain(cxb, cy, u);
 
       using Vec = Number __attribute__((ext_vector_type(NV)));
       Number kq[N1][N1];
@@ -541,6 +557,70 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
         sweep_y<N1, false, true>(P.K1, mz, s);
         sweep_x<N1, false, false>(P.M1, s, v);
         sweep_x<N1, false, true>(P.K1, u, v);
+      } else if constexpr (DIAGONAL) {
+        // sum_q t0 phi^2 + sum_d a_d phi d_d phi + t1 / h_d^2 (d_d phi)^2 with 1D tables S: phi^2, G: phi phi',
+        // M1: phi'^2 of the points (columns) at the DoFs (rows)
+        const Number *M = point_data(A, kTangentCoeffs, cxb, cy);
+        constexpr int C1 = NQ * kNX;
+        const bool idle = N1 == 3 && row == 3;
+        auto coefficients = [&](Number (&t)[N1][N1], auto value) {
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) t[j][i] = idle ? Number(0) : value(M + (N1 * j + i) * N1 * kNX);
+        };
+        auto first_order = [&](Number (&t)[N1][N1], int d) {
+          coefficients(t, [&](const Number *m) {
+            Number a = 0;
+            if (A.conv == 1) a = m[2 * C1] * A.vh[d];
+            if (A.conv == 2) a = m[(2 + d) * C1];
+            if (A.solid) a += m[(5 + d) * C1];
+            return a;
+          });
+        };
+        const ZTables<N1, Number> zt2(P, P.M1, P.G, lane);
+        Number t[N1][N1], e[N1][N1], k[N1][N1], h[N1][N1], x[N1][N1];
+        coefficients(t, [&](const Number *m) { return m[0]; });
+        z_forward<N1, false>(P.S, P.G, zt, t, e, e);
+        coefficients(t, [&](const Number *m) { return m[C1]; });
+        z_forward<N1, false>(P.S, P.G, zt, t, k, k);
+        z_forward<N1, false>(P.M1, P.G, zt2, t, t, t);
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) e[j][i] = fma(P.kz, t[j][i], e[j][i]);
+        const bool first = A.conv || A.solid;
+        if (first) {
+          first_order(t, 2);
+          z_forward<N1, true>(P.S, P.G, zt, t, h, x);
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) e[j][i] += x[j][i];
+        }
+        sweep_y<N1, false, false>(P.S, e, h);
+        sweep_y<N1, false, false>(P.S, k, x);
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) {
+            k[j][i] *= P.ky;
+            x[j][i] *= P.kx;
+          }
+        sweep_y<N1, false, true>(P.M1, k, h);
+        if (first) {
+          first_order(t, 1);
+          z_forward<N1, false>(P.S, P.G, zt, t, k, k);
+          sweep_y<N1, false, true>(P.G, k, h);
+        }
+        sweep_x<N1, false, false>(P.S, h, v);
+        sweep_x<N1, false, true>(P.M1, x, v);
+        if (first) {
+          first_order(t, 0);
+          z_forward<N1, false>(P.S, P.G, zt, t, k, k);
+          sweep_y<N1, false, false>(P.S, k, e);
+          sweep_x<N1, false, true>(P.G, e, v);
+        }
       } else {
         // ---- to the points: v = values, gz = z derivative ----
         Number gz[N1][N1], e[N1][N1];
@@ -569,12 +649,42 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
         }
         // ---- at the points (heat_diffuse_operator.cpp:1029-1077): e = c_m W v + D_x^T f_x + D_y^T f_y,
         //      gz becomes f_z ----
-        if constexpr (MAPPED) {
+        if constexpr (KMODE == KAPPA_TANGENT) {
+          // val = t0 u + t2..t4 . grad u, flux = t1 / h^2 grad u + t5..t7 u (tangent.hip); t2 alone for a
+          // constant velocity
           Number gx[N1][N1], gy[N1][N1];
           sweep_x<N1, false, false>(P.D, v, gx);
           sweep_y<N1, false, false>(P.D, v, gy);
-          const long pencil = cxb / kNX + (long)((P.nc[0] + kNX - 1) / kNX) * (cy + (long)P.nc[1] * min(cz, P.nc[2] - 1));
-          const Number *M = P.metric + (pencil * 7 * NQ + min(l, K)) * kNX + min(c, P.nc[0] - 1 - cxb);  // (metric_at)
+          const Number *M = point_data(A, kTangentCoeffs, cxb, cy);
+          const bool idle = N1 == 3 && row == 3;
+#pragma unroll
+          for (int j = 0; j < N1; ++j)
+#pragma unroll
+            for (int i = 0; i < N1; ++i) {
+              const Number *m = M + (N1 * j + i) * N1 * kNX;
+              constexpr int C1 = NQ * kNX;
+              const Number x = gx[j][i], y = gy[j][i], z = gz[j][i], uq = v[j][i], k = m[C1];
+              Number val = m[0] * uq;
+              if (A.conv == 1) val += m[2 * C1] * (A.vh[0] * x + A.vh[1] * y + A.vh[2] * z);
+              if (A.conv == 2) val += m[2 * C1] * x + m[3 * C1] * y + m[4 * C1] * z;
+              gx[j][i] = k * P.kx * x;
+              gy[j][i] = k * P.ky * y;
+              gz[j][i] = k * P.kz * z;
+              if (A.solid) {
+                gx[j][i] += m[5 * C1] * uq;
+                gy[j][i] += m[6 * C1] * uq;
+                gz[j][i] += m[7 * C1] * uq;
+              }
+              e[j][i] = val;
+              if (idle) e[j][i] = gx[j][i] = gy[j][i] = gz[j][i] = Number(0);
+            }
+          sweep_x<N1, true, true>(P.D, gx, e);
+          sweep_y<N1, true, true>(P.Dy, gy, e);
+        } else if constexpr (MAPPED) {
+          Number gx[N1][N1], gy[N1][N1];
+          sweep_x<N1, false, false>(P.D, v, gx);
+          sweep_y<N1, false, false>(P.D, v, gy);
+          const Number *M = point_data(P, kMetricComps, cxb, cy);
           const bool idle = N1 == 3 && row == 3;
 #pragma unroll
           for (int j = 0; j < N1; ++j)
@@ -913,14 +1023,137 @@ __global__ __launch_bounds__(256) void brick_fixup_kernel(Number *__restrict__ d
   }
 }
 
+template <int N1> struct TangentPoints {
+  BrickArgs<double, N1> A;
+  mpdg_heat_material mat;
+  double rdt, vol, rh[3], vel[3];  // 1 / dt, 1 / h: a division per point and term would take most of the time
+  const double *vf;
+  long n_dofs;
+};
+
+// The tangent's coefficients (tangent.hip) at the points of Q1..Q3 cells. One wavefront per pencil of 16
+// cells along x in the apply's lane layout, so that a coefficient of 16 cells is stored at once. What bounds
+// it: the stores, 6 of the 8 values per point with a constant velocity (Q2 70 x 50 x 33 with solidification,
+// 150 MB: 54 us with 8 values and the lanes of a cell side by side, 35 us here; 49 us with three wavefronts per
+// SIMD, which spill. Stored past the caches it is no faster and the apply that follows takes 77 us, not 56).
+template <int N1>
+__global__ __launch_bounds__(64 * kNW) __attribute__((amdgpu_waves_per_eu(N1 == 4 ? 1 : 2)))
+void tangent_points_kernel(const TangentPoints<N1> X, const double *__restrict__ T,
+                                                                  const double *__restrict__ T_old, double *__restrict__ td) {
+  using B = BrickShape<N1>;
+  constexpr int K = B::K, NQ = N1 * N1 * N1;
+  const auto &P = X.A;
+  const int lane = threadIdx.x & 63, row = lane >> 4, c = lane & 15, l = N1 == 2 ? row & 1 : row;
+  const int px = (P.nc[0] + kNX - 1) / kNX, pz = (P.nc[2] + B::ZPW - 1) / B::ZPW;
+  long p = (long)blockIdx.x * kNW + (threadIdx.x >> 6);
+  if (p >= (long)px * P.nc[1] * pz) return;
+  const int cxb = kNX * (int)(p % px);
+  p /= px;
+  const int cy = (int)(p % P.nc[1]), cz = B::ZPW * (int)(p / P.nc[1]) + (N1 == 2 ? row >> 1 : 0);
+  // lanes without a cell work on the mesh's last one and store nothing; Q2's idle row holds zeros
+  const int cx = min(cxb + c, P.nc[0] - 1);
+  const long sy = P.nd[0], at = K * cx + sy * ((long)K * cy + P.nd[1] * ((long)K * min(cz, P.nc[2] - 1) + min(l, K)));
+  auto load = [&](const double *f, double (&u)[N1][N1]) {
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) u[j][i] = N1 != 3 || row < 3 ? f[at + i + sy * j] : 0.0;
+  };
+  const ZTables<N1, double> zt(P, P.S, P.G, lane);
+  auto to_points = [&](const double *f, double (&v)[N1][N1]) {
+    double u[N1][N1], t[N1][N1];
+    load(f, u);
+    sweep_x<N1, false, false>(P.S, u, t);
+    sweep_y<N1, false, false>(P.S, t, u);
+    z_forward<N1, false>(P.S, P.G, zt, u, v, v);
+  };
+  double v[N1][N1], g[3][N1][N1], r[N1][N1];
+  {
+    double u[N1][N1], t[N1][N1];
+    load(T, u);
+    sweep_x<N1, false, false>(P.S, u, t);
+    sweep_y<N1, false, false>(P.S, t, u);
+    z_forward<N1, true>(P.S, P.G, zt, u, v, g[2]);
+    sweep_x<N1, false, false>(P.D, v, g[0]);
+    sweep_y<N1, false, false>(P.D, v, g[1]);
+  }
+  // r = (T - T_old) / dt + grad T . velocity, the factor of d rho c_p / dT
+  const bool solid = P.solid;
+  if (solid) {
+    to_points(T_old, r);
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        r[j][i] = (v[j][i] - r[j][i]) * X.rdt;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          g[d][j][i] *= X.rh[d];
+          if (!X.vf) r[j][i] += g[d][j][i] * X.vel[d];
+        }
+      }
+  }
+  const bool mine = cxb + c < P.nc[0] && cz < P.nc[2] && l <= K;
+  const long pencil = cxb / kNX + (long)px * (cy + (long)P.nc[1] * cz);
+  double *const out = td + (pencil * kTangentCoeffs * NQ + l) * kNX + c;
+  auto put = [&](int comp, int j, int i, double x) {
+    if (mine) out[(comp * NQ + (N1 * j + i) * N1) * kNX] = x;
+  };
+  double wz = 0.0;
+#pragma unroll
+  for (int a = 0; a < N1; ++a) wz = l == a ? P.w[a < N1 - 1 - a ? a : N1 - 1 - a] : wz;
+  auto weight = [&](int j, int i) {
+    return X.vol * wz * P.w[j < N1 - 1 - j ? j : N1 - 1 - j] * P.w[i < N1 - 1 - i ? i : N1 - 1 - i];
+  };
+  if (X.vf) {
+    double rc[N1][N1];
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        double k, drc, dk;
+        material(X.mat, v[j][i], rc[j][i], k, drc, dk);
+      }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      double w[N1][N1];
+      to_points(X.vf + d * X.n_dofs, w);
+#pragma unroll
+      for (int j = 0; j < N1; ++j)
+#pragma unroll
+        for (int i = 0; i < N1; ++i) {
+          if (solid) r[j][i] += g[d][j][i] * w[j][i];
+          put(2 + d, j, i, weight(j, i) * rc[j][i] * w[j][i] * X.rh[d]);
+        }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N1; ++j)
+#pragma unroll
+    for (int i = 0; i < N1; ++i) {
+      const double JxW = weight(j, i);
+      double rc, k, drc, dk;
+      material(X.mat, v[j][i], rc, k, drc, dk);
+      double m = rc * X.rdt;
+      if (solid) m += drc * r[j][i];
+      put(0, j, i, JxW * m);
+      put(1, j, i, JxW * k);
+      if (P.conv == 1) put(2, j, i, JxW * rc);
+      if (solid) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) put(5 + d, j, i, JxW * dk * g[d][j][i] * X.rh[d]);
+      }
+    }
+}
+
+// unit: the data per point carries the volume and the 1/h (mapped cells, the tangent)
 template <int N1, typename Number>
-int fill_brick_args(const OperatorData<Number> &op, BrickArgs<Number, N1> &A) {
-  const bool mapped = op.metric != nullptr;
+int fill_brick_args(const OperatorData<Number> &op, bool unit, BrickArgs<Number, N1> &A) {
   const FE1D &fe = fe1d(N1 - 1);
-  const double vol = mapped ? 1.0 : op.h[0] * op.h[1] * op.h[2];
+  const double vol = unit ? 1.0 : op.h[0] * op.h[1] * op.h[2];
   double Dy[kMaxN1][kMaxN1], Gz[kMaxN1][kMaxN1], M1[kMaxN1][kMaxN1] = {}, K1[kMaxN1][kMaxN1] = {};
-  const double ry = mapped ? 1.0 : (op.h[0] * op.h[0]) / (op.h[1] * op.h[1]);
-  const double rz = mapped ? 1.0 : (op.h[0] * op.h[0]) / (op.h[2] * op.h[2]);
+  const double ry = unit ? 1.0 : (op.h[0] * op.h[0]) / (op.h[1] * op.h[1]);
+  const double rz = unit ? 1.0 : (op.h[0] * op.h[0]) / (op.h[2] * op.h[2]);
   for (int q = 0; q < N1; ++q)
     for (int i = 0; i < N1; ++i) {
       Dy[q][i] = fe.D[q][i] * ry;
@@ -947,9 +1180,9 @@ int fill_brick_args(const OperatorData<Number> &op, BrickArgs<Number, N1> &A) {
   A.dmask = op.dmask;
   A.law = op.law;
   A.cm = (Number)(op.c_mass * vol);
-  A.kx = (Number)(mapped ? 1.0 : vol / (op.h[0] * op.h[0]));
-  A.ky = (Number)(mapped ? 1.0 : vol / (op.h[1] * op.h[1]));
-  A.kz = (Number)(mapped ? 1.0 : vol / (op.h[2] * op.h[2]));
+  A.kx = (Number)(unit ? 1.0 : vol / (op.h[0] * op.h[0]));
+  A.ky = (Number)(unit ? 1.0 : vol / (op.h[1] * op.h[1]));
+  A.kz = (Number)(unit ? 1.0 : vol / (op.h[2] * op.h[2]));
   A.kappa = (Number)op.kappa;
   for (int i = 0; i < 4; ++i) A.law_p[i] = (Number)op.law_p[i];
   A.kappa_arr = op.kappa_arr;
@@ -958,6 +1191,8 @@ int fill_brick_args(const OperatorData<Number> &op, BrickArgs<Number, N1> &A) {
   A.scratch = op.edge;
   A.T_old = A.q = nullptr;
   A.fa = A.fb = A.fc = Number(0);
+  A.conv = A.solid = 0;
+  A.vh[0] = A.vh[1] = A.vh[2] = Number(0);
   return A.g.total > 0 && (op.edge == nullptr || (size_t)A.g.total > op.edge_elems) ? MPDG_ERR_INVALID : MPDG_OK;
 }
 
@@ -981,7 +1216,7 @@ template <int N1, typename Number>
 int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                     hipEvent_t kernel_start, hipEvent_t kernel_end) {
   BrickArgs<Number, N1> A;
-  if (const int rc = fill_brick_args(op, A)) return rc;
+  if (const int rc = fill_brick_args(op, op.metric != nullptr, A)) return rc;
   if (kernel_start) (void)hipEventRecord(kernel_start, stream);
   if (op.metric) {
     switch (op.kappa_mode) {
@@ -1007,7 +1242,7 @@ int launch_brick_residual_n1(const OperatorData<double> &op, const double *src, 
                              double b, double c, double *dst, hipStream_t stream) {
   using Number = double;
   BrickArgs<Number, N1> A;
-  if (const int rc = fill_brick_args(op, A)) return rc;
+  if (const int rc = fill_brick_args(op, false, A)) return rc;
   A.fa = a;
   A.fb = b;
   A.fc = c;
@@ -1023,7 +1258,70 @@ int launch_brick_residual_n1(const OperatorData<double> &op, const double *src, 
   return finish_brick(A, dst, stream);
 }
 
+template <int N1>
+void fill_tangent_args(const OperatorData<double> &op, const double *vel, const double *vfield, int solid, BrickArgs<double, N1> &A) {
+  A.conv = tangent_convects(vel, vfield);
+  A.solid = solid;
+  for (int d = 0; d < 3; ++d) A.vh[d] = vel[d] / op.h[d];
+}
+
+// src null: the diagonal
+template <int N1>
+int launch_brick_tangent_n1(const OperatorData<double> &op, const double *td, const double *vel, const double *vfield, int solid,
+                            const double *src, double *dst, hipStream_t stream) {
+  using Number = double;
+  BrickArgs<Number, N1> A;
+  if (const int rc = fill_brick_args(op, true, A)) return rc;
+  fill_tangent_args(op, vel, vfield, solid, A);
+  A.metric = td;
+  A.kx = 1.0 / (op.h[0] * op.h[0]);
+  A.ky = 1.0 / (op.h[1] * op.h[1]);
+  A.kz = 1.0 / (op.h[2] * op.h[2]);
+  if (src) {
+    MPDG_BRICK(KAPPA_TANGENT, false, false);
+  } else {
+    const FE1D &fe = fe1d(N1 - 1);
+    double SS[kMaxN1][kMaxN1], SG[kMaxN1][kMaxN1], GG[kMaxN1][kMaxN1];
+    for (int q = 0; q < N1; ++q)
+      for (int i = 0; i < N1; ++i) {
+        SS[i][q] = fe.S[q][i] * fe.S[q][i];
+        SG[i][q] = fe.S[q][i] * fe.G[q][i];
+        GG[i][q] = fe.G[q][i] * fe.G[q][i];
+      }
+    A.S.set(SS);
+    A.G.set(SG);
+    A.M1.set(GG);
+    MPDG_BRICK(TANGENT_DIAGONAL, false, false);
+  }
+  return finish_brick(A, dst, stream);
+}
 #undef MPDG_BRICK
+
+template <int N1>
+int launch_brick_tangent_data_n1(const OperatorData<double> &op, double dt, const mpdg_heat_material &mat, int solid,
+                                 const double *vel, const double *vfield, const double *T, const double *T_old, double *td,
+                                 hipStream_t stream) {
+  TangentPoints<N1> X;
+  X.A.dmask = 0;
+  OperatorData<double> plain = op;
+  plain.edge = nullptr;
+  plain.edge_elems = 0;
+  (void)fill_brick_args(plain, false, X.A);  // (no scratch is used)
+  fill_tangent_args(op, vel, vfield, solid, X.A);
+  X.mat = mat;
+  X.rdt = 1.0 / dt;
+  X.vol = op.h[0] * op.h[1] * op.h[2];
+  for (int d = 0; d < 3; ++d) {
+    X.rh[d] = 1.0 / op.h[d];
+    X.vel[d] = vel[d];
+  }
+  X.vf = vfield;
+  X.n_dofs = op.n_dofs;
+  const long waves = (long)((op.nc[0] + kNX - 1) / kNX) * op.nc[1] * ((op.nc[2] + BrickShape<N1>::ZPW - 1) / BrickShape<N1>::ZPW);
+  hipLaunchKernelGGL(tangent_points_kernel<N1>, dim3((unsigned)((waves + kNW - 1) / kNW)), dim3(64 * kNW), 0, stream, X, T,
+                     T_old, td);
+  return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
+}
 
 }  // namespace
 
@@ -1052,4 +1350,24 @@ int launch_brick_residual(const OperatorData<double> &op, const double *T, const
     default: return MPDG_ERR_INVALID;
   }
 }
+int launch_brick_tangent_data(const OperatorData<double> &op, double dt, const mpdg_heat_material &mat, int solid,
+                              const double *vel, const double *vfield, const double *T, const double *T_old, double *td,
+                              hipStream_t stream) {
+  switch (op.degree) {
+    case 1: return launch_brick_tangent_data_n1<2>(op, dt, mat, solid, vel, vfield, T, T_old, td, stream);
+    case 2: return launch_brick_tangent_data_n1<3>(op, dt, mat, solid, vel, vfield, T, T_old, td, stream);
+    case 3: return launch_brick_tangent_data_n1<4>(op, dt, mat, solid, vel, vfield, T, T_old, td, stream);
+    default: return MPDG_ERR_INVALID;
+  }
+}
+int launch_brick_tangent(const OperatorData<double> &op, const double *td, const double *vel, const double *vfield, int solid,
+                         const double *src, double *dst, hipStream_t stream) {
+  switch (op.degree) {
+    case 1: return launch_brick_tangent_n1<2>(op, td, vel, vfield, solid, src, dst, stream);
+    case 2: return launch_brick_tangent_n1<3>(op, td, vel, vfield, solid, src, dst, stream);
+    case 3: return launch_brick_tangent_n1<4>(op, td, vel, vfield, solid, src, dst, stream);
+    default: return MPDG_ERR_INVALID;
+  }
+}
+
 }  // namespace mpdg

@@ -41,7 +41,7 @@ int mpdg_heat_op::vmult_cells(double *dst, const double *src, hipStream_t s) con
   if (d64.metric && d64.kappa_mode == KAPPA_LAW) MPDG_TRY(refresh_metric_k(s));  // k(T) with the current T
   if (tangent) {
     if (!td_bound) return MPDG_ERR_INVALID;
-    return launch_tangent_apply(d64, td.get(), tangent_convects(vel, vfield), solid, src, dst, s);
+    return launch_tangent_apply(d64, td.get(), vel, vfield, solid, src, dst, s);
   }
   if (!timing_on) return launch_apply<double>(d64, src, dst, s);
   if (timing_used == timing_events.size()) {
@@ -93,7 +93,8 @@ int mpdg_heat_op::vmult_f32(float *dst, const float *src, hipStream_t s) const {
 int mpdg_heat_op::diagonal64(double *diag, hipStream_t s) const {
   if (tangent) {
     if (!td_bound) return MPDG_ERR_INVALID;
-    MPDG_TRY(launch_tangent_diagonal(d64, td.get(), tangent_convects(vel, vfield), solid, diag, s));
+    MPDG_TRY(ensure_edge());
+    MPDG_TRY(launch_tangent_diagonal(d64, td.get(), vel, vfield, solid, diag, s));
     if (d64.robin_mask) MPDG_TRY(launch_boundary(d64, 1, nullptr, diag, nullptr, T_robin, s));
     return MPDG_OK;
   }
@@ -1268,7 +1269,7 @@ int mpdg_heat_op_set_tangent(mpdg_heat_op *op, const mpdg_heat_material *mat, in
   op->solid = do_solidification ? 1 : 0;
   for (int i = 0; i < 3; ++i) op->vel[i] = velocity3[i];
   const int n1 = op->d64.degree + 1;
-  MPDG_TRY(op->td.resize((size_t)kTangentCoeffs * op->d64.n_cells * n1 * n1 * n1));
+  MPDG_TRY(op->td.resize(point_data_elems(n1, op->d64.nc, kTangentCoeffs)));
   op->tangent = true;
   op->td_bound = false;
   return MPDG_OK;
@@ -1370,9 +1371,8 @@ int mpdg_heat_op_vmult_noalloc(const mpdg_heat_op *op, double *dst, const double
   if (!op || !dst || !src || op->precision != MPDG_FP64) return MPDG_ERR_INVALID;
   hipStream_t s = S(stream);
   if (op->tangent) {
-    // the full tangent's kernels use no scratch
     if (!op->td_bound) return MPDG_ERR_INVALID;
-    MPDG_TRY(launch_tangent_apply(op->d64, op->td.get(), tangent_convects(op->vel, op->vfield), op->solid, src, dst, s));
+    MPDG_TRY(launch_tangent_apply(op->d64, op->td.get(), op->vel, op->vfield, op->solid, src, dst, s));
   } else {
     if (op->d64.metric && op->d64.kappa_mode == KAPPA_LAW) {
       // k(T) on a mapped mesh rescales the metric into operator-owned arrays: only when they

@@ -70,20 +70,26 @@ struct OperatorData {
   }
 };
 
-// Where component comp of quadrature point q = (qx, qy, qz) of a cell's metric lies. Q1..Q3:
-// [pencil of 16 cells along x][comp][qy][qx][qz][cell of the pencil], so that each load of the apply's
-// wavefront (lane = 16 qz + cell) is contiguous (Q3 96^3 FP64 apply: 0.88 ms; 2.4 ms with [cell][comp][q],
-// where every lane reads its own line); Q4, whose kernel gives a lane consecutive qx: [cell][comp][q].
-__host__ __device__ __forceinline__ long metric_at(int n1, int nc0, long cell, int comp, int qx, int qy, int qz) {
+// Where component comp (of ncomp) of quadrature point q = (qx, qy, qz) of a cell lies in the per-point
+// arrays the library makes itself (the metric, the tangent's coefficients). Q1..Q3: [pencil of 16 cells
+// along x][comp][qy][qx][qz][cell of the pencil], so that each load of the apply's wavefront
+// (lane = 16 qz + cell) is contiguous (mapped Q3 96^3 FP64 apply: 0.82 ms; 2.4 ms with [cell][comp][q], where
+// every lane reads its own line); Q4, whose kernels give a lane consecutive qx: [cell][comp][q].
+__host__ __device__ __forceinline__ long point_data_at(int n1, int nc0, long cell, int ncomp, int comp, int qx, int qy, int qz) {
   const int nq = n1 * n1 * n1;
-  if (n1 == 5) return (cell * 7 + comp) * nq + qx + n1 * (qy + n1 * qz);
+  if (n1 == 5) return (cell * ncomp + comp) * nq + qx + n1 * (qy + n1 * qz);
   const long row = cell / nc0, cx = cell - row * nc0, pencil = row * ((nc0 + 15) / 16) + cx / 16;
-  return ((pencil * 7 + comp) * nq + (qy * n1 + qx) * n1 + qz) * 16 + cx % 16;
+  return ((pencil * ncomp + comp) * nq + (qy * n1 + qx) * n1 + qz) * 16 + cx % 16;
 }
-inline size_t metric_elems(int n1, const int *nc) {
+inline size_t point_data_elems(int n1, const int *nc, int ncomp) {
   const size_t cells_x = n1 == 5 ? nc[0] : (nc[0] + 15) / 16 * 16;
-  return cells_x * nc[1] * nc[2] * 7 * n1 * n1 * n1;
+  return cells_x * nc[1] * nc[2] * ncomp * n1 * n1 * n1;
 }
+constexpr int kMetricComps = 7;
+__host__ __device__ __forceinline__ long metric_at(int n1, int nc0, long cell, int comp, int qx, int qy, int qz) {
+  return point_data_at(n1, nc0, cell, kMetricComps, comp, qx, qy, qz);
+}
+inline size_t metric_elems(int n1, const int *nc) { return point_data_elems(n1, nc, kMetricComps); }
 
 // A 1D N1 x N1 table stored by its symmetry about the cell centre (Gauss-Lobatto nodes and
 // Gauss points are symmetric): T[N1-1-q][N1-1-i] = T[q][i] (ANTI = false, shape values) or

@@ -11,9 +11,12 @@
 //   t0 = JxW (rho_cp/dt [+ d rho_cp/dT ((T - T_old)/dt + grad T . v)])
 //   t1 = JxW k                                           (times 1/h_d^2 d u / d xi_d)
 //   t2..t4 = JxW rho_cp v_d / h_d          [velocity]     (times d u / d xi_d)
+//            (Q1..Q3 with a constant velocity: t2 = JxW rho_cp alone)
 //   t5..t7 = JxW dk/dT (grad T)_d / h_d  [solidification] (gradient slot, times u)
 // Coefficients a problem does not have (no velocity, no solidification) are neither written
-// nor read. The apply, residual and diagonal kernels are cell-local sum factorization with one
+// nor read. Q1..Q3: the coefficients and the apply have the lane layout of heat_brick.hip, one launch each
+// and the sums of shared planes (bind and apply of Q2 70 x 50 x 33 with solidification and a constant
+// velocity: 195 us with eight coloured launches, 135 us so). The kernels below are for Q4 and for the residual: cell-local sum factorization with one
 // thread per line of the cell's N1^3 tensor (N1^2 threads per cell) and LDS transposes between
 // the directions. A block holds a segment of an x-row of cells; it loads and stores its DoFs as
 // N1^2 lines along x with consecutive lanes on consecutive addresses, sums the shared x-faces in
@@ -46,6 +49,9 @@ Tables1D make_tables(int k) {
 
 template <int N1>
 constexpr int kCells = 256 / (N1 * N1);
+// LDS values of a cell's array: odd where neighbouring lanes are neighbouring cells (bank conflicts)
+template <int N1>
+constexpr int kCellStride = N1 < 5 ? N1 * N1 * N1 | 1 : N1 * N1 * N1;
 
 struct Geometry {
   int nc0, nc1, nc2;
@@ -54,7 +60,7 @@ struct Geometry {
   int nd[3];
   int dmask;
   double h[3], ih2[3], vol, dt;
-  int conv, solid;  // coefficients t2..t4 / t5..t7 present
+  int conv, solid;  // tangent_convects; coefficients t5..t7 present
 };
 
 __device__ __forceinline__ bool is_constrained(int m, const int *nd, int ix, int iy, int iz) {
@@ -85,8 +91,13 @@ struct Place {
   bool in_block, active;
   __device__ Place(const Geometry &g) {
     constexpr int L2 = N1 * N1, K = N1 - 1, CPB = kCells<N1>;
-    lc = threadIdx.x / L2;
-    r = threadIdx.x - lc * L2;
+    if (N1 < 5) {  // cells fastest: fewer bank conflicts (residual of Q3 50 x 40 x 30: 131 -> 118 us)
+      r = threadIdx.x / CPB;
+      lc = threadIdx.x - r * CPB;
+    } else {
+      lc = threadIdx.x / L2;
+      r = threadIdx.x - lc * L2;
+    }
     a = r / N1;
     b = r - a * N1;
     const int nseg = (g.nc0 + CPB - 1) / CPB;
@@ -110,8 +121,8 @@ struct Place {
     ix0 = K * x0;
     iy0 = K * cy;
     iz0 = K * cz;
-    in_block = lc < CPB;
-    active = lc < ncb;
+    in_block = threadIdx.x < CPB * L2;
+    active = in_block && lc < ncb;
     cell = row * g.nc0 + x0 + lc;
   }
   // DoF indices of entry e = r' kLine + x of the block's lines (r' = a' N1 + b': z-line a',
@@ -329,27 +340,6 @@ __device__ void scatter(const Geometry &g, const Place<N1> &p, double *dst, cons
   }
 }
 
-// material of the tangent (the oracle's `material`, material.templates.hpp:296-380, :546-598, :765-778)
-__device__ __forceinline__ void material(const mpdg_heat_material &m, double T, double &rc, double &k, double &drc,
-                                         double &dk) {
-  if (m.transition == MPDG_TRANSITION_NONE) {
-    rc = m.density[0] * m.specific_heat[0];
-    k = m.conductivity[0];
-    drc = dk = 0.0;
-    return;
-  }
-  const double inv = 1.0 / (m.liquidus - m.solidus);
-  const double fs = fmin(1.0, fmax(0.0, (m.liquidus - T) * inv));
-  const bool pure = fs == 0.0 || fs == 1.0;
-  const double c = 3.0 * fs * fs - 2.0 * fs * fs * fs, dc = pure ? 0.0 : -inv * (6.0 * fs - 6.0 * fs * fs);
-  auto blend = [&](const double *x) { return fs == 0.0 ? x[0] : (fs == 1.0 ? x[1] : x[0] + (x[1] - x[0]) * c); };
-  const double rho = blend(m.density), cp = blend(m.specific_heat);
-  k = blend(m.conductivity);
-  dk = (m.conductivity[1] - m.conductivity[0]) * dc;
-  rc = rho * cp;
-  drc = (m.specific_heat[1] - m.specific_heat[0]) * dc * rho + (m.density[1] - m.density[0]) * dc * cp;
-}
-
 struct TangentArgs {
   Geometry g;
   mpdg_heat_material mat;
@@ -361,7 +351,7 @@ struct TangentArgs {
 // velocity at the quadrature points (qz = 0..N1-1 of this thread's (qy, qx) column): the
 // constant vector, or the field's values (gathered into lds[0], evaluated through lds[1], lds[3])
 template <int N1>
-__device__ void velocity_at_points(const Tables1D &t, const TangentArgs &A, const Place<N1> &p, double (*lds)[kCells<N1> * N1 * N1 * N1],
+__device__ void velocity_at_points(const Tables1D &t, const TangentArgs &A, const Place<N1> &p, double (*lds)[kCells<N1> * kCellStride<N1>],
                                    int o, double (&w)[3][N1]) {
   if (!A.vf) {
 #pragma unroll
@@ -384,9 +374,9 @@ template <int N1>
 __global__ __launch_bounds__(256) void tangent_data_kernel(Tables1D t, TangentArgs A, const double *__restrict__ T,
                                                            const double *__restrict__ T_old, double *__restrict__ td) {
   constexpr int NQ = N1 * N1 * N1, CPB = kCells<N1>;
-  __shared__ double lds[5][CPB * NQ];
+  __shared__ double lds[5][CPB * kCellStride<N1>];
   const Place<N1> p(A.g);
-  const int o = (p.in_block ? p.lc : 0) * NQ;
+  const int o = (p.in_block ? p.lc : 0) * kCellStride<N1>;
   double u[N1], tq[N1], gx[N1], gy[N1], gz[N1], to[N1];
   gather<N1>(A.g, p, T, false, lds[4], u);
   evaluate<N1, true>(t, p, u, lds[0] + o, lds[1] + o, lds[2] + o, lds[3] + o, lds[4] + o, tq, gx, gy, gz);
@@ -419,9 +409,9 @@ template <int N1>
 __global__ __launch_bounds__(256) void tangent_apply_kernel(Tables1D t, Geometry g, const double *__restrict__ td,
                                                             const double *__restrict__ src, double *__restrict__ dst) {
   constexpr int NQ = N1 * N1 * N1, CPB = kCells<N1>;
-  __shared__ double lds[5][CPB * NQ];
+  __shared__ double lds[5][CPB * kCellStride<N1>];
   const Place<N1> p(g);
-  const int o = (p.in_block ? p.lc : 0) * NQ;
+  const int o = (p.in_block ? p.lc : 0) * kCellStride<N1>;
   double u[N1], v[N1], gx[N1], gy[N1], gz[N1];
   gather<N1>(g, p, src, true, lds[4], u);
   evaluate<N1, true>(t, p, u, lds[0] + o, lds[1] + o, lds[2] + o, lds[3] + o, lds[4] + o, v, gx, gy, gz);
@@ -453,10 +443,10 @@ __global__ __launch_bounds__(256) void tangent_residual_kernel(Tables1D t, Tange
                                                                const double *__restrict__ T_old,
                                                                const double *__restrict__ qv, double *__restrict__ dst) {
   constexpr int NQ = N1 * N1 * N1, CPB = kCells<N1>;
-  __shared__ double lds[5][CPB * NQ];
+  __shared__ double lds[5][CPB * kCellStride<N1>];
   const Place<N1> p(A.g);
   const Geometry &g = A.g;
-  const int o = (p.in_block ? p.lc : 0) * NQ;
+  const int o = (p.in_block ? p.lc : 0) * kCellStride<N1>;
   double u[N1], tq[N1], gx[N1], gy[N1], gz[N1], to[N1], qq[N1];
   gather<N1>(g, p, T, false, lds[4], u);
   evaluate<N1, true>(t, p, u, lds[0] + o, lds[1] + o, lds[2] + o, lds[3] + o, lds[4] + o, tq, gx, gy, gz);
@@ -503,9 +493,9 @@ __global__ __launch_bounds__(256) void tangent_diagonal_kernel(Tables1D t, Geome
                                                                double *__restrict__ diag) {
   constexpr int NQ = N1 * N1 * N1, CPB = kCells<N1>;
   constexpr int fx[7] = {0, 2, 0, 0, 1, 0, 0}, fy[7] = {0, 0, 2, 0, 0, 1, 0}, fz[7] = {0, 0, 0, 2, 0, 0, 1};
-  __shared__ double lds[2][CPB * NQ];
+  __shared__ double lds[2][CPB * kCellStride<N1>];
   const Place<N1> p(g);
-  double *B0 = lds[0] + (p.in_block ? p.lc : 0) * NQ, *B1 = lds[1] + (p.in_block ? p.lc : 0) * NQ;
+  double *B0 = lds[0] + (p.in_block ? p.lc : 0) * kCellStride<N1>, *B1 = lds[1] + (B0 - lds[0]);
   double d[N1], u[N1];
 #pragma unroll
   for (int i = 0; i < N1; ++i) d[i] = 0.0;
@@ -573,7 +563,7 @@ __global__ __launch_bounds__(256) void unit_constrained_kernel(double *v, Geomet
 
 Geometry geometry(const OperatorData<double> &op, double dt, int conv = 0, int solid = 0) {
   Geometry g{};
-  g.conv = conv ? 1 : 0;
+  g.conv = conv;
   g.solid = solid ? 1 : 0;
   g.nc0 = op.nc[0];
   g.nc1 = op.nc[1];
@@ -593,43 +583,33 @@ Geometry geometry(const OperatorData<double> &op, double dt, int conv = 0, int s
 
 int finish(hipStream_t) { return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE; }
 
-// one launch over all blocks (GEO.color = -1), or eight, one per colour (COLORS = 8)
-#define MPDG_TANGENT_DISPATCH(KERNEL, GEO, COLORS, ...)                                                           \
-  if (op.degree < 1 || op.degree > 4) return MPDG_ERR_INVALID;                                                   \
-  for (int color_ = (COLORS) > 1 ? 0 : -1; color_ < ((COLORS) > 1 ? (COLORS) : 0); ++color_) {                  \
-    GEO.color = color_;                                                                                          \
-    const long nb_ = tangent_blocks(op.degree + 1, op.nc, color_);                                               \
-    if (nb_ == 0) continue;                                                                                      \
-    switch (op.degree) {                                                                                         \
-      case 1: hipLaunchKernelGGL(KERNEL<2>, dim3(nb_), dim3(256), 0, s, __VA_ARGS__); break;                     \
-      case 2: hipLaunchKernelGGL(KERNEL<3>, dim3(nb_), dim3(256), 0, s, __VA_ARGS__); break;                     \
-      case 3: hipLaunchKernelGGL(KERNEL<4>, dim3(nb_), dim3(256), 0, s, __VA_ARGS__); break;                     \
-      default: hipLaunchKernelGGL(KERNEL<5>, dim3(nb_), dim3(256), 0, s, __VA_ARGS__); break;                    \
-    }                                                                                                            \
-  }
-
 }  // namespace
 
 int launch_tangent_data(const OperatorData<double> &op, double dt, const mpdg_heat_material &mat, int solid,
                         const double *vel, const double *vfield, const double *T, const double *T_old, double *td,
                         hipStream_t s) {
+  if (op.degree < 4) return launch_brick_tangent_data(op, dt, mat, solid, vel, vfield, T, T_old, td, s);
   TangentArgs A{};
   A.g = geometry(op, dt, tangent_convects(vel, vfield), solid);
   A.mat = mat;
   for (int d = 0; d < 3; ++d) A.vel[d] = vel[d];
   A.vf = vfield;
   A.solid = solid;
-  const Tables1D t = make_tables(op.degree);
-  MPDG_TANGENT_DISPATCH(tangent_data_kernel, A.g, 1, t, A, T, T_old, td)
+  hipLaunchKernelGGL(tangent_data_kernel<5>, dim3(tangent_blocks(5, op.nc)), dim3(256), 0, s, make_tables(op.degree), A, T, T_old,
+                     td);
   return finish(s);
 }
 
-int launch_tangent_apply(const OperatorData<double> &op, const double *td, int conv, int solid,
+int launch_tangent_apply(const OperatorData<double> &op, const double *td, const double *vel, const double *vfield, int solid,
                          const double *src, double *dst, hipStream_t s) {
-  Geometry g = geometry(op, 1.0, conv, solid);
+  if (op.degree < 4) return launch_brick_tangent(op, td, vel, vfield, solid, src, dst, s);
+  Geometry g = geometry(op, 1.0, tangent_convects(vel, vfield), solid);
   const Tables1D t = make_tables(op.degree);
   if (hipMemsetAsync(dst, 0, sizeof(double) * op.n_dofs, s) != hipSuccess) return MPDG_ERR_DEVICE;
-  MPDG_TANGENT_DISPATCH(tangent_apply_kernel, g, 8, t, g, td, src, dst)
+  for (g.color = 0; g.color < 8; ++g.color) {
+    const long nb = tangent_blocks(5, op.nc, g.color);
+    if (nb > 0) hipLaunchKernelGGL(tangent_apply_kernel<5>, dim3(nb), dim3(256), 0, s, t, g, td, src, dst);
+  }
   return finish(s);
 }
 
@@ -642,16 +622,33 @@ int launch_tangent_residual(const OperatorData<double> &op, double dt, const mpd
   for (int d = 0; d < 3; ++d) A.vel[d] = vel[d];
   A.vf = vfield;
   const Tables1D t = make_tables(op.degree);
-  MPDG_TANGENT_DISPATCH(tangent_residual_kernel, A.g, 8, t, A, T, T_old, q, dst)
+  if (op.degree < 1 || op.degree > 4) return MPDG_ERR_INVALID;
+  for (A.g.color = 0; A.g.color < 8; ++A.g.color) {
+    const long nb = tangent_blocks(op.degree + 1, op.nc, A.g.color);
+    if (nb == 0) continue;
+    switch (op.degree) {
+      case 1: hipLaunchKernelGGL(tangent_residual_kernel<2>, dim3(nb), dim3(256), 0, s, t, A, T, T_old, q, dst); break;
+      case 2: hipLaunchKernelGGL(tangent_residual_kernel<3>, dim3(nb), dim3(256), 0, s, t, A, T, T_old, q, dst); break;
+      case 3: hipLaunchKernelGGL(tangent_residual_kernel<4>, dim3(nb), dim3(256), 0, s, t, A, T, T_old, q, dst); break;
+      default: hipLaunchKernelGGL(tangent_residual_kernel<5>, dim3(nb), dim3(256), 0, s, t, A, T, T_old, q, dst); break;
+    }
+  }
   return finish(s);
 }
 
-int launch_tangent_diagonal(const OperatorData<double> &op, const double *td, int conv, int solid,
-                            double *diag, hipStream_t s) {
-  Geometry g = geometry(op, 1.0, conv, solid);
-  const Tables1D t = make_tables(op.degree);
-  if (hipMemsetAsync(diag, 0, sizeof(double) * op.n_dofs, s) != hipSuccess) return MPDG_ERR_DEVICE;
-  MPDG_TANGENT_DISPATCH(tangent_diagonal_kernel, g, 8, t, g, td, diag)
+int launch_tangent_diagonal(const OperatorData<double> &op, const double *td, const double *vel, const double *vfield,
+                            int solid, double *diag, hipStream_t s) {
+  Geometry g = geometry(op, 1.0, tangent_convects(vel, vfield), solid);
+  if (op.degree < 4) {
+    if (const int rc = launch_brick_tangent(op, td, vel, vfield, solid, nullptr, diag, s)) return rc;
+  } else {
+    const Tables1D t = make_tables(op.degree);
+    if (hipMemsetAsync(diag, 0, sizeof(double) * op.n_dofs, s) != hipSuccess) return MPDG_ERR_DEVICE;
+    for (g.color = 0; g.color < 8; ++g.color) {
+      const long nb = tangent_blocks(5, op.nc, g.color);
+      if (nb > 0) hipLaunchKernelGGL(tangent_diagonal_kernel<5>, dim3(nb), dim3(256), 0, s, t, g, td, diag);
+    }
+  }
   if (op.dmask)
     hipLaunchKernelGGL(unit_constrained_kernel, dim3((op.n_dofs + 255) / 256), dim3(256), 0, s, diag, g, op.n_dofs);
   return finish(s);

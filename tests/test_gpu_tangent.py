@@ -118,6 +118,31 @@ def test_tangent_velocity_field_matches_oracle(cuda, degree, nc, L, dmask, solid
     assert np.linalg.norm(dst.cpu().numpy() - ref) <= 1e-12 * np.linalg.norm(ref)
 
 
+# edges of the wavefronts' pencils (16 cells along x) and of the bricks (4 cells along z, Q1: 8)
+@pytest.mark.parametrize("field", [False, True])
+@pytest.mark.parametrize("degree,nc,solid", [(1, (17, 3, 9), True), (1, (16, 1, 8), False), (2, (33, 2, 5), True), (2, (1, 3, 4), False),
+                                             (3, (18, 2, 5), True)])
+def test_tangent_at_brick_edges(cuda, degree, nc, solid, field):
+    torch = cuda
+    import meltpooldg_amd as M
+    L = tuple(0.1 * n for n in nc)
+    orc, op, T, T_old, Td, Tod = pair(torch, M, degree, nc, L, 0b000001, solid, (0.2, -0.4, 0.1))
+    if field:
+        # the constant velocity as a field: the coefficients are then stored per direction
+        v = torch.tensor([0.2, -0.4, 0.1], dtype=torch.float64, device="cuda").repeat_interleave(op.n_dofs)
+        op.set_velocity_field(v)
+        op.bind_temperature(Td, Tod)
+    src = np.random.default_rng(6).uniform(-1, 1, orc.n_dofs)
+    dst = torch.full((orc.n_dofs,), float("nan"), dtype=torch.float64, device="cuda")
+    op.vmult(dst, torch.tensor(src, device="cuda"))
+    ref = orc.vmult(src, threads=1)
+    assert np.linalg.norm(dst.cpu().numpy() - ref) <= 1e-12 * np.linalg.norm(ref)
+    d = torch.empty_like(dst)
+    op.compute_diagonal(d)
+    ref = orc.diagonal()
+    assert np.linalg.norm(d.cpu().numpy() - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
 def test_velocity_field_needs_the_tangent(cuda):
     torch = cuda
     import meltpooldg_amd as M
