@@ -57,24 +57,16 @@ struct BrickGrid {
 };
 constexpr int kMaxSteps = 16, kMaxPencils = 2;
 
-// Steps along y and pencils along x per brick. Long bricks share fewer planes and amortise the
-// table set-up; short ones give the chip enough wavefronts: about 2048 workgroups while a brick is
-// shorter than 16 steps (Q2 64^3 FP32: 25.5 us; 1024: 29, 4096: 33; Q3 64^3 per cell FP32: 43 us against 48
-// and 49), then two pencils along x where more than 1024 remain (the x planes' fix-up is strided:
-// Q3 128^3 FP64 per point 619 us against 634 with one, 643 with four, whose LDS halves the occupancy).
-// The rule depends on the mesh only, so every apply of a mesh sums in the same order.
-BrickGrid brick_grid(int k, const int *nc) {
+constexpr int zc_of(int k) { return k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC; }
+BrickGrid brick_grid(int k, const int *nc, const int *brick) {
   BrickGrid g;
-  const int zc = k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC;
-  const int px = (nc[0] + kNX - 1) / kNX;
+  const int zc = zc_of(k), px = (nc[0] + kNX - 1) / kNX;
+  g.cells[0] = kNX * brick[0];
+  g.cells[1] = brick[1];
   g.cells[2] = zc;
+  g.nb[0] = (px + brick[0] - 1) / brick[0];
+  g.nb[1] = (nc[1] + brick[1] - 1) / brick[1];
   g.nb[2] = (nc[2] + zc - 1) / zc;
-  const long steps = (long)px * g.nb[2] * nc[1];  // workgroup steps of the whole apply
-  g.cells[1] = (int)std::min<long>({kMaxSteps, std::max<long>(1, steps / 2048), nc[1]});
-  g.nb[1] = (nc[1] + g.cells[1] - 1) / g.cells[1];
-  const int xb = (int)std::min<long>({kMaxPencils, std::max<long>(1, (long)px * g.nb[1] * g.nb[2] / 512), px});
-  g.cells[0] = kNX * xb;
-  g.nb[0] = (px + xb - 1) / xb;
   const long nd[3] = {(long)k * nc[0] + 1, (long)k * nc[1] + 1, (long)k * nc[2] + 1};
   long o = 0;
   g.off[0] = 0;
@@ -1176,7 +1168,7 @@ int fill_brick_args(const OperatorData<Number> &op, bool unit, BrickArgs<Number,
     A.nd[d] = op.nd[d];
   }
   A.n_cells = op.n_cells;
-  A.g = brick_grid(N1 - 1, op.nc);
+  A.g = brick_grid(N1 - 1, op.nc, op.brick);
   A.dmask = op.dmask;
   A.law = op.law;
   A.cm = (Number)(op.c_mass * vol);
@@ -1325,7 +1317,41 @@ int launch_brick_tangent_data_n1(const OperatorData<double> &op, double dt, cons
 
 }  // namespace
 
-size_t brick_scratch_elems(int degree, const int *nc) { return (size_t)brick_grid(degree, nc).total; }
+// Long bricks share fewer planes and set their tables up less often; short ones give every CU work, and end
+// the launch evenly. Taken is the shape with the least modelled time, in steps of one CU: full rounds of the
+// workgroups that are resident at once (4 per CU, Q1: 6), the rest (no faster than the latency of one
+// workgroup, which shows below 2.5 per CU), start-up, and the sums of the shared planes (the x planes'
+// strided, 8 times the others'). Measured over 28 meshes and kernels: 1.6% above the best shape on average
+// (at most 15%); about 2048 workgroups for every mesh: 5.7% (24%) (Q2 48 x 80 x 56 FP64 35.6 -> 28.7 us, Q2 70 x 50 x 33
+// 25.7 -> 22.6, Q3 75 x 62 x 49 FP32 49.6 -> 45.4, Q1 200 x 150 x 170 97.5 -> 88.5, Q2 64^3 and Q3 128^3 the
+// same shapes). It depends on the mesh only, so every apply of a mesh sums in the same order.
+void choose_brick(int k, const int *nc, int *brick) {
+  brick[0] = brick[1] = 1;
+  if (k > 3) return;
+  struct { double resident, latency, startup, planes; } static const model[4] = {
+      {}, {6, 4, 0.2, 1.0}, {4, 2.5, 0.7, 0.0}, {4, 2.5, 0.2, 0.5}};
+  const auto &m = model[k];
+  const long zc = zc_of(k), px = (nc[0] + kNX - 1) / kNX, nz = (nc[2] + zc - 1) / zc, cus = 256;
+  const double nd[3] = {k * (double)nc[0] + 1, k * (double)nc[1] + 1, k * (double)nc[2] + 1};
+  const double steps = (double)px * nc[1] * nz / cus;
+  double best = 0.0;
+  for (long xb = std::min<long>(kMaxPencils, px); xb >= 1; --xb)
+    for (long seg = std::min(kMaxSteps, nc[1]); seg >= 1; --seg) {
+      const long nx = (px + xb - 1) / xb, ny = (nc[1] + seg - 1) / seg, n = nx * ny * nz;
+      const long round = cus * (long)m.resident, rest = n % round;
+      double t = (double)(n / round) * m.resident;
+      if (rest) t += std::max(m.latency, (double)((rest + cus - 1) / cus));
+      t *= (double)(xb * seg) + m.startup;
+      t += steps * (m.planes * ((ny - 1) / nd[1] + (nz - 1) / nd[2]) + 8.0 * (nx - 1) / nd[0]);
+      if (best == 0.0 || t < best) {
+        best = t;
+        brick[0] = (int)xb;
+        brick[1] = (int)seg;
+      }
+    }
+}
+
+size_t brick_scratch_elems(int degree, const int *nc, const int *brick) { return (size_t)brick_grid(degree, nc, brick).total; }
 
 template <typename Number>
 int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,

@@ -26,6 +26,9 @@ __device__ __forceinline__ Number law_kappa(int law, const Number *p, Number T) 
   return p[0] + (p[1] - p[0]) * (Number(3) - Number(2) * fs) * fs * fs;
 }
 
+// the bricks of a Q1..Q3 mesh (heat_brick.hip): {pencils along x, steps along y}
+void choose_brick(int degree, const int *n_cells, int *brick);
+
 // Everything a level operator needs on the device (pointers are device memory).
 template <typename Number>
 struct OperatorData {
@@ -57,6 +60,7 @@ struct OperatorData {
   // columns meet, all zero between applies; Q1..Q3: the bricks' upper planes, written by every apply
   Number *edge = nullptr;
   size_t edge_elems = 0;
+  int brick[2] = {1, 1};  // Q1..Q3: pencils along x and steps along y of the apply's bricks
   void set_mesh(int k, const int *ncells, const double *ext) {
     degree = k;
     for (int d = 0; d < 3; ++d) {
@@ -67,6 +71,7 @@ struct OperatorData {
     }
     n_dofs = (long)nd[0] * nd[1] * nd[2];
     n_cells = (long)nc[0] * nc[1] * nc[2];
+    choose_brick(degree, nc, brick);
   }
 };
 
@@ -157,13 +162,13 @@ template <typename Number>
 int launch_apply(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                  hipEvent_t kernel_start = nullptr, hipEvent_t kernel_end = nullptr);
 // entries of OperatorData::edge the apply of a mesh of degree k and n_cells cells needs
-size_t apply_edge_elems(int degree, const int *n_cells, bool fp32);
+size_t apply_edge_elems(int degree, const int *n_cells, const int *brick, bool fp32);
 
 // heat_brick.hip: the apply for Q1..Q3 and the scratch entries (OperatorData::edge) it needs
 template <typename Number>
 int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                  hipEvent_t kernel_start, hipEvent_t kernel_end);
-size_t brick_scratch_elems(int degree, const int *n_cells);
+size_t brick_scratch_elems(int degree, const int *n_cells, const int *brick);
 // Q1..Q3, Cartesian cells: dst -= c_m M (a T + b T_old + c q) + K_k T in one pass (T_old is not read when
 // b = 0, q when null); constrained DoFs count as zero and are left alone, a conductivity law is evaluated at
 // T as given. dst must not overlap the inputs.
