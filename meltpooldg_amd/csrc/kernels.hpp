@@ -14,10 +14,51 @@ namespace mpdg {
 enum KappaMode { KAPPA_CONST = MPDG_KAPPA_CONST, KAPPA_QP = MPDG_KAPPA_QP, KAPPA_CELL = MPDG_KAPPA_CELL, KAPPA_LAW = MPDG_KAPPA_LAW };
 enum LawId { LAW_TANH = MPDG_LAW_TANH, LAW_MUSHY = MPDG_LAW_MUSHY };
 
+// tanh |x| = -E / (E + 2) with E = e^y - 1 = 2^n (e^r - 1) + (2^n - 1), y = -2 |x|, r = y - n ln 2 (ln 2 in two
+// parts, e^r - 1 by its Taylor series on |r| <= ln 2 / 2): small x keep their relative accuracy, and the
+// rounding errors of e^r - 1, E and E + 2 are carried into the quotient's correction. Largest error over 4M
+// arguments |x| <= 25, in units of 2^-53 (2^-24) of the result: 1.16 (FP32 1.4), the device library's 1.34
+// (2.33). The law is evaluated at every point of every apply, and the library's tanh and the division by
+// the width took a third to a half of it: Q2 64^3 FP64 92 -> 63 us, Q3 64^3 178 -> 131 us, FP32 unchanged.
+template <typename Number> struct TanhSeries;
+template <> struct TanhSeries<double> {
+  static constexpr int N = 12;
+  static constexpr double c[N] = {1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0, 1.0 / 3628800.0,
+                                  1.0 / 362880.0,     1.0 / 40320.0,     1.0 / 5040.0,     1.0 / 720.0,
+                                  1.0 / 120.0,        1.0 / 24.0,        1.0 / 6.0,        0.5};
+  static constexpr double log2e = 1.4426950408889634, ln2_hi = 0x1.62e42fefa3800p-1, ln2_lo = 0x1.ef35793c76730p-45;
+};
+template <> struct TanhSeries<float> {
+  static constexpr int N = 7;
+  static constexpr float c[N] = {1.0f / 40320.0f, 1.0f / 5040.0f, 1.0f / 720.0f, 1.0f / 120.0f, 1.0f / 24.0f, 1.0f / 6.0f, 0.5f};
+  static constexpr float log2e = 1.44269504f, ln2_hi = 0x1.62e400p-1f, ln2_lo = 0x1.7f7d1cp-20f;
+};
+__device__ __forceinline__ double reciprocal_estimate(double d) {
+  const double v = __builtin_amdgcn_rcp(d);
+  return fma(fma(-d, v, 1.0), v, v);
+}
+__device__ __forceinline__ float reciprocal_estimate(float d) { return __builtin_amdgcn_rcpf(d); }
+template <typename Number> __device__ __forceinline__ Number law_tanh(Number x) {
+  using C = TanhSeries<Number>;
+  constexpr bool carry = sizeof(Number) == 8;
+  const Number one = 1, y = -2 * fabs(x), n = rint(y * C::log2e);
+  const Number a = fma(n, -C::ln2_hi, y), r = fma(n, -C::ln2_lo, a), r2 = r * r;
+  Number q = C::c[0];
+#pragma unroll
+  for (int i = 1; i < C::N; ++i) q = fma(q, r, C::c[i]);
+  const Number p = fma(r2, q, r), p_lo = carry ? fma(r2, q, r - p) + fma(n, -C::ln2_lo, a - r) : Number(0);
+  const Number s = ldexp(one, (int)n), h = s - one, h_lo = s - (h + one);
+  const Number e = fma(s, p, h), e_lo = fma(s, p_lo, fma(s, p, h - e)) + h_lo;
+  const Number d = e + 2, d_lo = e - (d - 2), v = reciprocal_estimate(d), t = e * v;
+  const Number u = fma(fma(-(d_lo + e_lo), t, fma(-d, t, e)) + e_lo, v, t);
+  return copysign(y < -40 ? one : u, x);
+}
+
 template <typename Number>
 __device__ __forceinline__ Number law_kappa(int law, const Number *p, Number T) {
   if (law == LAW_TANH) {
-    return p[0] * (Number(1) + p[1] * tanh((T - p[2]) / p[3]));
+    const Number inv = Number(1) / p[3];
+    return p[0] * (Number(1) + p[1] * law_tanh((T - p[2]) * inv));
   }
   // mushy zone (liquid_solid): p = {k_liquid, k_solid, T_solidus, T_liquidus}
   const Number inv = Number(1) / (p[3] - p[2]);

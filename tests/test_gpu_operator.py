@@ -493,6 +493,29 @@ def test_residual_in_one_pass_agrees_with_its_parts(cuda, degree, nc, mode, dmas
     assert scale > 0 and float((one - parts).abs().max()) < 1e-12 * scale
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("degree", [1, 2, 3, 4])
+def test_law_of_one_temperature_is_a_constant_conductivity(cuda, degree, precision):
+    """k(T) = k0 (1 + a tanh((T - T0) / w)) from tiny to saturated arguments, against the same number as a
+    constant; the bound is the rounding of the interpolated T times its factor and of the sums."""
+    torch = cuda
+    import meltpooldg_amd as M
+    g = M.HeatDiffuseMultiPhaseOperator(degree, (5, 4, 3), (1.0, 0.8, 0.6), rho_cp=1.0, precision=precision)
+    dt = torch.float64 if precision == 0 else torch.float32
+    eps = float(torch.finfo(dt).eps)
+    g.reset_time_increment(1.0)
+    x = torch.rand(g.n_dofs, dtype=dt, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    y, ref = torch.empty_like(x), torch.empty_like(x)
+    for arg in (0.0, 1e-9, -3e-4, 0.17, -0.18, 0.5, -1.0, 2.5, -7.0, 18.9, -20.1, 1e6, -1e30):
+        w = 0.25
+        T = torch.full_like(x, arg * w)
+        g.set_conductivity_law(M.LAW_TANH, (2.0, 0.75, 0.0, w), T)
+        g.vmult(y, x)
+        g.set_conductivity_constant(2.0 * (1.0 + 0.75 * float(np.tanh(float(T[0]) / w))))
+        g.vmult(ref, x)
+        assert float((y - ref).abs().max()) <= 200 * eps * float(ref.abs().max()), arg
+
+
 def test_nonfinite_sources_stay_in_the_cells_that_hold_them(cuda):
     """A NaN in one DoF reaches the DoFs of the cells that hold it and no others (nothing of one cell is
     multiplied into another, as by the idle or paired lanes of a matrix instruction)."""
