@@ -400,18 +400,27 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
   // holds zeros.
   const long zoff = sz * (K * min(cz, P.nc[2] - 1) + min(l, K));
 
-  // constrained planes that touch the pencil at (cxb, cy): zero the DoFs on them
+  // constrained planes that touch the brick (a z plane would otherwise be tested for in every step of every
+  // brick: Q1 283 x 252 x 459 FP32 526 -> 443 us)
+  int bmask = P.dmask;
+  if (cx0 > 0) bmask &= ~1;
+  if (cx_end < P.nc[0]) bmask &= ~2;
+  if (cy0 > 0) bmask &= ~4;
+  if (cy_end < P.nc[1]) bmask &= ~8;
+  if (bz > 0) bmask &= ~16;
+  if (bz + 1 < P.g.nb[2]) bmask &= ~32;
+  // ... that touch the pencil at (cxb, cy): zero the DoFs on them
   auto constrain = [&](int cxb, int cy, auto &u) {
-    const auto &A = fresh_args<BrickArgs<Number, N1>>();
-    int m = A.dmask;
+    int m = bmask;
     if (m) {
       if (cxb > 0) m &= ~1;
-      if (cxb + kNX < A.nc[0]) m &= ~2;
+      if (cxb + kNX < fresh_args<BrickArgs<Number, N1>>().nc[0]) m &= ~2;
       if (cy > 0) m &= ~4;
-      if (cy + 1 < A.nc[1]) m &= ~8;
+      if (cy + 1 < fresh_args<BrickArgs<Number, N1>>().nc[1]) m &= ~8;
     }
     if (m) {
       const int cx = cxb + opaque(c), z = opaque(iz);
+      const auto &A = fresh_args<BrickArgs<Number, N1>>();
       const bool con_z = ((m & 16) && z == 0) || ((m & 32) && z == A.nd[2] - 1);
 #pragma unroll
       for (int j = 0; j < N1; ++j)
@@ -511,7 +520,7 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
 #pragma unroll
         for (int j = 0; j < N1; ++j)
 #pragma unroll
-          for (int i = 0; i < N1; ++i) kq[j][i] = p[N1 * j + i];
+          for (int i = 0; i < N1; ++i) kq[j][i] = N1 == 2 ? __builtin_nontemporal_load(p + N1 * j + i) : p[N1 * j + i];
       }
       if constexpr (KMODE == KAPPA_LAW && !LAW_OF_SRC) {
         Number a[N1][N1], t[N1][N1];
@@ -628,7 +637,7 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
           for (int j = 0; j < N1; ++j)
 #pragma unroll
             for (int i = 0; i < N1; ++i) kq[j][i] = law_kappa<Number>(P.law, P.law_p, v[j][i]);
-          if (A.dmask) {
+          if (bmask) {
             load_rows(src, cxb, cy, true, u);
             constrain(cxb, cy, u);
             to_points(u);
