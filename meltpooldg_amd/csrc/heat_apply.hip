@@ -725,11 +725,12 @@ size_t edge_elems_shape(const int *nc) {
   const long ny = (nc[1] + G::BY - 1) / G::BY, nz = (nc[2] + G::BZ - 1) / G::BZ;
   return (size_t)((ny - 1) * (nz - 1) * ((long)(N1 - 1) * nc[0] + 1));
 }
-size_t apply_edge_elems(int degree, const int *nc, const int *brick, bool fp32) {
-  if (degree >= 1 && degree <= 3) return brick_scratch_elems(degree, nc, brick);
-  if (degree != 4) return 0;
-  return fp32 ? edge_elems_shape<5, float, false>(nc) : edge_elems_shape<5, double, false>(nc);
+template <typename Number> size_t apply_edge_elems(const OperatorData<Number> &op) {
+  if (op.degree >= 1 && op.degree <= 3) return brick_scratch_elems(op.degree, op.nc, op.brick, op.brick_cells);
+  return op.degree == 4 ? edge_elems_shape<5, Number, false>(op.nc) : 0;
 }
+template size_t apply_edge_elems<double>(const OperatorData<double> &);
+template size_t apply_edge_elems<float>(const OperatorData<float> &);
 
 // LDS beyond 64 KiB per workgroup has to be allowed per kernel before its first launch
 template <int N1, typename Number, int KMODE, bool MAPPED>

@@ -56,11 +56,13 @@ struct BrickGrid {
   long total;      // scratch entries
 };
 constexpr int kMaxSteps = 16, kMaxPencils = 2;
+constexpr int kCellsZ = 4;  // cells along z of a wavefront with one cell per lane
 
-constexpr int zc_of(int k) { return k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC; }
-BrickGrid brick_grid(int k, const int *nc, const int *brick) {
+constexpr int zc_of(int k, bool cells) { return cells ? kCellsZ : k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC; }
+// cells: of the kernel with one cell per lane
+BrickGrid brick_grid(int k, const int *nc, const int *brick, bool cells) {
   BrickGrid g;
-  const int zc = zc_of(k), px = (nc[0] + kNX - 1) / kNX;
+  const int zc = zc_of(k, cells), px = (nc[0] + kNX - 1) / kNX;
   g.cells[0] = kNX * brick[0];
   g.cells[1] = brick[1];
   g.cells[2] = zc;
@@ -943,6 +945,252 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
   }
 }
 
+// ---- the apply of Q1 and Q2 on Cartesian cells: one lane per cell ----
+
+// sweep of a cell's values [z][y][x] along direction DIR (0 x, 1 y, 2 z)
+template <int N1, int DIR, bool TR, bool ADD, typename Number, typename Mat>
+__device__ __forceinline__ void sweep_cell(const Mat &M, const Number (&in)[N1][N1][N1], Number (&out)[N1][N1][N1]) {
+#pragma unroll
+  for (int a = 0; a < N1; ++a)
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+      auto at = [&](auto &v, int t) -> auto & { return DIR == 0 ? v[a][b][t] : (DIR == 1 ? v[a][t][b] : v[t][a][b]); };
+#pragma unroll
+      for (int q = 0; q < N1; ++q) {
+        Number s = ADD ? at(out, q) : Number(0);
+#pragma unroll
+        for (int t = 0; t < N1; ++t) s = fma(TR ? M(t, q) : M(q, t), at(in, t), s);
+        at(out, q) = s;
+      }
+    }
+}
+// f(z, y, x) for every value or point of a cell
+template <int N1, typename F> __device__ __forceinline__ void for_cell(F f) {
+#pragma unroll
+  for (int l = 0; l < N1; ++l)
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) f(l, j, i);
+}
+// values at the points of the field in u (u is overwritten)
+template <int N1, typename Number, typename Mat>
+__device__ __forceinline__ void cell_to_points(const Mat &S, Number (&u)[N1][N1][N1], Number (&v)[N1][N1][N1]) {
+  sweep_cell<N1, 0, false, false>(S, u, v);
+  sweep_cell<N1, 1, false, false>(S, v, u);
+  sweep_cell<N1, 2, false, false>(S, u, v);
+}
+// e += D^T (k * (D v)) along DIR
+template <int N1, int DIR, typename Number, typename Mat, typename MatT>
+__device__ __forceinline__ void flux_cell(const Mat &D, const MatT &Dt, const Number (&v)[N1][N1][N1], const Number (&k)[N1][N1][N1],
+                                          Number (&e)[N1][N1][N1]) {
+#pragma unroll
+  for (int a = 0; a < N1; ++a)
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+      auto at = [&](auto &x, int t) -> auto & { return DIR == 0 ? x[a][b][t] : (DIR == 1 ? x[a][t][b] : x[t][a][b]); };
+      Number f[N1];
+#pragma unroll
+      for (int q = 0; q < N1; ++q) {
+        Number g = 0;
+#pragma unroll
+        for (int t = 0; t < N1; ++t) g = fma(D(q, t), at(v, t), g);
+        f[q] = at(k, q) * g;
+      }
+#pragma unroll
+      for (int t = 0; t < N1; ++t)
+#pragma unroll
+        for (int q = 0; q < N1; ++q) at(e, t) = fma(Dt(q, t), f[q], at(e, t));
+    }
+}
+// value of the lane 16 below (the cell below in z)
+__device__ __forceinline__ double from_cell_below(double x, int lane) {
+  const int lo = __builtin_amdgcn_ds_bpermute(4 * (lane - 16), __double2loint(x));
+  const int hi = __builtin_amdgcn_ds_bpermute(4 * (lane - 16), __double2hiint(x));
+  return __hiloint2double(hi, lo);
+}
+
+// A whole cell per lane: a wavefront (= workgroup) holds 16 x 4 cells (x, z) and marches along y, pencils of
+// 16 cells side by side along x done one after the other. All sweeps are register-local: per 64 cells Q2
+// takes half the VALU instructions of the kernel above, whose lane rows hold four planes, and there is no
+// barrier. What bounds it: the VALU, at two or three wavefronts per SIMD (Q2 FP64: 230 registers). Against the
+// kernel above with these degrees: Q2 100^3 k per point FP64 178 -> 140 us, FP32 126 -> 79 us (101 us for a
+// kernel with LDS transposes between the sweeps), with a law FP32 196 -> 118 us (136), Q2 64^3 one k per cell
+// FP32 29 -> 24 us, Q1 112 x 116 x 132 k per point FP32 47 -> 33 us (40). Mapped cells, the residual and the
+// tangent have more values per point than fit (Q2 FP64: tangent of 70 x 50 x 33 47 -> 123 us, mapped
+// 100 x 80 x 70 289 -> 316 us, residual with a law 80 us both) and stay above, as does Q3.
+template <int N1, typename Number, int KMODE>
+__global__ __launch_bounds__(64) void heat_cells_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__ src,
+                                                        Number *__restrict__ dst) {
+  constexpr int K = N1 - 1, NQ = N1 * N1 * N1;
+  constexpr bool TENSOR = KMODE == KAPPA_CONST || KMODE == KAPPA_CELL;
+  __shared__ double yrow[kMaxPencils][N1 * N1][64];  // top rows of the previous y step's cells
+  __shared__ double xcol[N1 * N1][kCellsZ];          // last x column of the previous pencil
+  const int lane = threadIdx.x, c = lane & 15, zc = lane >> 4;
+  const int nbr = gridDim.x, xcd = blockIdx.x & 7;
+  int b = xcd * (nbr >> 3) + min(xcd, nbr & 7) + (blockIdx.x >> 3);
+  const int bx = b % P.g.nb[0];
+  b /= P.g.nb[0];
+  const int by = b % P.g.nb[1], bz = b / P.g.nb[1];
+  const int cz = bz * kCellsZ + zc, cy0 = by * P.g.cells[1], cx0 = bx * P.g.cells[0];
+  const int cy_end = min(cy0 + P.g.cells[1], P.nc[1]), cx_end = min(cx0 + P.g.cells[0], P.nc[0]);
+  const long sy = P.nd[0], sz = (long)P.nd[0] * P.nd[1];
+  // lanes without a cell work on the mesh's last one: sums pass upwards in x and z only
+  const int czc = min(cz, P.nc[2] - 1);
+  // constrained planes that touch the brick
+  int bmask = P.dmask;
+  if (cx0 > 0) bmask &= ~1;
+  if (cx_end < P.nc[0]) bmask &= ~2;
+  if (cy0 > 0) bmask &= ~4;
+  if (cy_end < P.nc[1]) bmask &= ~8;
+  if (bz > 0) bmask &= ~16;
+  if (bz + 1 < P.g.nb[2]) bmask &= ~32;
+  // ... that touch the cell: zero plane l's DoFs on them
+  auto constrain_plane = [&](int cx, int cy, int l, auto &u) {
+    int m = bmask;
+    if (cx > 0) m &= ~1;
+    if (cx + 1 < P.nc[0]) m &= ~2;
+    if (cy > 0) m &= ~4;
+    if (cy + 1 < P.nc[1]) m &= ~8;
+    if (cz > 0) m &= ~16;
+    if (cz + 1 < P.nc[2]) m &= ~32;
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        const int faces = (i == 0 ? 1 : 0) | (i == K ? 2 : 0) | (j == 0 ? 4 : 0) | (j == K ? 8 : 0) | (l == 0 ? 16 : 0) |
+                          (l == K ? 32 : 0);
+        if (m & faces) u[j][i] = 0;
+      }
+  };
+  auto constrain = [&](int cx, int cy, Number (&u)[N1][N1][N1]) {
+    if (bmask) {
+#pragma unroll
+      for (int l = 0; l < N1; ++l) constrain_plane(cx, cy, l, u[l]);
+    }
+  };
+  auto cell_dofs = [&](const Number *field, int cx, int cy) {
+    return field + sz * ((long)K * czc) + sy * ((long)K * cy) + K * min(cx, P.nc[0] - 1);
+  };
+  auto load = [&](const Number *field, int cx, int cy, Number (&u)[N1][N1][N1]) {
+    const Number *p = cell_dofs(field, cx, cy);
+    for_cell<N1>([&](int l, int j, int i) { u[l][j][i] = p[sz * l + sy * j + i]; });
+  };
+  auto half = [](int a) { return a < N1 - 1 - a ? a : N1 - 1 - a; };
+  for (int cy = cy0; cy < cy_end; ++cy) {
+    const bool last = cy + 1 == cy_end;
+    int pen = 0;
+    for (int cxb = cx0; cxb < cx_end; cxb += kNX, ++pen) {
+      const int cx = cxb + c;
+      const long cell = min(cx, P.nc[0] - 1) + (long)P.nc[0] * (cy + (long)P.nc[1] * czc);
+      Number u[N1][N1][N1], v[N1][N1][N1];
+      load(src, cx, cy, u);
+      constrain(cx, cy, u);
+      if constexpr (TENSOR) {
+        // a conductivity that is constant on a Cartesian cell:
+        // J u = M_x [M_y (c_m M_z + k k_z K_z) + k k_y K_y M_z] u + k k_x K_x M_y M_z u
+        const Number kc = KMODE == KAPPA_CELL ? P.kappa_arr[cell] : P.kappa;
+        const Number kx = kc * P.kx, ky = kc * P.ky, kz = kc * P.kz;
+        Number m[N1][N1][N1], p[N1][N1][N1];
+        sweep_cell<N1, 2, false, false>(P.K1, u, p);
+        sweep_cell<N1, 2, false, false>(P.M1, u, m);
+        for_cell<N1>([&](int l, int j, int i) { p[l][j][i] = fma(P.cm, m[l][j][i], kz * p[l][j][i]); });
+        sweep_cell<N1, 1, false, false>(P.M1, m, u);
+        sweep_cell<N1, 1, false, false>(P.M1, p, v);
+        for_cell<N1>([&](int l, int j, int i) {
+          m[l][j][i] *= ky;
+          u[l][j][i] *= kx;
+        });
+        sweep_cell<N1, 1, false, true>(P.K1, m, v);
+        sweep_cell<N1, 0, false, false>(P.M1, v, m);
+        sweep_cell<N1, 0, false, true>(P.K1, u, m);
+        for_cell<N1>([&](int l, int j, int i) { v[l][j][i] = m[l][j][i]; });
+      } else {
+        Number e[N1][N1][N1], k[N1][N1][N1];
+        if constexpr (KMODE == KAPPA_LAW) {
+          load(P.T, cx, cy, k);
+          cell_to_points<N1>(P.S, k, v);
+          for_cell<N1>([&](int l, int j, int i) { k[l][j][i] = law_kappa<Number>(P.law, P.law_p, v[l][j][i]); });
+        } else {
+          const Number *p = P.kappa_arr + cell * NQ;
+          for_cell<N1>([&](int l, int j, int i) { k[l][j][i] = p[(N1 * l + j) * N1 + i]; });
+        }
+        cell_to_points<N1>(P.S, u, v);
+        // at the points (heat_diffuse_operator.cpp:1029-1077): e = c_m W v + D^T f
+        for_cell<N1>([&](int l, int j, int i) {
+          const Number w = (P.w[half(l)] * P.w[half(j)]) * P.w[half(i)];
+          k[l][j][i] *= w * P.kx;
+          e[l][j][i] = (w * P.cm) * v[l][j][i];
+        });
+        flux_cell<N1, 0>(P.D, P.D, v, k, e);
+        flux_cell<N1, 1>(P.D, P.Dy, v, k, e);
+        flux_cell<N1, 2>(P.D, P.Gz, v, k, e);  // (Gz: here the collocation derivative times k_z / k_x)
+        sweep_cell<N1, 2, true, false>(P.S, e, u);
+        sweep_cell<N1, 1, true, false>(P.S, u, e);
+        sweep_cell<N1, 0, true, false>(P.S, e, v);
+      }
+      // ---- per plane, from the top: sums over the brick's cells (along y through LDS, along x to the next
+      //      lane, along z to the lane 16 above), then the stores: to dst, or to the classes of the brick's
+      //      upper planes ----
+      const bool more = cxb + kNX < cx_end, hy = last && cy_end != P.nc[1], hx = cx_end != P.nc[0];
+      const bool on = cx < P.nc[0] && cz < P.nc[2], end_z = cz == P.nc[2] - 1, end_x = cx == cx_end - 1;
+      const long ny1 = P.g.nb[1] - 1, nz1 = P.g.nb[2] - 1;
+      double up[N1][N1];
+#pragma unroll
+      for (int l = K; l >= 0; --l) {
+        double r[N1][N1];
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) r[j][i] = (double)v[l][j][i];
+        if (cy > cy0) {
+#pragma unroll
+          for (int i = 0; i < N1; ++i) r[0][i] += yrow[pen][N1 * l + i][lane];
+        }
+        if (!last) {
+#pragma unroll
+          for (int i = 0; i < N1; ++i) yrow[pen][N1 * l + i][lane] = r[K][i];
+        }
+#pragma unroll
+        for (int j = 0; j < N1; ++j) {
+          if (j == K && !last) continue;
+          r[j][0] += from_previous_cell(r[j][K], pen > 0 ? xcol[N1 * l + j][zc] : 0.0);
+          if (more && c == kNX - 1) xcol[N1 * l + j][zc] = r[j][K];
+#pragma unroll
+          for (int i = 0; i < N1; ++i) {
+            if (l == K) up[j][i] = from_cell_below(r[j][i], lane);
+            if (l == 0) r[j][i] += zc > 0 ? up[j][i] : 0.0;
+          }
+        }
+        if (bmask) constrain_plane(cx, cy, l, r);
+        if (!on || (l == K && !end_z && zc != kCellsZ - 1)) continue;
+        const bool hz = l == K && !end_z;
+        const int iz = K * cz + l;
+#pragma unroll
+        for (int j = 0; j < N1; ++j) {
+          if (j == K && !last) continue;
+          const bool y = j == K && hy;
+          const int iy = K * cy + j;
+          Number *o = (hz ? P.scratch + P.g.off[4] + bz * sz : dst + sz * iz) + sy * iy;
+          if (y) o = P.scratch + (hz ? P.g.off[6] + (by + ny1 * bz) * sy : P.g.off[2] + (by + ny1 * iz) * sy);
+          o += K * cx;
+#pragma unroll
+          for (int i = 0; i < K; ++i) o[i] = (Number)r[j][i];
+          if (end_x) {
+            o += K;
+            if (hx) {
+              if (y) o = P.scratch + (hz ? P.g.off[7] + (bx * ny1 + by) * nz1 + bz : P.g.off[3] + (bx * ny1 + by) * P.nd[2] + iz);
+              else o = P.scratch + (hz ? P.g.off[5] + (bx * nz1 + bz) * P.nd[1] + iy : P.g.off[1] + ((long)bx * P.nd[2] + iz) * P.nd[1] + iy);
+            }
+            *o = (Number)r[j][K];
+          }
+        }
+      }
+      if (more) lds_fence();  // (xcol: other lanes read it)
+    }
+  }
+}
+
 // dst += the classes of the planes bricks share, in class order (sums in FP64). A wavefront takes up
 // to 64 kFixup DoFs of a line: of an x row of the shared z planes, then of the shared y planes (rows
 // off the z planes), then of a y line of the shared x planes (off both). All its loads are issued
@@ -1147,9 +1395,10 @@ void tangent_points_kernel(const TangentPoints<N1> X, const double *__restrict__
     }
 }
 
-// unit: the data per point carries the volume and the 1/h (mapped cells, the tangent)
+// unit: the data per point carries the volume and 1/h (mapped cells, the tangent); cells: for the kernel with
+// one cell per lane
 template <int N1, typename Number>
-int fill_brick_args(const OperatorData<Number> &op, bool unit, BrickArgs<Number, N1> &A) {
+int fill_brick_args(const OperatorData<Number> &op, bool unit, BrickArgs<Number, N1> &A, bool cells = false) {
   const FE1D &fe = fe1d(N1 - 1);
   const double vol = unit ? 1.0 : op.h[0] * op.h[1] * op.h[2];
   double Dy[kMaxN1][kMaxN1], Gz[kMaxN1][kMaxN1], M1[kMaxN1][kMaxN1] = {}, K1[kMaxN1][kMaxN1] = {};
@@ -1158,7 +1407,7 @@ int fill_brick_args(const OperatorData<Number> &op, bool unit, BrickArgs<Number,
   for (int q = 0; q < N1; ++q)
     for (int i = 0; i < N1; ++i) {
       Dy[q][i] = fe.D[q][i] * ry;
-      Gz[q][i] = fe.G[q][i] * rz;
+      Gz[q][i] = (cells ? fe.D : fe.G)[q][i] * rz;
       for (int j = 0; j < N1; ++j) {
         M1[i][j] += fe.S[q][i] * fe.qw[q] * fe.S[q][j];
         K1[i][j] += fe.G[q][i] * fe.qw[q] * fe.G[q][j];
@@ -1177,7 +1426,7 @@ int fill_brick_args(const OperatorData<Number> &op, bool unit, BrickArgs<Number,
     A.nd[d] = op.nd[d];
   }
   A.n_cells = op.n_cells;
-  A.g = brick_grid(N1 - 1, op.nc, op.brick);
+  A.g = brick_grid(N1 - 1, op.nc, cells ? op.brick_cells : op.brick, cells);
   A.dmask = op.dmask;
   A.law = op.law;
   A.cm = (Number)(op.c_mass * vol);
@@ -1213,11 +1462,20 @@ template <int N1, typename Number> dim3 brick_blocks(const BrickArgs<Number, N1>
 #define MPDG_BRICK(KM, MP, RES_) \
   hipLaunchKernelGGL((heat_brick_kernel<N1, Number, KM, MP, RES_>), brick_blocks(A), dim3(64 * kNW), 0, stream, A, src, dst)
 
+#define MPDG_APPLY(KM)                                                                                                 \
+  do {                                                                                                                 \
+    if constexpr (N1 < 4)                                                                                              \
+      hipLaunchKernelGGL((heat_cells_kernel<N1, Number, KM>), brick_blocks(A), dim3(64), 0, stream, A, src, dst);      \
+    else                                                                                                               \
+      MPDG_BRICK(KM, false, false);                                                                                    \
+  } while (0)
+
 template <int N1, typename Number>
 int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                     hipEvent_t kernel_start, hipEvent_t kernel_end) {
   BrickArgs<Number, N1> A;
-  if (const int rc = fill_brick_args(op, op.metric != nullptr, A)) return rc;
+  const bool cells = N1 < 4 && !op.metric;
+  if (const int rc = fill_brick_args(op, op.metric != nullptr, A, cells)) return rc;
   if (kernel_start) (void)hipEventRecord(kernel_start, stream);
   if (op.metric) {
     switch (op.kappa_mode) {
@@ -1227,10 +1485,10 @@ int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *d
     }
   } else {
     switch (op.kappa_mode) {
-      case KAPPA_CONST: MPDG_BRICK(KAPPA_CONST, false, false); break;
-      case KAPPA_QP: MPDG_BRICK(KAPPA_QP, false, false); break;
-      case KAPPA_CELL: MPDG_BRICK(KAPPA_CELL, false, false); break;
-      case KAPPA_LAW: MPDG_BRICK(KAPPA_LAW, false, false); break;
+      case KAPPA_CONST: MPDG_APPLY(KAPPA_CONST); break;
+      case KAPPA_QP: MPDG_APPLY(KAPPA_QP); break;
+      case KAPPA_CELL: MPDG_APPLY(KAPPA_CELL); break;
+      case KAPPA_LAW: MPDG_APPLY(KAPPA_LAW); break;
       default: return MPDG_ERR_INVALID;
     }
   }
@@ -1296,6 +1554,7 @@ int launch_brick_tangent_n1(const OperatorData<double> &op, const double *td, co
   }
   return finish_brick(A, dst, stream);
 }
+#undef MPDG_APPLY
 #undef MPDG_BRICK
 
 template <int N1>
@@ -1328,19 +1587,17 @@ int launch_brick_tangent_data_n1(const OperatorData<double> &op, double dt, cons
 
 // Long bricks share fewer planes and set their tables up less often; short ones give every CU work, and end
 // the launch evenly. Taken is the shape with the least modelled time, in steps of one CU: full rounds of the
-// workgroups that are resident at once (4 per CU, Q1: 6), the rest (no faster than the latency of one
-// workgroup, which shows below 2.5 per CU), start-up, and the sums of the shared planes (the x planes'
-// strided, 8 times the others'). Measured over 28 meshes and kernels: 1.6% above the best shape on average
-// (at most 15%); about 2048 workgroups for every mesh: 5.7% (24%) (Q2 48 x 80 x 56 FP64 35.6 -> 28.7 us, Q2 70 x 50 x 33
-// 25.7 -> 22.6, Q3 75 x 62 x 49 FP32 49.6 -> 45.4, Q1 200 x 150 x 170 97.5 -> 88.5, Q2 64^3 and Q3 128^3 the
-// same shapes). It depends on the mesh only, so every apply of a mesh sums in the same order.
-void choose_brick(int k, const int *nc, int *brick) {
-  brick[0] = brick[1] = 1;
-  if (k > 3) return;
-  struct { double resident, latency, startup, planes; } static const model[4] = {
-      {}, {6, 4, 0.2, 1.0}, {4, 2.5, 0.7, 0.0}, {4, 2.5, 0.2, 0.5}};
-  const auto &m = model[k];
-  const long zc = zc_of(k), px = (nc[0] + kNX - 1) / kNX, nz = (nc[2] + zc - 1) / zc, cus = 256;
+// workgroups that are resident at once, the rest (no faster than the latency of one workgroup, which shows
+// below `latency` per CU), start-up, and the sums of the shared planes (of the x planes, which are strided,
+// separately). Measured over 28 meshes and kernels: 1.6% above the best shape on average (at most 15%); about
+// 2048 workgroups for every mesh: 5.7% (24%) (Q3 75 x 62 x 49 FP32 49.6 -> 45.4 us, mapped Q3 96^3 FP64
+// 809 -> 781 us, Q2 and Q3 64^3 and 128^3 the same shapes); one cell per lane: 24 meshes, 2.5% (9%). It depends
+// on the mesh only, so every apply of a mesh sums in the same order.
+struct BrickModel {
+  double resident, latency, startup, planes, x_planes;
+};
+static void least_time(const BrickModel &m, int k, const int *nc, int zc, int *brick) {
+  const long px = (nc[0] + kNX - 1) / kNX, nz = (nc[2] + zc - 1) / zc, cus = 256;
   const double nd[3] = {k * (double)nc[0] + 1, k * (double)nc[1] + 1, k * (double)nc[2] + 1};
   const double steps = (double)px * nc[1] * nz / cus;
   double best = 0.0;
@@ -1351,7 +1608,7 @@ void choose_brick(int k, const int *nc, int *brick) {
       double t = (double)(n / round) * m.resident;
       if (rest) t += std::max(m.latency, (double)((rest + cus - 1) / cus));
       t *= (double)(xb * seg) + m.startup;
-      t += steps * (m.planes * ((ny - 1) / nd[1] + (nz - 1) / nd[2]) + 8.0 * (nx - 1) / nd[0]);
+      t += steps * (m.planes * ((ny - 1) / nd[1] + (nz - 1) / nd[2]) + m.x_planes * (nx - 1) / nd[0]);
       if (best == 0.0 || t < best) {
         best = t;
         brick[0] = (int)xb;
@@ -1359,8 +1616,18 @@ void choose_brick(int k, const int *nc, int *brick) {
       }
     }
 }
+void choose_brick(int k, const int *nc, int *brick, int *brick_cells) {
+  static const BrickModel bricks[4] = {{}, {6, 4, 0.2, 1.0, 8}, {4, 2.5, 0.7, 0.0, 8}, {4, 2.5, 0.2, 0.5, 8}};
+  static const BrickModel cells = {12, 12, 0.2, 0.5, 1};
+  if (k > 3) return;
+  least_time(bricks[k], k, nc, zc_of(k, false), brick);
+  if (k < 3) least_time(cells, k, nc, zc_of(k, true), brick_cells);
+}
 
-size_t brick_scratch_elems(int degree, const int *nc, const int *brick) { return (size_t)brick_grid(degree, nc, brick).total; }
+size_t brick_scratch_elems(int degree, const int *nc, const int *brick, const int *brick_cells) {
+  const size_t n = brick_grid(degree, nc, brick, false).total;
+  return degree < 3 ? std::max(n, (size_t)brick_grid(degree, nc, brick_cells, true).total) : n;
+}
 
 template <typename Number>
 int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,

@@ -22,7 +22,7 @@ inline int dev_ok() { return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ER
 // operator
 // ===========================================================================
 int mpdg_heat_op::ensure_edge() const {
-  const size_t n = apply_edge_elems(d64.degree, d64.nc, d64.brick, precision == MPDG_FP32);
+  const size_t n = precision == MPDG_FP32 ? apply_edge_elems(d32) : apply_edge_elems(d64);
   if (precision == MPDG_FP64) {
     MPDG_TRY(d64.degree < 4 ? edge64.resize(n) : edge64.resize_zeroed(n));
     d64.edge = edge64.get();
@@ -497,7 +497,7 @@ struct GMGPrecond : mpdg_precond {
       MPDG_TRY(L.t2.resize(t2));
     }
     for (auto &L : lev) {
-      const size_t ne = apply_edge_elems(L->od.degree, L->od.nc, L->od.brick, std::is_same<T, float>::value);
+      const size_t ne = apply_edge_elems(L->od);
       MPDG_TRY(L->edge.resize_zeroed(ne));
       L->od.edge = L->edge.get();
       L->od.edge_elems = ne;
@@ -1386,12 +1386,12 @@ int mpdg_heat_op_vmult_noalloc(const mpdg_heat_op *op, double *dst, const double
       return MPDG_ERR_TOO_LARGE;
     if (op->d64.degree < 4) {
       // the operator's scratch, allocated when it was created
-      if (op->d64.edge_elems != apply_edge_elems(op->d64.degree, op->d64.nc, op->d64.brick, false)) return MPDG_ERR_NOMEM;
+      if (op->d64.edge_elems != apply_edge_elems(op->d64)) return MPDG_ERR_NOMEM;
       MPDG_TRY(launch_apply<double>(op->d64, src, dst, s));
       if (op->d64.robin_mask) MPDG_TRY(launch_boundary(op->d64, 0, nullptr, dst, src, op->T_robin, s));
       return MPDG_OK;
     }
-    const size_t need = apply_edge_elems(op->d64.degree, op->d64.nc, op->d64.brick, false);
+    const size_t need = apply_edge_elems(op->d64);
     double *scr = nullptr;
     MPDG_TRY(scratch_address(&scr));
     OperatorData<double> od = op->d64;

@@ -67,8 +67,9 @@ __device__ __forceinline__ Number law_kappa(int law, const Number *p, Number T) 
   return p[0] + (p[1] - p[0]) * (Number(3) - Number(2) * fs) * fs * fs;
 }
 
-// the bricks of a Q1..Q3 mesh (heat_brick.hip): {pencils along x, steps along y}
-void choose_brick(int degree, const int *n_cells, int *brick);
+// the bricks of a Q1..Q3 mesh (heat_brick.hip): {pencils along x, steps along y}, and those of the kernel with
+// one cell per lane
+void choose_brick(int degree, const int *n_cells, int *brick, int *brick_cells);
 
 // Everything a level operator needs on the device (pointers are device memory).
 template <typename Number>
@@ -101,7 +102,7 @@ struct OperatorData {
   // columns meet, all zero between applies; Q1..Q3: the bricks' upper planes, written by every apply
   Number *edge = nullptr;
   size_t edge_elems = 0;
-  int brick[2] = {1, 1};  // Q1..Q3: pencils along x and steps along y of the apply's bricks
+  int brick[2] = {1, 1}, brick_cells[2] = {1, 1};  // Q1..Q3: choose_brick
   void set_mesh(int k, const int *ncells, const double *ext) {
     degree = k;
     for (int d = 0; d < 3; ++d) {
@@ -112,7 +113,7 @@ struct OperatorData {
     }
     n_dofs = (long)nd[0] * nd[1] * nd[2];
     n_cells = (long)nc[0] * nc[1] * nc[2];
-    choose_brick(degree, nc, brick);
+    choose_brick(degree, nc, brick, brick_cells);
   }
 };
 
@@ -203,13 +204,13 @@ template <typename Number>
 int launch_apply(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                  hipEvent_t kernel_start = nullptr, hipEvent_t kernel_end = nullptr);
 // entries of OperatorData::edge the apply of a mesh of degree k and n_cells cells needs
-size_t apply_edge_elems(int degree, const int *n_cells, const int *brick, bool fp32);
+template <typename Number> size_t apply_edge_elems(const OperatorData<Number> &op);
 
 // heat_brick.hip: the apply for Q1..Q3 and the scratch entries (OperatorData::edge) it needs
 template <typename Number>
 int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
                  hipEvent_t kernel_start, hipEvent_t kernel_end);
-size_t brick_scratch_elems(int degree, const int *n_cells, const int *brick);
+size_t brick_scratch_elems(int degree, const int *n_cells, const int *brick, const int *brick_cells);
 // Q1..Q3, Cartesian cells: dst -= c_m M (a T + b T_old + c q) + K_k T in one pass (T_old is not read when
 // b = 0, q when null); constrained DoFs count as zero and are left alone, a conductivity law is evaluated at
 // T as given. dst must not overlap the inputs.
