@@ -56,14 +56,13 @@ struct BrickGrid {
   long total;      // scratch entries
 };
 constexpr int kMaxSteps = 16, kMaxPencils = 2;
-constexpr int kCellsZ = 4;  // cells along z of a wavefront with one cell per lane
 
-constexpr int zc_of(int k, bool cells) { return cells ? kCellsZ : k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC; }
-// cells: of the kernel with one cell per lane
+constexpr int zc_of(int k) { return k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC; }
+// brick: {pencils along x, steps along y, cells of a pencil}, the last for the kernel with one cell per lane
 BrickGrid brick_grid(int k, const int *nc, const int *brick, bool cells) {
   BrickGrid g;
-  const int zc = zc_of(k, cells), px = (nc[0] + kNX - 1) / kNX;
-  g.cells[0] = kNX * brick[0];
+  const int lx = cells ? brick[2] : kNX, zc = cells ? 64 / lx : zc_of(k), px = (nc[0] + lx - 1) / lx;
+  g.cells[0] = lx * brick[0];
   g.cells[1] = brick[1];
   g.cells[2] = zc;
   g.nb[0] = (px + brick[0] - 1) / brick[0];
@@ -1003,15 +1002,15 @@ __device__ __forceinline__ void flux_cell(const Mat &D, const MatT &Dt, const Nu
         for (int q = 0; q < N1; ++q) at(e, t) = fma(Dt(q, t), f[q], at(e, t));
     }
 }
-// value of the lane 16 below (the cell below in z)
-__device__ __forceinline__ double from_cell_below(double x, int lane) {
-  const int lo = __builtin_amdgcn_ds_bpermute(4 * (lane - 16), __double2loint(x));
-  const int hi = __builtin_amdgcn_ds_bpermute(4 * (lane - 16), __double2hiint(x));
+// value of a lower lane (the cell below in z)
+__device__ __forceinline__ double from_lane(double x, int lane) {
+  const int lo = __builtin_amdgcn_ds_bpermute(4 * lane, __double2loint(x));
+  const int hi = __builtin_amdgcn_ds_bpermute(4 * lane, __double2hiint(x));
   return __hiloint2double(hi, lo);
 }
 
-// A whole cell per lane: a wavefront (= workgroup) holds 16 x 4 cells (x, z) and marches along y, pencils of
-// 16 cells side by side along x done one after the other. All sweeps are register-local: per 64 cells Q2
+// A whole cell per lane: a wavefront (= workgroup) holds LX x 64 / LX cells (x, z) and marches along y, pencils of
+// LX cells side by side along x done one after the other. All sweeps are register-local: per 64 cells Q2
 // takes half the VALU instructions of the kernel above, whose lane rows hold four planes, and there is no
 // barrier. What bounds it: the VALU, at two or three wavefronts per SIMD (Q2 FP64: 230 registers). Against the
 // kernel above with these degrees: Q2 100^3 k per point FP64 178 -> 140 us, FP32 126 -> 79 us (101 us for a
@@ -1019,20 +1018,20 @@ __device__ __forceinline__ double from_cell_below(double x, int lane) {
 // FP32 29 -> 24 us, Q1 112 x 116 x 132 k per point FP32 47 -> 33 us (40). Mapped cells, the residual and the
 // tangent have more values per point than fit (Q2 FP64: tangent of 70 x 50 x 33 47 -> 123 us, mapped
 // 100 x 80 x 70 289 -> 316 us, residual with a law 80 us both) and stay above, as does Q3.
-template <int N1, typename Number, int KMODE>
+template <int N1, typename Number, int KMODE, int LX>
 __global__ __launch_bounds__(64) void heat_cells_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__ src,
                                                         Number *__restrict__ dst) {
-  constexpr int K = N1 - 1, NQ = N1 * N1 * N1;
+  constexpr int K = N1 - 1, NQ = N1 * N1 * N1, LZ = 64 / LX;
   constexpr bool TENSOR = KMODE == KAPPA_CONST || KMODE == KAPPA_CELL;
   __shared__ double yrow[kMaxPencils][N1 * N1][64];  // top rows of the previous y step's cells
-  __shared__ double xcol[N1 * N1][kCellsZ];          // last x column of the previous pencil
-  const int lane = threadIdx.x, c = lane & 15, zc = lane >> 4;
+  __shared__ double xcol[N1 * N1][LZ];          // last x column of the previous pencil
+  const int lane = threadIdx.x, c = lane % LX, zc = lane / LX;
   const int nbr = gridDim.x, xcd = blockIdx.x & 7;
   int b = xcd * (nbr >> 3) + min(xcd, nbr & 7) + (blockIdx.x >> 3);
   const int bx = b % P.g.nb[0];
   b /= P.g.nb[0];
   const int by = b % P.g.nb[1], bz = b / P.g.nb[1];
-  const int cz = bz * kCellsZ + zc, cy0 = by * P.g.cells[1], cx0 = bx * P.g.cells[0];
+  const int cz = bz * LZ + zc, cy0 = by * P.g.cells[1], cx0 = bx * P.g.cells[0];
   const int cy_end = min(cy0 + P.g.cells[1], P.nc[1]), cx_end = min(cx0 + P.g.cells[0], P.nc[0]);
   const long sy = P.nd[0], sz = (long)P.nd[0] * P.nd[1];
   // lanes without a cell work on the mesh's last one: sums pass upwards in x and z only
@@ -1080,7 +1079,7 @@ __global__ __launch_bounds__(64) void heat_cells_kernel(const BrickArgs<Number, 
   for (int cy = cy0; cy < cy_end; ++cy) {
     const bool last = cy + 1 == cy_end;
     int pen = 0;
-    for (int cxb = cx0; cxb < cx_end; cxb += kNX, ++pen) {
+    for (int cxb = cx0; cxb < cx_end; cxb += LX, ++pen) {
       const int cx = cxb + c;
       const long cell = min(cx, P.nc[0] - 1) + (long)P.nc[0] * (cy + (long)P.nc[1] * czc);
       Number u[N1][N1][N1], v[N1][N1][N1];
@@ -1130,9 +1129,9 @@ __global__ __launch_bounds__(64) void heat_cells_kernel(const BrickArgs<Number, 
         sweep_cell<N1, 0, true, false>(P.S, e, v);
       }
       // ---- per plane, from the top: sums over the brick's cells (along y through LDS, along x to the next
-      //      lane, along z to the lane 16 above), then the stores: to dst, or to the classes of the brick's
+      //      lane, along z to the next row of lanes), then the stores: to dst, or to the classes of the brick's
       //      upper planes ----
-      const bool more = cxb + kNX < cx_end, hy = last && cy_end != P.nc[1], hx = cx_end != P.nc[0];
+      const bool more = cxb + LX < cx_end, hy = last && cy_end != P.nc[1], hx = cx_end != P.nc[0];
       const bool on = cx < P.nc[0] && cz < P.nc[2], end_z = cz == P.nc[2] - 1, end_x = cx == cx_end - 1;
       const long ny1 = P.g.nb[1] - 1, nz1 = P.g.nb[2] - 1;
       double up[N1][N1];
@@ -1154,16 +1153,17 @@ __global__ __launch_bounds__(64) void heat_cells_kernel(const BrickArgs<Number, 
 #pragma unroll
         for (int j = 0; j < N1; ++j) {
           if (j == K && !last) continue;
-          r[j][0] += from_previous_cell(r[j][K], pen > 0 ? xcol[N1 * l + j][zc] : 0.0);
-          if (more && c == kNX - 1) xcol[N1 * l + j][zc] = r[j][K];
+          const double carried = pen > 0 ? xcol[N1 * l + j][zc] : 0.0, left = from_previous_cell(r[j][K], carried);
+          r[j][0] += c == 0 ? carried : left;
+          if (more && c == LX - 1) xcol[N1 * l + j][zc] = r[j][K];
 #pragma unroll
           for (int i = 0; i < N1; ++i) {
-            if (l == K) up[j][i] = from_cell_below(r[j][i], lane);
+            if (l == K) up[j][i] = from_lane(r[j][i], lane - LX);
             if (l == 0) r[j][i] += zc > 0 ? up[j][i] : 0.0;
           }
         }
         if (bmask) constrain_plane(cx, cy, l, r);
-        if (!on || (l == K && !end_z && zc != kCellsZ - 1)) continue;
+        if (!on || (l == K && !end_z && zc != LZ - 1)) continue;
         const bool hz = l == K && !end_z;
         const int iz = K * cz + l;
 #pragma unroll
@@ -1465,7 +1465,10 @@ template <int N1, typename Number> dim3 brick_blocks(const BrickArgs<Number, N1>
 #define MPDG_APPLY(KM)                                                                                                 \
   do {                                                                                                                 \
     if constexpr (N1 < 4)                                                                                              \
-      hipLaunchKernelGGL((heat_cells_kernel<N1, Number, KM>), brick_blocks(A), dim3(64), 0, stream, A, src, dst);      \
+      if (op.brick_cells[2] == 8)                                                                                      \
+        hipLaunchKernelGGL((heat_cells_kernel<N1, Number, KM, 8>), brick_blocks(A), dim3(64), 0, stream, A, src, dst); \
+      else                                                                                                             \
+        hipLaunchKernelGGL((heat_cells_kernel<N1, Number, KM, 16>), brick_blocks(A), dim3(64), 0, stream, A, src, dst); \
     else                                                                                                               \
       MPDG_BRICK(KM, false, false);                                                                                    \
   } while (0)
@@ -1596,8 +1599,8 @@ int launch_brick_tangent_data_n1(const OperatorData<double> &op, double dt, cons
 struct BrickModel {
   double resident, latency, startup, planes, x_planes;
 };
-static void least_time(const BrickModel &m, int k, const int *nc, int zc, int *brick) {
-  const long px = (nc[0] + kNX - 1) / kNX, nz = (nc[2] + zc - 1) / zc, cus = 256;
+static void least_time(const BrickModel &m, int k, const int *nc, int lx, int zc, int *brick) {
+  const long px = (nc[0] + lx - 1) / lx, nz = (nc[2] + zc - 1) / zc, cus = 256;
   const double nd[3] = {k * (double)nc[0] + 1, k * (double)nc[1] + 1, k * (double)nc[2] + 1};
   const double steps = (double)px * nc[1] * nz / cus;
   double best = 0.0;
@@ -1620,8 +1623,14 @@ void choose_brick(int k, const int *nc, int *brick, int *brick_cells) {
   static const BrickModel bricks[4] = {{}, {6, 4, 0.2, 1.0, 8}, {4, 2.5, 0.7, 0.0, 8}, {4, 2.5, 0.2, 0.5, 8}};
   static const BrickModel cells = {12, 12, 0.2, 0.5, 1};
   if (k > 3) return;
-  least_time(bricks[k], k, nc, zc_of(k, false), brick);
-  if (k < 3) least_time(cells, k, nc, zc_of(k, true), brick_cells);
+  least_time(bricks[k], k, nc, kNX, zc_of(k), brick);
+  if (k > 2) return;
+  // Pencils of 8 cells where those of 16 leave many lanes without a cell; they load and store shorter runs and
+  // share more x planes. Q2 17 x 90 x 90 k per point FP32 31.6 -> 26.8 us, with a law 44.5 -> 35.3; 24 x 50 x 50
+  // 16.0 -> 16.1 us (FP64 21.9 -> 20.7); on the other side 56^3 FP64 22.4 -> 25.3 us, 72^3 56.5 -> 52.9 us.
+  auto lanes = [&](int lx) { return (nc[0] + lx - 1) / lx * lx * (double)((nc[2] + 64 / lx - 1) / (64 / lx) * (64 / lx)); };
+  brick_cells[2] = lanes(16) >= 1.2 * lanes(8) ? 8 : 16;
+  least_time(cells, k, nc, brick_cells[2], 64 / brick_cells[2], brick_cells);
 }
 
 size_t brick_scratch_elems(int degree, const int *nc, const int *brick, const int *brick_cells) {

@@ -102,7 +102,7 @@ struct OperatorData {
   // columns meet, all zero between applies; Q1..Q3: the bricks' upper planes, written by every apply
   Number *edge = nullptr;
   size_t edge_elems = 0;
-  int brick[2] = {1, 1}, brick_cells[2] = {1, 1};  // Q1..Q3: choose_brick
+  int brick[2] = {1, 1}, brick_cells[3] = {1, 1, 16};  // Q1..Q3: choose_brick
   void set_mesh(int k, const int *ncells, const double *ext) {
     degree = k;
     for (int d = 0; d < 3; ++d) {

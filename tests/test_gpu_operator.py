@@ -445,7 +445,14 @@ BRICK_CASES = [(1, (1, 1, 1), "const", 0, 0), (1, (15, 2, 8), "cell", 0, 0b10000
                (3, (33, 40, 140), "qp", 0, 0b100000), (2, (70, 65, 60), "const", 1, 0), (1, (40, 90, 120), "law", 0, 0)]
 
 
-@pytest.mark.parametrize("degree,nc,mode,precision,dmask", BRICK_CASES)
+# one cell per lane: pencils of 8 cells along x with 8 along z (17 to 24 cells along x, 8 or fewer), of 16 with 4
+LANE_CASES = [(1, (8, 3, 9), "qp", 0, 0b010101), (2, (17, 5, 8), "law", 1, 0), (2, (24, 4, 17), "cell", 0, 0b111111),
+              (1, (20, 9, 15), "law", 0, 0b101010), (2, (7, 17, 7), "qp", 1, 0b000011), (2, (16, 5, 5), "law", 0, 0b110000),
+              (1, (23, 2, 8), "const", 1, 0), (2, (1, 1, 1), "qp", 0, 0), (2, (25, 3, 4), "const", 0, 0b001000),
+              (1, (64, 104, 172), "qp", 0, 0)]  # (bricks of two pencils)
+
+
+@pytest.mark.parametrize("degree,nc,mode,precision,dmask", BRICK_CASES + LANE_CASES)
 def test_vmult_at_brick_edges(cuda, degree, nc, mode, precision, dmask):
     torch = cuda
     orc, gop, _ = make_pair(torch, degree, nc, mode=mode, precision=precision, dirichlet=dmask, seed=21)
