@@ -133,86 +133,117 @@ int launch_coarse_matrix(const OperatorData<T> &od, double c_mass, const double 
 // matrix [[A11, A12], [A21, A22]] one step writes
 //   A11 <- A11^-1,  A12 <- A11^-1 A12,  A22 <- A22 - A21 A11^-1 A12,  A21 <- -A21 A11^-1
 // (the scalar step with 1x1 blocks is the textbook in-place Gauss-Jordan); after the last block
-// the array holds A^-1. Four launches per block: diagonal block, row panel, rank-nb update of
-// everything outside the block's rows and columns (which reads the old column panel and the new
-// row panel), column panel.
+// the array holds A^-1. Two launches per block: both panels (the old column panel is kept in old_col), and the
+// rank-nb update of everything outside the block's rows and columns, whose workgroup with the next
+// diagonal block inverts that too. What bounds it: the chain of launches, each a few microseconds of
+// latencies on a few workgroups. n = 729: 23 blocks in 0.61 ms; four launches per block, with the panels by
+// one thread per row or column and the diagonal block by a workgroup with two barriers per pivot, took
+// 2.0 ms and were the longest part of a multigrid update.
 constexpr int kGJB = 32;    // block width
 constexpr int kGJTile = 64;  // update tile (64 x 64 per workgroup, 4 x 4 per thread)
 
-__global__ __launch_bounds__(256) void gjb_diag_kernel(double *A, int n, int k0, int nb) {
-  __shared__ double D[kGJB][kGJB + 1];
+// Inverse of the nb x nb block in D (padded with the identity) into A, by the first wavefront: lane = 32 (half of
+// the columns) + row, 16 values in registers; the pivot row goes through LDS
+__device__ __forceinline__ void gjb_invert_block(double (&D)[kGJB][kGJB + 1], double (&R)[kGJB], double *A, int n, int k0, int nb) {
+  const int lane = threadIdx.x, i = lane & 31, h = lane >> 5;
+  if (lane >= 64) return;
+  double a[16];
+#pragma unroll
+  for (int m = 0; m < 16; ++m) a[m] = i < nb && 16 * h + m < nb ? D[i][16 * h + m] : (i == 16 * h + m ? 1.0 : 0.0);
+#pragma unroll
+  for (int k = 0; k < kGJB; ++k) {
+    if (i == k) {
+#pragma unroll
+      for (int m = 0; m < 16; ++m) R[16 * h + m] = a[m];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const double piv = 1.0 / R[k], mine = a[k % 16], other = __shfl_xor(mine, 32);
+    const double f = (h == k / 16 ? mine : other) * piv, scale = i == k ? piv : 1.0, g = i == k ? 0.0 : f;
+#pragma unroll
+    for (int m = 0; m < 16; ++m) a[m] = fma(-g, R[16 * h + m], a[m] * scale);
+    if (h == k / 16) a[k % 16] = i == k ? piv : -f;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+#pragma unroll
+  for (int m = 0; m < 16; ++m)
+    if (i < nb && 16 * h + m < nb) A[(long)(k0 + i) * n + k0 + 16 * h + m] = a[m];
+}
+
+__global__ __launch_bounds__(256) void gjb_diag_kernel(double *A, int n, int nb) {
+  __shared__ double D[kGJB][kGJB + 1], R[kGJB];
   for (int e = threadIdx.x; e < nb * nb; e += 256) {
     const int i = e / nb, j = e - i * nb;
-    D[i][j] = A[(long)(k0 + i) * n + k0 + j];
+    D[i][j] = A[(long)i * n + j];
   }
   __syncthreads();
-  constexpr int kPer = kGJB * kGJB / 256;
-  for (int k = 0; k < nb; ++k) {
-    const double piv = 1.0 / D[k][k];
-    double v[kPer];
+  gjb_invert_block(D, R, A, n, 0, nb);
+}
+
+// A12 <- A11^-1 A12 (workgroups 0 .. tiles - 1, 32 columns each) and A21 <- -A21 A11^-1 with the old A21 to old_col
+// (n x 32; the other workgroups, 32 rows each)
+__global__ __launch_bounds__(256) void gjb_panel_kernel(double *A, double *old_col, int n, int k0, int nb, int tiles) {
+  __shared__ double D[kGJB][kGJB + 1], X[kGJB][kGJB + 1];
+  const bool rows = (int)blockIdx.x < tiles;  // the row panel
+  const int t0 = kGJB * (rows ? blockIdx.x : blockIdx.x - tiles), c = threadIdx.x & 31, g = threadIdx.x >> 5;
+  if (t0 == k0) return;
 #pragma unroll
-    for (int m = 0; m < kPer; ++m) {
-      const int e = threadIdx.x + 256 * m, i = e / kGJB, j = e - i * kGJB;
-      double x = 0.0;
-      if (i < nb && j < nb) {
-        if (i == k && j == k) x = piv;
-        else if (i == k) x = D[k][j] * piv;
-        else if (j == k) x = -D[i][k] * piv;
-        else x = D[i][j] - D[i][k] * D[k][j] * piv;
-      }
-      v[m] = x;
+  for (int m = 0; m < 4; ++m) {
+    const int r = g + 8 * m;
+    D[r][c] = r < nb && c < nb ? A[(long)(k0 + r) * n + k0 + c] : 0.0;
+    if (rows) {
+      X[r][c] = r < nb && t0 + c < n ? A[(long)(k0 + r) * n + t0 + c] : 0.0;
+    } else {
+      X[r][c] = t0 + r < n && c < nb ? A[(long)(t0 + r) * n + k0 + c] : 0.0;
+      if (t0 + r < n) old_col[(long)(t0 + r) * kGJB + c] = X[r][c];
     }
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < kPer; ++m) {
-      const int e = threadIdx.x + 256 * m, i = e / kGJB, j = e - i * kGJB;
-      if (i < nb && j < nb) D[i][j] = v[m];
-    }
-    __syncthreads();
   }
-  for (int e = threadIdx.x; e < nb * nb; e += 256) {
-    const int i = e / nb, j = e - i * nb;
-    A[(long)(k0 + i) * n + k0 + j] = D[i][j];
+  __syncthreads();
+  double s[4] = {};
+#pragma unroll 8
+  for (int q = 0; q < kGJB; ++q)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) s[m] += rows ? D[g + 8 * m][q] * X[q][c] : X[g + 8 * m][q] * D[q][c];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const int r = g + 8 * m;
+    if (rows) {
+      if (r < nb && t0 + c < n) A[(long)(k0 + r) * n + t0 + c] = s[m];
+    } else {
+      if (t0 + r < n && c < nb) A[(long)(t0 + r) * n + k0 + c] = -s[m];
+    }
   }
 }
 
-// A12 <- A11^-1 A12, one thread per column outside the block
-__global__ __launch_bounds__(256) void gjb_row_kernel(double *A, int n, int k0, int nb) {
-  __shared__ double D[kGJB][kGJB + 1];
-  for (int e = threadIdx.x; e < nb * nb; e += 256) {
-    const int i = e / nb, j = e - i * nb;
-    D[i][j] = A[(long)(k0 + i) * n + k0 + j];
-  }
-  __syncthreads();
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= n || (j >= k0 && j < k0 + nb)) return;
-  double c[kGJB];
-#pragma unroll
-  for (int r = 0; r < kGJB; ++r) c[r] = r < nb ? A[(long)(k0 + r) * n + j] : 0.0;
-#pragma unroll
-  for (int r = 0; r < kGJB; ++r) {
-    if (r >= nb) break;
-    double s = 0.0;
-#pragma unroll
-    for (int q = 0; q < kGJB; ++q) s += (q < nb ? D[r][q] : 0.0) * c[q];
-    A[(long)(k0 + r) * n + j] = s;
-  }
-}
-
-// A22 <- A22 - A21 A12 for rows and columns outside the block (A12 already updated)
-__global__ __launch_bounds__(256) void gjb_update_kernel(double *A, int n, int k0, int nb) {
-  __shared__ double Ct[kGJB][kGJTile + 1], Rt[kGJB][kGJTile + 1];
+// A22 <- A22 - (old A21) A12 for rows and columns outside the block (A12 already updated); then the next block's
+// inverse
+__global__ __launch_bounds__(256) void gjb_update_kernel(double *A, const double *old_col, int n, int k0, int nb) {
+  __shared__ double Ct[kGJB][kGJTile + 1], Rt[kGJB][kGJTile + 1], D[kGJB][kGJB + 1], R[kGJB];
   const int i0 = blockIdx.y * kGJTile, j0 = blockIdx.x * kGJTile;
   for (int e = threadIdx.x; e < kGJTile * kGJB; e += 256) {
-    const int ii = e / kGJB, c = e - ii * kGJB;
-    Ct[c][ii] = (i0 + ii < n && c < nb) ? A[(long)(i0 + ii) * n + k0 + c] : 0.0;
+    const int ii = e / kGJB, c = e - ii * kGJB, i = i0 + ii;
+    Ct[c][ii] = i < n && c < nb && !(i >= k0 && i < k0 + nb) ? old_col[(long)i * kGJB + c] : 0.0;
   }
   for (int e = threadIdx.x; e < kGJTile * kGJB; e += 256) {
     const int c = e / kGJTile, jj = e - c * kGJTile;
     Rt[c][jj] = (j0 + jj < n && c < nb) ? A[(long)(k0 + c) * n + j0 + jj] : 0.0;
   }
-  __syncthreads();
   const int ty = threadIdx.x / 16, tx = threadIdx.x - ty * 16;
+  auto outside = [&](int i, int j) {
+    return i < n && j < n && !(i >= k0 && i < k0 + nb) && !(j >= k0 && j < k0 + nb);
+  };
+  double v[4][4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int i = i0 + ty + 16 * m, j = j0 + tx + 16 * p;
+      v[m][p] = outside(i, j) ? A[(long)i * n + j] : 0.0;
+    }
+  __syncthreads();
   double acc[4][4] = {};
 #pragma unroll 8
   for (int c = 0; c < kGJB; ++c) {
@@ -227,49 +258,31 @@ __global__ __launch_bounds__(256) void gjb_update_kernel(double *A, int n, int k
 #pragma unroll
       for (int p = 0; p < 4; ++p) acc[m][p] = fma(a[m], b[p], acc[m][p]);
   }
+  const int k1 = k0 + kGJB, nb1 = min(kGJB, n - k1);
+  const bool next = i0 == j0 && k1 < n && k1 >= i0 && k1 < i0 + kGJTile;  // (blocks do not straddle tiles)
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int i = i0 + ty + 16 * m;
-    if (i >= n || (i >= k0 && i < k0 + nb)) continue;
+  for (int m = 0; m < 4; ++m)
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-      const int j = j0 + tx + 16 * p;
-      if (j < n && !(j >= k0 && j < k0 + nb)) A[(long)i * n + j] -= acc[m][p];
+      const int i = i0 + ty + 16 * m, j = j0 + tx + 16 * p;
+      const double x = v[m][p] - acc[m][p];
+      if (next && i >= k1 && i < k1 + nb1 && j >= k1 && j < k1 + nb1) D[i - k1][j - k1] = x;
+      else if (outside(i, j)) A[(long)i * n + j] = x;
     }
+  if (next) {  // (uniform)
+    __syncthreads();
+    gjb_invert_block(D, R, A, n, k1, nb1);
   }
 }
 
-// A21 <- -A21 A11^-1, one thread per row outside the block
-__global__ __launch_bounds__(256) void gjb_col_kernel(double *A, int n, int k0, int nb) {
-  __shared__ double D[kGJB][kGJB + 1];
-  for (int e = threadIdx.x; e < nb * nb; e += 256) {
-    const int i = e / nb, j = e - i * nb;
-    D[i][j] = A[(long)(k0 + i) * n + k0 + j];
-  }
-  __syncthreads();
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n || (i >= k0 && i < k0 + nb)) return;
-  double r[kGJB];
-#pragma unroll
-  for (int q = 0; q < kGJB; ++q) r[q] = q < nb ? A[(long)i * n + k0 + q] : 0.0;
-#pragma unroll
-  for (int c = 0; c < kGJB; ++c) {
-    if (c >= nb) break;
-    double s = 0.0;
-#pragma unroll
-    for (int q = 0; q < kGJB; ++q) s += r[q] * (q < nb ? D[q][c] : 0.0);
-    A[(long)i * n + k0 + c] = -s;
-  }
-}
-
-int launch_gauss_jordan_inverse(double *A, int n, hipStream_t s) {
-  const int b1 = (n + 255) / 256, bt = (n + kGJTile - 1) / kGJTile;
-  for (int k0 = 0; k0 < n; k0 += kGJB) {
+size_t gauss_jordan_scratch(int n) { return (size_t)n * kGJB; }
+int launch_gauss_jordan_inverse(double *A, double *scratch, int n, hipStream_t s) {
+  const int tiles = (n + kGJB - 1) / kGJB, bt = (n + kGJTile - 1) / kGJTile;
+  hipLaunchKernelGGL(gjb_diag_kernel, dim3(1), dim3(256), 0, s, A, n, std::min(kGJB, n));
+  for (int k0 = 0; k0 < n && tiles > 1; k0 += kGJB) {
     const int nb = std::min(kGJB, n - k0);
-    hipLaunchKernelGGL(gjb_diag_kernel, dim3(1), dim3(256), 0, s, A, n, k0, nb);
-    hipLaunchKernelGGL(gjb_row_kernel, dim3(b1), dim3(256), 0, s, A, n, k0, nb);
-    hipLaunchKernelGGL(gjb_update_kernel, dim3(bt, bt), dim3(256), 0, s, A, n, k0, nb);
-    hipLaunchKernelGGL(gjb_col_kernel, dim3(b1), dim3(256), 0, s, A, n, k0, nb);
+    hipLaunchKernelGGL(gjb_panel_kernel, dim3(2 * tiles), dim3(256), 0, s, A, scratch, n, k0, nb, tiles);
+    hipLaunchKernelGGL(gjb_update_kernel, dim3(bt, bt), dim3(256), 0, s, A, scratch, n, k0, nb);
   }
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }

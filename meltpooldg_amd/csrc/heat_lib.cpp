@@ -364,7 +364,7 @@ template <typename T>
 struct GMGPrecond : mpdg_precond {
   mpdg_gmg_params prm{};
   std::vector<std::unique_ptr<Level<T>>> lev;  // 0 = coarsest
-  DeviceArray<double> coarse_inv, coarse_elem, cvec_part, eig_hist, kcell64, kcell_pp[2];
+  DeviceArray<double> coarse_inv, coarse_elem, coarse_col, cvec_part, eig_hist, kcell64, kcell_pp[2];
   ReductionScratch red;
   int nc_coarse_dofs = 0;
   // update(): the coarse matrix and the levels below the finest run on streams of their own
@@ -745,7 +745,8 @@ struct GMGPrecond : mpdg_precond {
     MPDG_TRY(coarse_elem.resize((size_t)od.n_cells * n1 * n1 * n1 * n1 * n1 * n1));
     MPDG_TRY(launch_coarse_matrix<T>(od, f.c_mass, kc, f.kappa, coarse_inv.get(), coarse_elem.get(), s));
     // the inverse of a symmetric matrix is symmetric: row-major == column-major for the gemv
-    return launch_gauss_jordan_inverse(coarse_inv.get(), (int)od.n_dofs, s);
+    MPDG_TRY(coarse_col.resize(gauss_jordan_scratch((int)od.n_dofs)));
+    return launch_gauss_jordan_inverse(coarse_inv.get(), coarse_col.get(), (int)od.n_dofs, s);
   }
 
   int prolongate_add(Level<T> &F, const Level<T> &C, hipStream_t s) {

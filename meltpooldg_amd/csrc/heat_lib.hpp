@@ -21,7 +21,9 @@ namespace mpdg {
 template <typename T>
 int launch_coarse_matrix(const OperatorData<T> &od, double c_mass, const double *kc, double kconst, double *A,
                          double *E, hipStream_t s);
-int launch_gauss_jordan_inverse(double *A, int n, hipStream_t s);
+// scratch: gauss_jordan_scratch(n) values
+size_t gauss_jordan_scratch(int n);
+int launch_gauss_jordan_inverse(double *A, double *scratch, int n, hipStream_t s);
 
 #define MPDG_TRY_INNER(...)         \
   do {                              \

@@ -393,3 +393,27 @@ def test_least_squares_projection_reference_mode(cuda):
     expect = np.linalg.norm(bn - Jg.cpu().numpy()) / np.linalg.norm(bn)
     _, _, (_, r0, _) = case.step()
     assert abs(r0 - expect) <= 1e-6 * expect
+
+
+# edges of the coarse inverse's blocks (32) and update tiles (64): 8, 27, 32, 36, 64, 96, 125, 729 unknowns
+@pytest.mark.parametrize("degree,nc,dmask", [(1, (1, 1, 1), 0), (2, (1, 1, 1), 0b000001), (1, (3, 3, 1), 0), (1, (2, 2, 3), 0),
+                                             (1, (3, 3, 3), 0b100000), (1, (3, 3, 5), 0), (4, (1, 1, 1), 0), (2, (4, 4, 4), 0b000011)])
+def test_coarse_inverse_at_block_edges(cuda, degree, nc, dmask):
+    """One level: the preconditioner is the dense inverse of the operator (condition below 1e3 here)."""
+    torch = cuda
+    import meltpooldg_amd as M
+    op = M.HeatDiffuseMultiPhaseOperator(degree, nc, (1.0, 0.9, 1.1), rho_cp=1.0, dirichlet_faces=dmask)
+    op.reset_time_increment(1.0)
+    op.set_conductivity_constant(0.01)
+    pc = M.GMGPreconditioner(op, precision=M.FP64, n_cells_coarse=max(nc), coarse_degree=degree)
+    b = torch.rand(op.n_dofs, dtype=torch.float64, device="cuda", generator=torch.Generator(device="cuda").manual_seed(4))
+    if dmask:  # the operator leaves constrained rows out, the coarse matrix has the identity there
+        ones, inside = torch.ones_like(b), torch.empty_like(b)
+        op.vmult(inside, ones)
+        b = torch.where(inside == 0.0, torch.zeros_like(b), b)
+    x, back = torch.empty_like(b), torch.empty_like(b)
+    for _ in range(2):  # a second set-up starts from the first one's arrays
+        pc.update()
+        pc.vmult(x, b)
+        op.vmult(back, x)
+        assert float((back - b).abs().max()) < 1e-11 * float(b.abs().max())
