@@ -552,11 +552,14 @@ int cg_direction(double *p, const double *z, long n, const CGState *st, hipStrea
 // written only when a later step of the same call reads it: a degree-p call (p >= 2) from a
 // nonzero x moves 6 + 7 (p - 2) + 6 vectors instead of 7 p, and a degree-1 call from x = 0
 // moves 3 instead of 4.
-template <typename T>
+// SUMS: Ax without the classes of its shared planes, which are added here (the pass over the planes alone takes
+// 4 us on the coarse levels and 10 us on Q3 64^3, three times per level and cycle)
+template <typename T, bool SUMS>
 __global__ __launch_bounds__(256) void cheb_kernel(T *x, T *d, const T *b, const T *Ax, const T *inv, long n,
-                                                   T c1, T c2, int zero_start, int read_d, int write_d) {
+                                                   T c1, T c2, int zero_start, int read_d, int write_d, BrickSums<T> sums) {
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    const T r = zero_start ? b[i] : b[i] - Ax[i];
+    T r = b[i];
+    if (!zero_start) r -= SUMS ? brick_sum(sums, Ax[i], (unsigned)i) : Ax[i];
     const T di = read_d ? c1 * d[i] + c2 * inv[i] * r : c2 * inv[i] * r;
     if (write_d) d[i] = di;
     x[i] = zero_start ? di : x[i] + di;
@@ -564,15 +567,20 @@ __global__ __launch_bounds__(256) void cheb_kernel(T *x, T *d, const T *b, const
 }
 template <typename T>
 int launch_chebyshev_step(T *x, T *d, const T *b, const T *Ax, const T *inv, long n, double c1, double c2,
-                          bool zero_start, bool read_d, bool write_d, hipStream_t s) {
-  hipLaunchKernelGGL(cheb_kernel<T>, dim3(std::min<long>((n + 255) / 256, 8192)), dim3(256), 0, s, x, d, b, Ax, inv,
-                     n, (T)c1, (T)c2, zero_start ? 1 : 0, read_d ? 1 : 0, write_d ? 1 : 0);
+                          bool zero_start, bool read_d, bool write_d, hipStream_t s, const BrickSums<T> &sums) {
+  const dim3 grid(std::min<long>((n + 255) / 256, 8192)), block(256);
+  if (sums.active)
+    hipLaunchKernelGGL((cheb_kernel<T, true>), grid, block, 0, s, x, d, b, Ax, inv, n, (T)c1, (T)c2, zero_start ? 1 : 0,
+                       read_d ? 1 : 0, write_d ? 1 : 0, sums);
+  else
+    hipLaunchKernelGGL((cheb_kernel<T, false>), grid, block, 0, s, x, d, b, Ax, inv, n, (T)c1, (T)c2, zero_start ? 1 : 0,
+                       read_d ? 1 : 0, write_d ? 1 : 0, sums);
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }
 template int launch_chebyshev_step<float>(float *, float *, const float *, const float *, const float *, long,
-                                          double, double, bool, bool, bool, hipStream_t);
+                                          double, double, bool, bool, bool, hipStream_t, const BrickSums<float> &);
 template int launch_chebyshev_step<double>(double *, double *, const double *, const double *, const double *, long,
-                                           double, double, bool, bool, bool, hipStream_t);
+                                           double, double, bool, bool, bool, hipStream_t, const BrickSums<double> &);
 
 // r = b - Ax
 template <typename T>

@@ -806,18 +806,18 @@ int launch_apply_shape(const OperatorData<Number> &op, const Number *src, Number
 
 template <typename Number>
 int launch_apply(const OperatorData<Number> &op_in, const Number *src, Number *dst, hipStream_t stream,
-                 hipEvent_t kernel_start, hipEvent_t kernel_end) {
+                 hipEvent_t kernel_start, hipEvent_t kernel_end, BrickSums<Number> *sums) {
   const OperatorData<Number> op = kernel_view(op_in);
   if (op.metric == nullptr && op_in.metric != nullptr) return MPDG_ERR_INVALID;  // metric_k not computed
-  if (op.degree >= 1 && op.degree <= 3) return launch_brick<Number>(op, src, dst, stream, kernel_start, kernel_end);
+  if (op.degree >= 1 && op.degree <= 3) return launch_brick<Number>(op, src, dst, stream, kernel_start, kernel_end, sums);
   if (op.degree != 4) return MPDG_ERR_INVALID;
   if (op.metric) return launch_apply_shape<5, Number, true>(op, src, dst, stream, kernel_start, kernel_end);
   return launch_apply_shape<5, Number, false>(op, src, dst, stream, kernel_start, kernel_end);
 }
 
 template int launch_apply<double>(const OperatorData<double> &, const double *, double *, hipStream_t, hipEvent_t,
-                                  hipEvent_t);
+                                  hipEvent_t, BrickSums<double> *);
 template int launch_apply<float>(const OperatorData<float> &, const float *, float *, hipStream_t, hipEvent_t,
-                                 hipEvent_t);
+                                 hipEvent_t, BrickSums<float> *);
 
 }  // namespace mpdg

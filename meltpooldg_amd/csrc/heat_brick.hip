@@ -46,15 +46,6 @@ template <int N1> struct BrickShape {
   static constexpr int ZC = kNW * ZPW;         // cells along z per brick
 };
 
-// A brick is cells[0] x cells[1] x cells[2] cells: pencils of kNX cells side by side along x, done one
-// after the other, steps along y, pencils along z. Shared-plane classes: bit 0 upper x plane, bit 1
-// upper y plane, bit 2 upper z plane.
-struct BrickGrid {
-  int nb[3];       // bricks
-  int cells[3];    // cells of a full brick
-  long off[8];     // scratch offset of each class (off[0] unused)
-  long total;      // scratch entries
-};
 constexpr int kMaxSteps = 16, kMaxPencils = 2;
 
 constexpr int zc_of(int k) { return k == 1 ? BrickShape<2>::ZC : BrickShape<3>::ZC; }
@@ -1475,7 +1466,7 @@ template <int N1, typename Number> dim3 brick_blocks(const BrickArgs<Number, N1>
 
 template <int N1, typename Number>
 int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
-                    hipEvent_t kernel_start, hipEvent_t kernel_end) {
+                    hipEvent_t kernel_start, hipEvent_t kernel_end, BrickSums<Number> *sums) {
   BrickArgs<Number, N1> A;
   const bool cells = N1 < 4 && !op.metric;
   if (const int rc = fill_brick_args(op, op.metric != nullptr, A, cells)) return rc;
@@ -1496,6 +1487,10 @@ int launch_brick_n1(const OperatorData<Number> &op, const Number *src, Number *d
     }
   }
   if (kernel_end) (void)hipEventRecord(kernel_end, stream);
+  if (sums && A.g.total > 0 && op.n_dofs < (1l << 31)) {
+    *sums = BrickSums<Number>(A.scratch, A.g, N1 - 1, op.nd);
+    return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
+  }
   return finish_brick(A, dst, stream);
 }
 
@@ -1640,16 +1635,18 @@ size_t brick_scratch_elems(int degree, const int *nc, const int *brick, const in
 
 template <typename Number>
 int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
-                 hipEvent_t kernel_start, hipEvent_t kernel_end) {
+                 hipEvent_t kernel_start, hipEvent_t kernel_end, BrickSums<Number> *sums) {
   switch (op.degree) {
-    case 1: return launch_brick_n1<2, Number>(op, src, dst, stream, kernel_start, kernel_end);
-    case 2: return launch_brick_n1<3, Number>(op, src, dst, stream, kernel_start, kernel_end);
-    case 3: return launch_brick_n1<4, Number>(op, src, dst, stream, kernel_start, kernel_end);
+    case 1: return launch_brick_n1<2, Number>(op, src, dst, stream, kernel_start, kernel_end, sums);
+    case 2: return launch_brick_n1<3, Number>(op, src, dst, stream, kernel_start, kernel_end, sums);
+    case 3: return launch_brick_n1<4, Number>(op, src, dst, stream, kernel_start, kernel_end, sums);
     default: return MPDG_ERR_INVALID;
   }
 }
-template int launch_brick<double>(const OperatorData<double> &, const double *, double *, hipStream_t, hipEvent_t, hipEvent_t);
-template int launch_brick<float>(const OperatorData<float> &, const float *, float *, hipStream_t, hipEvent_t, hipEvent_t);
+template int launch_brick<double>(const OperatorData<double> &, const double *, double *, hipStream_t, hipEvent_t, hipEvent_t,
+                                  BrickSums<double> *);
+template int launch_brick<float>(const OperatorData<float> &, const float *, float *, hipStream_t, hipEvent_t, hipEvent_t,
+                                 BrickSums<float> *);
 
 int launch_brick_residual(const OperatorData<double> &op, const double *T, const double *T_old, const double *q, double a,
                           double b, double c, double *dst, hipStream_t stream) {

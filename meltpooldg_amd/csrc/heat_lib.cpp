@@ -352,8 +352,8 @@ int upload_int(DeviceArray<int> &dst, const std::vector<int> &src) {
 }
 
 template <typename T>
-int level_apply(const OperatorData<T> &od, const T *src, T *dst, hipStream_t s) {
-  return launch_apply<T>(od, src, dst, s);
+int level_apply(const OperatorData<T> &od, const T *src, T *dst, hipStream_t s, BrickSums<T> *sums = nullptr) {
+  return launch_apply<T>(od, src, dst, s, nullptr, nullptr, sums);
 }
 
 // Geometric multigrid V-cycle: recipe of unit_tests/gmg.cc:343-383, :447-635
@@ -801,9 +801,10 @@ struct GMGPrecond : mpdg_precond {
                                           L.cheb_c2[0], true, false, !last, s));
         continue;
       }
-      MPDG_TRY(level_apply<T>(L.od, L.x.get(), L.Ax.get(), s));
+      BrickSums<T> sums;
+      MPDG_TRY(level_apply<T>(L.od, L.x.get(), L.Ax.get(), s, &sums));
       MPDG_TRY(launch_chebyshev_step<T>(L.x.get(), L.d.get(), L.b.get(), L.Ax.get(), L.inv.get(), n, L.cheb_c1[k],
-                                        L.cheb_c2[k], false, !first, !last, s));
+                                        L.cheb_c2[k], false, !first, !last, s, sums));
     }
     return MPDG_OK;
   }

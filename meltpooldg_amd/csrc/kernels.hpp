@@ -67,6 +67,67 @@ __device__ __forceinline__ Number law_kappa(int law, const Number *p, Number T) 
   return p[0] + (p[1] - p[0]) * (Number(3) - Number(2) * fs) * fs * fs;
 }
 
+// A brick of the Q1..Q3 apply is cells[0] x cells[1] x cells[2] cells: pencils of cells side by side along x,
+// done one after the other, steps along y, pencils along z. Shared-plane classes: bit 0 upper x plane, bit 1
+// upper y plane, bit 2 upper z plane.
+struct BrickGrid {
+  int nb[3];       // bricks
+  int cells[3];    // cells of a full brick
+  long off[8];     // scratch offset of each class (off[0] unused)
+  long total;      // scratch entries
+};
+// n / d for n < 2^31 by a multiplication: m = floor(2^(31 + s) / d) + 1 with 2^s >= d exceeds 2^(31 + s) / d by at
+// most 1, so that n m / 2^(31 + s) exceeds n / d by less than 1 / 2^s <= 1 / d
+struct FixedDivisor {
+  unsigned long m = 1;
+  int d = 1, shift = 0;
+  FixedDivisor() = default;
+  explicit FixedDivisor(int divisor) : d(divisor) {
+    int s = 0;
+    while ((1l << s) < d) ++s;
+    shift = 31 + s;
+    m = (1ul << shift) / d + 1;
+  }
+  __host__ __device__ __forceinline__ unsigned quotient(unsigned n) const { return (unsigned)((n * m) >> shift); }
+};
+// The classes an apply left to its reader: v + brick_sum is what the apply's own pass over the shared planes
+// would have stored, in the same order of summation
+template <typename Number> struct BrickSums {
+  const Number *scratch = nullptr;
+  BrickGrid g{};
+  FixedDivisor nd0, nd1, plane[3];  // grid sizes, DoFs between shared planes
+  int nd2 = 1;
+  bool active = false;
+  BrickSums() = default;
+  BrickSums(const Number *scratch_, const BrickGrid &g_, int K, const int *nd)
+      : scratch(scratch_), g(g_), nd0(nd[0]), nd1(nd[1]), nd2(nd[2]), active(true) {
+    for (int d = 0; d < 3; ++d) plane[d] = FixedDivisor(K * g.cells[d]);
+  }
+};
+#ifdef __HIPCC__
+template <typename Number> __device__ __forceinline__ Number brick_sum(const BrickSums<Number> &B, Number v, unsigned i) {
+  const unsigned row = B.nd0.quotient(i), iz = B.nd1.quotient(row);
+  const int at[3] = {(int)(i - row * B.nd0.d), (int)(row - iz * B.nd1.d), (int)iz};
+  int h[3];  // the shared plane a coordinate lies on (-1: none)
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const int q = (int)B.plane[d].quotient(at[d]);
+    h[d] = q * B.plane[d].d == at[d] && q < B.g.nb[d] ? q - 1 : -1;
+  }
+  if (h[0] < 0 && h[1] < 0 && h[2] < 0) return v;
+  const long ny1 = B.g.nb[1] - 1, nz1 = B.g.nb[2] - 1;
+  double s = (double)v;
+  if (h[0] >= 0) s += (double)B.scratch[B.g.off[1] + ((long)h[0] * B.nd2 + at[2]) * B.nd1.d + at[1]];
+  if (h[1] >= 0) s += (double)B.scratch[B.g.off[2] + (h[1] + ny1 * at[2]) * B.nd0.d + at[0]];
+  if (h[0] >= 0 && h[1] >= 0) s += (double)B.scratch[B.g.off[3] + (h[0] * ny1 + h[1]) * B.nd2 + at[2]];
+  if (h[2] >= 0) s += (double)B.scratch[B.g.off[4] + ((long)h[2] * B.nd1.d + at[1]) * B.nd0.d + at[0]];
+  if (h[0] >= 0 && h[2] >= 0) s += (double)B.scratch[B.g.off[5] + (h[0] * nz1 + h[2]) * B.nd1.d + at[1]];
+  if (h[1] >= 0 && h[2] >= 0) s += (double)B.scratch[B.g.off[6] + (h[1] + ny1 * h[2]) * B.nd0.d + at[0]];
+  if (h[0] >= 0 && h[1] >= 0 && h[2] >= 0) s += (double)B.scratch[B.g.off[7] + (h[0] * ny1 + h[1]) * nz1 + h[2]];
+  return (Number)s;
+}
+#endif
+
 // the bricks of a Q1..Q3 mesh (heat_brick.hip): {pencils along x, steps along y}, and those of the kernel with
 // one cell per lane
 void choose_brick(int degree, const int *n_cells, int *brick, int *brick_cells);
@@ -200,16 +261,18 @@ void fill_apply_args(const OperatorData<Number> &op, ApplyArgs<Number, N1> &A) {
 // heat_apply.hip; `kernel_start` and `kernel_end`, when given, are recorded on the stream
 // right before and after the cell kernel (between the face-row pre-pass and the edge fix-up)
 // so that the event pair times that kernel alone
+// sums (Q1..Q3): where given, dst may be left without the classes of the planes that workgroups share; if so
+// *sums is active and the next reader adds them (brick_sum), before another apply uses op.edge
 template <typename Number>
 int launch_apply(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
-                 hipEvent_t kernel_start = nullptr, hipEvent_t kernel_end = nullptr);
+                 hipEvent_t kernel_start = nullptr, hipEvent_t kernel_end = nullptr, BrickSums<Number> *sums = nullptr);
 // entries of OperatorData::edge the apply of a mesh of degree k and n_cells cells needs
 template <typename Number> size_t apply_edge_elems(const OperatorData<Number> &op);
 
 // heat_brick.hip: the apply for Q1..Q3 and the scratch entries (OperatorData::edge) it needs
 template <typename Number>
 int launch_brick(const OperatorData<Number> &op, const Number *src, Number *dst, hipStream_t stream,
-                 hipEvent_t kernel_start, hipEvent_t kernel_end);
+                 hipEvent_t kernel_start, hipEvent_t kernel_end, BrickSums<Number> *sums = nullptr);
 size_t brick_scratch_elems(int degree, const int *n_cells, const int *brick, const int *brick_cells);
 // Q1..Q3, Cartesian cells: dst -= c_m M (a T + b T_old + c q) + K_k T in one pass (T_old is not read when
 // b = 0, q when null); constrained DoFs count as zero and are left alone, a conductivity law is evaluated at

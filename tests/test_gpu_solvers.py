@@ -417,3 +417,23 @@ def test_coarse_inverse_at_block_edges(cuda, degree, nc, dmask):
         pc.vmult(x, b)
         op.vmult(back, x)
         assert float((back - b).abs().max()) < 1e-11 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("degree,nc", [(1, (40, 24, 20)), (2, (36, 20, 12)), (3, (36, 12, 20))])
+def test_vcycle_is_symmetric_over_many_bricks(cuda, degree, nc):
+    """Equal smoothing before and after the correction: the cycle is a symmetric operator, unless a smoothing step
+    misses or repeats what workgroups sum on their shared planes (FP64; several bricks in every direction)."""
+    torch = cuda
+    import meltpooldg_amd as M
+    op = M.HeatDiffuseMultiPhaseOperator(degree, nc, (1.0, 0.7, 0.5), rho_cp=1.0)
+    op.reset_time_increment(0.1)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    op.set_conductivity_qp(0.5 + torch.rand(op.n_q_points, dtype=torch.float64, device="cuda", generator=g))
+    pc = M.GMGPreconditioner(op, precision=M.FP64, n_cells_coarse=6, coarse_degree=1)
+    pc.update()
+    x, y = (torch.rand(op.n_dofs, dtype=torch.float64, device="cuda", generator=g) - 0.5 for _ in range(2))
+    vx, vy = torch.empty_like(x), torch.empty_like(x)
+    for _ in range(2):
+        pc.vmult(vx, x)
+        pc.vmult(vy, y)
+        assert abs(float(y @ vx) - float(x @ vy)) < 1e-11 * float(x.norm() * vy.norm())
