@@ -195,15 +195,21 @@ __device__ __forceinline__ bool reduce_to_last_block(double (&v)[NQ], double *pa
   __shared__ bool is_last;
   block_reduce<NQ>(v, sh);
   if (threadIdx.x == 0) {
+    // Exchanges whose results are used: the increment is issued after they were performed, in the memory that
+    // all XCDs share. (A device-scope release would write back the L2's dirty lines, those of the kernel's
+    // own vectors among them, at the end of every workgroup.)
+    unsigned long long done = 0;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) partials[q * kRedBlocks + blockIdx.x] = v[q];
-    __threadfence();
-    const unsigned t = atomicAdd(counter, 1u);
+    for (int q = 0; q < NQ; ++q)
+      done |= __hip_atomic_exchange(reinterpret_cast<unsigned long long *>(partials + q * kRedBlocks + blockIdx.x),
+                                    (unsigned long long)__double_as_longlong(v[q]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned one = 1;
+    asm volatile("" : "+v"(one) : "v"(done));
+    const unsigned t = __hip_atomic_fetch_add(counter, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     is_last = (t == gridDim.x - 1);
   }
   __syncthreads();
   if (!is_last) return false;
-  __threadfence();
   // thread t adds the partials t, t + 256, ... in that order; all its loads are issued first
   constexpr int PER = kRedBlocks / 256;
   double part[NQ][PER];
@@ -212,7 +218,10 @@ __device__ __forceinline__ bool reduce_to_last_block(double (&v)[NQ], double *pa
     const int b = threadIdx.x + 256 * r;
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
-      part[q][r] = b < (int)gridDim.x ? __builtin_nontemporal_load(partials + q * kRedBlocks + b) : 0.0;
+      part[q][r] = b < (int)gridDim.x ? __longlong_as_double((long long)__hip_atomic_load(
+                                            reinterpret_cast<const unsigned long long *>(partials + q * kRedBlocks + b),
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                                      : 0.0;
   }
   double w[NQ];
 #pragma unroll

@@ -136,7 +136,7 @@ int launch_coarse_matrix(const OperatorData<T> &od, double c_mass, const double 
 // the array holds A^-1. Two launches per block: both panels (the old column panel is kept in old_col), and the
 // rank-nb update of everything outside the block's rows and columns, whose workgroup with the next
 // diagonal block inverts that too. What bounds it: the chain of launches, each a few microseconds of
-// latencies on a few workgroups. n = 729: 23 blocks in 0.61 ms; four launches per block, with the panels by
+// latencies on a few workgroups. n = 729: 23 blocks in 0.74 ms; four launches per block, with the panels by
 // one thread per row or column and the diagonal block by a workgroup with two barriers per pivot, took
 // 2.0 ms and were the longest part of a multigrid update.
 constexpr int kGJB = 32;    // block width
