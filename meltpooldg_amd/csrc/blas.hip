@@ -246,6 +246,23 @@ __device__ __forceinline__ bool reduce_to_last_block(double (&v)[NQ], double *pa
 // 5-20 %)
 inline int red_blocks(long n) { return (int)std::max<long>(1, std::min<long>(kRedBlocks, (n + 8191) / 8192)); }
 
+// v += a . b, four grid strides per trip with their loads issued together; each thread adds in index order
+template <typename TA, typename TB> __device__ __forceinline__ void dot_strides(const TA *a, const TB *b, long n, double &v) {
+  const long st = (long)gridDim.x * 256;
+  long i = (long)blockIdx.x * 256 + threadIdx.x;
+  for (; i + 3 * st < n; i += 4 * st) {
+    double x[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      x[u] = (double)a[i + u * st];
+      y[u] = (double)b[i + u * st];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v += x[u] * y[u];
+  }
+  for (; i < n; i += st) v += (double)a[i] * (double)b[i];
+}
+
 // ---- generic dot product into a device scalar ----
 template <typename TA, typename TB>
 __global__ __launch_bounds__(256) void dot_kernel(const TA *a, const TB *b, long n, double *partials,
@@ -327,7 +344,7 @@ __global__ __launch_bounds__(256) void cg_alpha_kernel(const double *p, const do
                                                        unsigned *counter, CGState *st) {
   if (st->done) return;
   double v[1] = {0.0};
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) v[0] += p[i] * q[i];
+  dot_strides(p, q, n, v[0]);
   if (reduce_to_last_block<1>(v, partials, counter) && threadIdx.x == 0) {
     st->pq = v[0];
     st->alpha = st->rz / v[0];
@@ -472,14 +489,24 @@ __global__ __launch_bounds__(256) void fcg32_update_kernel(double *x, double *r,
   if (st->done) return;
   const double alpha = st->alpha;
   double v[2] = {0.0, 0.0};
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
-    r32[i] = (float)ri;
+  const long stride = (long)gridDim.x * 256;
+  long i = (long)blockIdx.x * 256 + threadIdx.x;
+  auto step = [&](long at, double xi, double pi, double r_old, double qi, float zi) {
+    x[at] = xi + alpha * pi;
+    const double ri = r_old - alpha * qi;
+    r[at] = ri;
+    r32[at] = (float)ri;
     v[0] += ri * ri;
-    v[1] += ri * (double)z[i];  // r_new . z_old for the flexible beta
+    v[1] += ri * (double)zi;  // r_new . z_old for the flexible beta
+  };
+  for (; i + stride < n; i += 2 * stride) {  // two strides' loads in flight
+    const long k = i + stride;
+    const double x0 = x[i], x1 = x[k], p0 = p[i], p1 = p[k], r0 = r[i], r1 = r[k], q0 = q[i], q1 = q[k];
+    const float z0 = z[i], z1 = z[k];
+    step(i, x0, p0, r0, q0, z0);
+    step(k, x1, p1, r1, q1, z1);
   }
+  if (i < n) step(i, x[i], p[i], r[i], q[i], z[i]);
   if (reduce_to_last_block<2>(v, partials, counter) && threadIdx.x == 0) {
     st->rr = v[0];
     st->iters += 1;
@@ -493,7 +520,7 @@ __global__ __launch_bounds__(256) void fcg32_beta_kernel(const double *r, const 
                                                          unsigned *counter, CGState *st) {
   if (st->done) return;
   double v[1] = {0.0};
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) v[0] += r[i] * (double)z[i];
+  dot_strides(r, z, n, v[0]);
   if (reduce_to_last_block<1>(v, partials, counter) && threadIdx.x == 0) {
     const double num = st->flexible ? v[0] - st->rzold_new : v[0];
     st->beta = num / st->rz;
