@@ -838,22 +838,25 @@ int launch_ell_dir_fields(const EllFields<T> &F, const int *odims, const int *id
 // shared vertex's partial sum to the next cell. lo / hi: homogeneous Dirichlet end (the end
 // value is dropped on input and output, as the ELL form drops its rows and columns).
 // DIR 1, 2: one thread per line along DIR, kHSeg coarse cells per thread (restriction
-// recomputes the carry of the cell before its segment). DIR 0: one wavefront per x line,
-// the line staged in LDS.
+// recomputes the carry of the cell before its segment), or one where that leaves fewer threads than
+// kHThreads: the cells follow each other with a load latency each (z passes of the 4^3 to 16^3 levels of Q3
+// 12 us to restrict and 10 us to prolong with four, 6 and 5 us with one; whole V-cycle of Q2 64^3 404 -> 363 us).
+// DIR 0: one wavefront per x line, the line staged in LDS.
 // ---------------------------------------------------------------------------
 template <typename T, int K> struct HTab { T v[2 * K + 1][K + 1]; };
 constexpr int kHSeg = 4;
+constexpr long kHThreads = 1 << 18;  // four wavefronts per SIMD
 
 // element i of line (t, by): base + i * stride, base = t + by * bstride
 template <typename T, int K>
 __global__ __launch_bounds__(256) void hprolong_kernel(const T *__restrict__ in, T *__restrict__ out, long nl,
                                                        long ibstride, long obstride, long istride, long ostride,
-                                                       int ncc, HTab<T, K> P, int lo, int hi, int add) {
+                                                       int ncc, int seg, HTab<T, K> P, int lo, int hi, int add) {
   const long t = (long)blockIdx.x * 256 + threadIdx.x;
   if (t >= nl) return;
   const long ib = t + ibstride * blockIdx.y, ob = t + obstride * blockIdx.y;
   const int nfine = 2 * K * ncc + 1, ncoarse = K * ncc + 1;
-  const int c0 = blockIdx.z * kHSeg, c1 = min(ncc, c0 + kHSeg);
+  const int c0 = blockIdx.z * seg, c1 = min(ncc, c0 + seg);
   for (int cc = c0; cc < c1; ++cc) {
     T c[K + 1];
 #pragma unroll
@@ -861,6 +864,9 @@ __global__ __launch_bounds__(256) void hprolong_kernel(const T *__restrict__ in,
       const int n = K * cc + j;
       c[j] = ((lo && n == 0) || (hi && n == ncoarse - 1)) ? T(0) : in[ib + istride * n];
     }
+    T old[2 * K];  // (loaded together: between the stores each would wait for its own)
+#pragma unroll
+    for (int m = 0; m < 2 * K; ++m) old[m] = add ? out[ob + ostride * (2 * K * cc + m)] : T(0);
 #pragma unroll
     for (int m = 0; m < 2 * K; ++m) {
       const int g = 2 * K * cc + m;
@@ -868,8 +874,7 @@ __global__ __launch_bounds__(256) void hprolong_kernel(const T *__restrict__ in,
 #pragma unroll
       for (int j = 0; j <= K; ++j) a += P.v[m][j] * c[j];
       if (lo && g == 0) a = 0;
-      const long o = ob + ostride * g;
-      out[o] = add ? out[o] + a : a;
+      out[ob + ostride * g] = add ? old[m] + a : a;
     }
     if (cc == ncc - 1) {
       const long o = ob + ostride * (nfine - 1);
@@ -881,13 +886,13 @@ __global__ __launch_bounds__(256) void hprolong_kernel(const T *__restrict__ in,
 // the fields of FS in turn (each with the same lines)
 template <typename T, int K>
 __global__ __launch_bounds__(256) void hrestrict_kernel(EllFields<T> FS, long nl, long ibstride, long obstride,
-                                                        long istride, long ostride, int ncc, HTab<T, K> P, int lo,
-                                                        int hi) {
+                                                        long istride, long ostride, int ncc, int seg, HTab<T, K> P,
+                                                        int lo, int hi) {
   const long t = (long)blockIdx.x * 256 + threadIdx.x;
   if (t >= nl) return;
   const long ib = t + ibstride * blockIdx.y, ob = t + obstride * blockIdx.y;
   const int nfine = 2 * K * ncc + 1, ncoarse = K * ncc + 1;
-  const int c0 = blockIdx.z * kHSeg, c1 = min(ncc, c0 + kHSeg);
+  const int c0 = blockIdx.z * seg, c1 = min(ncc, c0 + seg);
   for (int fi = 0; fi < FS.nf; ++fi) {
     const T *__restrict__ in = FS.in[fi];
     const T *__restrict__ in2 = FS.in2[fi];
@@ -1018,11 +1023,12 @@ static int htransfer_k(bool restrict_mode, int dir, const EllFields<T> &FS, cons
     os = odims[0];
     gy = (unsigned)odims[2];
   }
-  const dim3 grid((unsigned)((nl + 255) / 256), gy, (ncc + kHSeg - 1) / kHSeg);
+  const int seg = nl * gy * ((ncc + kHSeg - 1) / kHSeg) < kHThreads ? 1 : kHSeg;
+  const dim3 grid((unsigned)((nl + 255) / 256), gy, (ncc + seg - 1) / seg);
   if (restrict_mode)
-    hipLaunchKernelGGL((hrestrict_kernel<T, K>), grid, dim3(256), 0, s, FS, nl, ibs, obs, is, os, ncc, P, lo, hi);
+    hipLaunchKernelGGL((hrestrict_kernel<T, K>), grid, dim3(256), 0, s, FS, nl, ibs, obs, is, os, ncc, seg, P, lo, hi);
   else
-    hipLaunchKernelGGL((hprolong_kernel<T, K>), grid, dim3(256), 0, s, in, out, nl, ibs, obs, is, os, ncc, P, lo, hi,
+    hipLaunchKernelGGL((hprolong_kernel<T, K>), grid, dim3(256), 0, s, in, out, nl, ibs, obs, is, os, ncc, seg, P, lo, hi,
                        add ? 1 : 0);
   return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ERR_DEVICE;
 }
@@ -1088,6 +1094,7 @@ __global__ __launch_bounds__(256) void dense_gemv_part_kernel(const double *__re
   const int len = (n + kGemvSeg - 1) / kGemvSeg;
   const int j0 = k * len, j1 = min(n, j0 + len);
   double acc = 0.0;
+#pragma unroll 8
   for (int j = j0; j < j1; ++j) acc += A[(long)j * n + i] * (double)x[j];
   part[(long)k * n + i] = acc;
 }
