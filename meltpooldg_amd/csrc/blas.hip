@@ -359,19 +359,27 @@ __global__ __launch_bounds__(256) void cg_update_kernel(double *x, double *r, co
   if (st->done) return;
   const double alpha = st->alpha;
   double v[2] = {0.0, 0.0};
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
+  const long stride = (long)gridDim.x * 256;
+  long i = (long)blockIdx.x * 256 + threadIdx.x;
+  // w: the inverse diagonal (JACOBI) or the old z, whose product is r_new . z_old for the flexible beta
+  const double *wp = JACOBI ? inv : z;
+  auto step = [&](long at, double xi, double pi, double r_old, double qi, double w) {
+    x[at] = xi + alpha * pi;
+    const double ri = r_old - alpha * qi;
+    r[at] = ri;
     v[0] += ri * ri;
-    if (JACOBI) {
-      const double zi = inv ? inv[i] * ri : ri;
-      z[i] = zi;
-      v[1] += ri * zi;
-    } else {
-      v[1] += ri * z[i];  // r_new . z_old for the flexible beta
-    }
+    const double zi = JACOBI ? (inv ? w * ri : ri) : w;
+    if (JACOBI) z[at] = zi;
+    v[1] += ri * zi;
+  };
+  for (; i + stride < n; i += 2 * stride) {  // two strides' loads in flight
+    const long k = i + stride;
+    const double x0 = x[i], x1 = x[k], p0 = p[i], p1 = p[k], r0 = r[i], r1 = r[k], q0 = q[i], q1 = q[k];
+    const double w0 = wp ? wp[i] : 1.0, w1 = wp ? wp[k] : 1.0;
+    step(i, x0, p0, r0, q0, w0);
+    step(k, x1, p1, r1, q1, w1);
   }
+  if (i < n) step(i, x[i], p[i], r[i], q[i], wp ? wp[i] : 1.0);
   if (reduce_to_last_block<2>(v, partials, counter) && threadIdx.x == 0) {
     st->rr = v[0];
     st->iters += 1;
@@ -392,7 +400,7 @@ __global__ __launch_bounds__(256) void cg_beta_kernel(const double *r, const dou
                                                       unsigned *counter, CGState *st) {
   if (st->done) return;
   double v[1] = {0.0};
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) v[0] += r[i] * z[i];
+  dot_strides(r, z, n, v[0]);
   if (reduce_to_last_block<1>(v, partials, counter) && threadIdx.x == 0) {
     const double num = st->flexible ? v[0] - st->rzold_new : v[0];
     st->beta = num / st->rz;
