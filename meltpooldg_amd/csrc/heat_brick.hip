@@ -26,11 +26,12 @@
 //     brick_fixup_kernel adds the classes to dst in a fixed order: no atomics and no zeroed
 //     rows, and vmult is bitwise repeatable.
 //
-// What bounds it: at Q3 FP64 with k per point, HBM (2.5 GB moved of 2.0 GB that the apply cannot do
-// without, 870 VALU instructions per 64 lanes and step) -- Q3 128^3, whole vmult: 0.663 ms for the column
+// What bounds it: at Q3 FP64 with k per point, HBM (2.22 GB moved of 1.99 GB that the apply cannot do
+// without, 863 VALU instructions per 64 lanes and step) -- Q3 128^3, whole vmult: 0.663 ms for the column
 // kernel with LDS transposes, scatter and atomics it replaces, 0.566 ms here; elsewhere the VALU (Q3 128^3,
-// constant k: FP64 0.62 -> 0.43 ms, FP32 0.42 -> 0.28 ms; Q2 64^3 FP32 35.7 -> 25.5 us; Q3 75 x 62 x 49 FP32
-// 83.8 -> 50.5 us; mapped Q3 96^3 FP64, bound by the stored metric, 1.08 -> 0.82 ms).
+// constant k: FP64 0.62 -> 0.43 ms, FP32 0.42 -> 0.28 ms; Q3 75 x 62 x 49 FP32 83.8 -> 45.4 us; mapped Q3 96^3
+// FP64, bound by the stored metric, 1.08 -> 0.78 ms). Q1 and Q2 on Cartesian cells run heat_cells_kernel
+// below, one lane per cell; here they run mapped, as residual and as the full tangent.
 #include "tangent.hpp"
 
 namespace mpdg {
