@@ -238,13 +238,11 @@ __device__ __forceinline__ bool reduce_to_last_block(double (&v)[NQ], double *pa
   return true;
 }
 
-// workgroups of a reduction: one per 8192 elements, at most kRedBlocks. Every workgroup ends with a
-// device-scope release (L2 write-back) and an atomic on one counter, so fewer, longer workgroups
-// pay where the vector is small: a Q2 64^3 laser step (2.1 M DoFs, 256 instead of 1024
-// workgroups) runs 2.8 % faster, one workgroup per 16384 elements 2-4 % slower; above 8.4 M
-// elements the count stays at kRedBlocks (capping it at 512 or 256 slows the Q3 128^3 step by
-// 5-20 %)
-inline int red_blocks(long n) { return (int)std::max<long>(1, std::min<long>(kRedBlocks, (n + 8191) / 8192)); }
+// workgroups of a reduction: one per 4096 elements, at most kRedBlocks. More of them have more loads in
+// flight; each ends with an atomic on one counter (40 Jacobi CG iterations of Q1 64^3 with one per 8192 / 4096 /
+// 2048 elements: 1.87 / 1.67 / 1.64 ms, of Q2 64^3 4.76 / 4.34 / 4.47 ms, multigrid set-up of Q3 64^3
+// 3.37 / 3.22 / 3.29 ms)
+inline int red_blocks(long n) { return (int)std::max<long>(1, std::min<long>(kRedBlocks, (n + 4095) / 4096)); }
 
 // v += a . b, four grid strides per trip with their loads issued together; each thread adds in index order
 template <typename TA, typename TB> __device__ __forceinline__ void dot_strides(const TA *a, const TB *b, long n, double &v) {
