@@ -58,6 +58,10 @@ typedef struct mpdg_heat_op mpdg_heat_op;
 
 /* --- operator: HeatDiffuseMultiPhaseOperator<3,double> as an OperatorMatrixFree
        (include/meltpooldg/core/operator_base.hpp:189-282) --- */
+/* Q1..Q3: also allocates the apply's scratch, the DoFs of the planes that workgroups share (0.1 to 0.4
+   vectors on large meshes, up to 1.5 on small ones), so that no apply allocates it and the first one can be
+   captured; one device allocation, 25 to 60 us. Where that fails the first apply tries again. Q4: the
+   first apply allocates. */
 int mpdg_heat_op_create(const mpdg_heat_desc *desc, mpdg_heat_op **op);
 int mpdg_heat_op_destroy(mpdg_heat_op *op);
 long mpdg_heat_op_n_dofs(const mpdg_heat_op *op);

@@ -1168,9 +1168,9 @@ int mpdg_heat_op_create(const mpdg_heat_desc *desc, mpdg_heat_op **out) {
   op->d32.set_mesh(desc->degree, desc->n_cells, desc->extent);
   op->d64.dmask = op->d32.dmask = desc->dirichlet_faces & 63;
   op->d64.c_mass = op->d32.c_mass = desc->rho_cp;  // dt = 1 until reset_time_increment
-  // the apply's scratch, so that mpdg_heat_op_vmult_noalloc finds it; where there is no room (or no
-  // device yet) the first apply tries again and reports the error
-  if (op->precision == MPDG_FP64 && desc->degree < 4 && op->ensure_edge() != MPDG_OK) (void)hipGetLastError();
+  // the apply's scratch, so that a first apply under graph capture and mpdg_heat_op_vmult_noalloc find it;
+  // where there is no room (or no device yet) the first apply tries again and reports the error
+  if (desc->degree < 4 && op->ensure_edge() != MPDG_OK) (void)hipGetLastError();
   *out = op;
   return MPDG_OK;
 }

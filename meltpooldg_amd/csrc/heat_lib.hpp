@@ -164,7 +164,7 @@ struct mpdg_heat_op {
   mutable mpdg::DeviceArray<float> metric32_k, kq32;
   const double *coords = nullptr;
   mutable mpdg::ReductionScratch red;
-  // apply scratch for the rows where four columns meet (OperatorData::edge), zero between applies
+  // apply scratch (OperatorData::edge)
   mutable mpdg::DeviceArray<double> edge64;
   mutable mpdg::DeviceArray<float> edge32;
   // full Newton tangent (mpdg_heat_op_set_tangent): material, velocity, per-qp data at the bound T
@@ -188,7 +188,7 @@ struct mpdg_heat_op {
 
   // mapped meshes with per-qp / k(T) conductivity: fold the conductivity into metric_k
   int refresh_metric_k(hipStream_t s) const;
-  // allocates (zeroed) and binds the apply's edge scratch on first use
+  // allocates and binds the apply's scratch where that is not done yet
   int ensure_edge() const;
   long n_dofs() const { return d64.n_dofs; }
   long n_cells() const { return d64.n_cells; }

@@ -575,3 +575,24 @@ def test_robin_at_tile_edges(cuda, degree, nc, dmask):
     assert rel_err(y.cpu().numpy(), orc.vmult(x)) < 1e-12
     assert rel_err(d.cpu().numpy(), orc.inverse_diagonal()) < 1e-12
     assert rel_err((r - cells).cpu().numpy(), ref) < 1e-11
+
+
+@pytest.mark.parametrize("degree", [1, 2, 3])
+def test_first_apply_of_an_fp32_operator_can_be_captured(cuda, degree):
+    torch = cuda
+    orc, gop, _ = make_pair(torch, degree, (40, 3, 2), mode="cell", precision=1, seed=51)
+    x = torch.rand(orc.n_dofs, dtype=torch.float32, device="cuda", generator=torch.Generator(device="cuda").manual_seed(52))
+    y = torch.zeros_like(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gop.vmult(y, x)
+    for seed in (53, 54, 55):
+        x.copy_(torch.rand(orc.n_dofs, device="cuda", generator=torch.Generator(device="cuda").manual_seed(seed)))
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = y.clone()
+        gop.vmult(y, x)
+        torch.cuda.synchronize()
+        assert torch.equal(replayed, y)
+        assert rel_err(y.cpu().numpy(), orc.vmult(x.cpu().numpy().astype(np.float64))) < 1e-5

@@ -1,0 +1,47 @@
+"""What an operator asks of the HIP runtime, seen from a program that stands in for the runtime
+(tests/cxx/host_calls.cpp): no GPU is needed and nothing is launched."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def host_calls(tmp_path_factory):
+    """Runs the program; returns its lines after each argument that is a word, as (word, lines)."""
+    exe = str(tmp_path_factory.mktemp("host_calls") / "host_calls")
+    lib = os.path.join(ROOT, "meltpooldg_amd")
+    r = subprocess.run(["g++", "-std=c++17", "-O1", os.path.join(ROOT, "tests", "cxx", "host_calls.cpp"), "-o", exe, "-L" + lib,
+                        "-lmpdg_heat", "-Wl,-rpath," + lib, "-rdynamic"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+    def run(*words):
+        r = subprocess.run([exe] + [str(w) for w in words], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stdout + r.stderr
+        steps = []
+        for line in r.stdout.splitlines():
+            if line.split()[0] in ("alloc", "launch", "rc"):
+                steps[-1][1].append(line)
+            else:
+                steps.append((line, []))
+        return steps
+
+    return run
+
+
+def lines(step, word):
+    return [line for line in step[1] if line.startswith(word)]
+
+
+# the first apply of an operator can stand in a graph capture, where nothing may be allocated: also on the
+# meshes whose applies share no rows between columns of cells
+@pytest.mark.parametrize("degree", [1, 2, 3])
+@pytest.mark.parametrize("nc", [(64, 64, 64), (40, 3, 2), (5, 40, 3), (33, 17, 9)])
+def test_first_apply_allocates_nothing(host_calls, degree, nc):
+    for precision, apply in ((0, "vmult"), (0, "vmult_noalloc"), (1, "vmult_f32")):
+        create, first = host_calls("create", degree, *nc, precision, apply)
+        assert lines(create, "rc") == ["rc 0"]
+        assert not lines(first, "alloc")
+        assert lines(first, "launch") and lines(first, "rc") == ["rc 0"]
