@@ -60,8 +60,8 @@ typedef struct mpdg_heat_op mpdg_heat_op;
        (include/meltpooldg/core/operator_base.hpp:189-282) --- */
 /* Q1..Q3: also allocates the apply's scratch, the DoFs of the planes that workgroups share (0.1 to 0.4
    vectors on large meshes, up to 1.5 on small ones), so that no apply allocates it and the first one can be
-   captured; one device allocation, 25 to 60 us. Where that fails the first apply tries again. Q4: the
-   first apply allocates. */
+   captured; one device allocation, 25 to 60 us. Where that fails, or another device is current then, the
+   first apply allocates. Q4: the first apply allocates. */
 int mpdg_heat_op_create(const mpdg_heat_desc *desc, mpdg_heat_op **op);
 int mpdg_heat_op_destroy(mpdg_heat_op *op);
 long mpdg_heat_op_n_dofs(const mpdg_heat_op *op);
@@ -142,7 +142,8 @@ int mpdg_heat_op_vmult_f32(const mpdg_heat_op *op, float *dst, const float *src,
    counterpart in the reference: it is for callers that cannot allocate device memory (code
    under HIP graph capture, tight serving loops, harnesses that forbid it). Same result as
    mpdg_heat_op_vmult, bit for bit (same kernels). The apply's scratch is, for Q1..Q3, the
-   operator's own, allocated by mpdg_heat_op_create (MPDG_ERR_NOMEM when that had no room);
+   operator's own, allocated by mpdg_heat_op_create (MPDG_ERR_NOMEM when that had no room or another
+   device was current);
    for Q4, a fixed per-GPU array of 2^20 doubles (8 MiB). Meshes beyond a fixed maximum get
    MPDG_ERR_TOO_LARGE: more than 2^20 DoFs on the rows along x where four columns of cells
    meet (about 0.75 M for Q3 on 128^3 cells, 0.64 M for mapped Q3 on 96^3 cells, 0.27 M for

@@ -21,8 +21,26 @@ inline int dev_ok() { return hipGetLastError() == hipSuccess ? MPDG_OK : MPDG_ER
 // ===========================================================================
 // operator
 // ===========================================================================
+namespace {
+int current_device() {
+  int device = -1;
+  (void)hipGetDevice(&device);
+  return device;
+}
+}  // namespace
+
 int mpdg_heat_op::ensure_edge() const {
   const size_t n = precision == MPDG_FP32 ? apply_edge_elems(d32) : apply_edge_elems(d64);
+  const int device = current_device();
+  if (device != edge_device) {
+    // made before the caller selected the GPU that it runs on, whose kernels may not reach another's memory
+    edge64.release();
+    edge32.release();
+    d64.edge = nullptr;
+    d32.edge = nullptr;
+    d64.edge_elems = d32.edge_elems = 0;
+    edge_device = device;
+  }
   if (precision == MPDG_FP64) {
     MPDG_TRY(d64.degree < 4 ? edge64.resize(n) : edge64.resize_zeroed(n));
     d64.edge = edge64.get();
@@ -33,6 +51,11 @@ int mpdg_heat_op::ensure_edge() const {
     d32.edge_elems = n;
   }
   return MPDG_OK;
+}
+
+bool mpdg_heat_op::edge_ready() const {
+  const size_t n = apply_edge_elems(d64);
+  return n == 0 || (d64.edge_elems == n && edge_device == current_device());
 }
 
 int mpdg_heat_op::vmult_cells(double *dst, const double *src, hipStream_t s) const {
@@ -1390,7 +1413,7 @@ int mpdg_heat_op_vmult_noalloc(const mpdg_heat_op *op, double *dst, const double
       return MPDG_ERR_TOO_LARGE;
     if (op->d64.degree < 4) {
       // the operator's scratch, allocated when it was created
-      if (op->d64.edge_elems != apply_edge_elems(op->d64)) return MPDG_ERR_NOMEM;
+      if (!op->edge_ready()) return MPDG_ERR_NOMEM;
       MPDG_TRY(launch_apply<double>(op->d64, src, dst, s));
       if (op->d64.robin_mask) MPDG_TRY(launch_boundary(op->d64, 0, nullptr, dst, src, op->T_robin, s));
       return MPDG_OK;

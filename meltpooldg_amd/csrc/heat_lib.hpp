@@ -167,6 +167,7 @@ struct mpdg_heat_op {
   // apply scratch (OperatorData::edge)
   mutable mpdg::DeviceArray<double> edge64;
   mutable mpdg::DeviceArray<float> edge32;
+  mutable int edge_device = -1;  // the GPU it lies on
   // full Newton tangent (mpdg_heat_op_set_tangent): material, velocity, per-qp data at the bound T
   bool tangent = false;
   mpdg_heat_material mat{};
@@ -188,8 +189,9 @@ struct mpdg_heat_op {
 
   // mapped meshes with per-qp / k(T) conductivity: fold the conductivity into metric_k
   int refresh_metric_k(hipStream_t s) const;
-  // allocates and binds the apply's scratch where that is not done yet
+  // allocates and binds the apply's scratch where that is not done yet for the current device
   int ensure_edge() const;
+  bool edge_ready() const;  // FP64: it is
   long n_dofs() const { return d64.n_dofs; }
   long n_cells() const { return d64.n_cells; }
   int vmult(double *dst, const double *src, hipStream_t s) const;

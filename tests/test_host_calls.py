@@ -45,3 +45,22 @@ def test_first_apply_allocates_nothing(host_calls, degree, nc):
         assert lines(create, "rc") == ["rc 0"]
         assert not lines(first, "alloc")
         assert lines(first, "launch") and lines(first, "rc") == ["rc 0"]
+
+
+# an operator made before its caller selects the GPU that it runs on
+@pytest.mark.parametrize("degree,precision,apply", [(1, 0, "vmult"), (2, 1, "vmult_f32"), (3, 0, "vmult"), (3, 1, "vmult_f32")])
+def test_scratch_follows_the_device_of_the_apply(host_calls, degree, precision, apply):
+    create, _, there, again = host_calls("create", degree, 20, 9, 10, precision, "device", 1, apply, apply)
+    assert [line.split()[1] for line in lines(create, "alloc")] == ["0"]
+    assert [line.split()[1] for line in lines(there, "alloc")] == ["1"]
+    assert lines(there, "launch") and lines(there, "rc") == ["rc 0"]
+    assert not lines(again, "alloc") and lines(again, "launch") and lines(again, "rc") == ["rc 0"]
+
+
+def test_noalloc_refuses_scratch_of_another_device(host_calls):
+    _, _, there, _, back = host_calls("create", 2, 20, 9, 10, 0, "device", 1, "vmult_noalloc", "device", 0, "vmult_noalloc")
+    assert there[1] == ["rc -2"]
+    assert not lines(back, "alloc") and lines(back, "launch") and lines(back, "rc") == ["rc 0"]
+    # no planes are shared here: no scratch is needed
+    _, _, there = host_calls("create", 2, 3, 1, 2, 0, "device", 1, "vmult_noalloc")
+    assert lines(there, "launch") and lines(there, "rc") == ["rc 0"]
