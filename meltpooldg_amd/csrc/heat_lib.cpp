@@ -1399,6 +1399,7 @@ int mpdg_heat_op_vmult_noalloc(const mpdg_heat_op *op, double *dst, const double
   hipStream_t s = S(stream);
   if (op->tangent) {
     if (!op->td_bound) return MPDG_ERR_INVALID;
+    if (op->d64.degree < 4 && !op->edge_ready()) return MPDG_ERR_NOMEM;
     MPDG_TRY(launch_tangent_apply(op->d64, op->td.get(), op->vel, op->vfield, op->solid, src, dst, s));
   } else {
     if (op->d64.metric && op->d64.kappa_mode == KAPPA_LAW) {

@@ -2,6 +2,7 @@
 // precedence over the runtime's), allocates host memory for them and launches nothing. It prints what it is
 // told to do by its arguments and, in between, each call that matters to a caller:
 //   create DEGREE NX NY NZ PRECISION | device D | refuse BYTES (allocations of at least that many fail)
+//   tangent (of a material without transition, bound to a temperature)
 //   vmult | vmult_f32 | vmult_noalloc          prints "alloc DEVICE BYTES", "launch BLOCKS" and "rc CODE"
 #include <cstdio>
 #include <cstdlib>
@@ -82,6 +83,14 @@ int main(int argc, char **argv) {
       d.precision = (int)number();
       d.extent[0] = d.extent[1] = d.extent[2] = d.rho_cp = 1.0;
       std::printf("rc %d\n", mpdg_heat_op_create(&d, &op));
+    } else if (what == "tangent") {
+      mpdg_heat_material m{};
+      m.density[0] = m.specific_heat[0] = m.conductivity[0] = 1.0;
+      const double velocity[3] = {0.0, 0.0, 0.0};
+      (void)mpdg_heat_op_reset_time_increment(op, 1.0);
+      int rc = mpdg_heat_op_set_tangent(op, &m, 0, velocity);
+      if (rc == MPDG_OK) rc = mpdg_heat_op_bind_temperature(op, unused, unused, nullptr);
+      std::printf("rc %d\n", rc);
     } else if (what == "vmult") {
       std::printf("rc %d\n", mpdg_heat_op_vmult(op, unused, unused, nullptr));
     } else if (what == "vmult_f32") {

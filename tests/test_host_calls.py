@@ -64,3 +64,10 @@ def test_noalloc_refuses_scratch_of_another_device(host_calls):
     # no planes are shared here: no scratch is needed
     _, _, there = host_calls("create", 2, 3, 1, 2, 0, "device", 1, "vmult_noalloc")
     assert lines(there, "launch") and lines(there, "rc") == ["rc 0"]
+
+
+@pytest.mark.parametrize("degree", [1, 2, 3])
+def test_noalloc_of_a_tangent_without_scratch_is_out_of_memory(host_calls, degree):
+    _, create, _, tangent, apply = host_calls("refuse", 64, "create", degree, 20, 9, 10, 0, "refuse", 2 ** 40, "tangent", "vmult_noalloc")
+    assert create[1] == ["rc 0"] and lines(tangent, "rc") == ["rc 0"]
+    assert apply[1] == ["rc -2"]
