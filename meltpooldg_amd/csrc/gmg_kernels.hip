@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void coarse_matrix_kernel(CoarseTables t, int 
         const double b[3] = {t.G[qx][j0] * t.S[qy][j1] * t.S[qz][j2], t.S[qx][j0] * t.G[qy][j1] * t.S[qz][j2],
                              t.S[qx][j0] * t.S[qy][j1] * t.G[qz][j2]};
         if (metric) {
-          auto M = [&](int comp) -> double { return metric[metric_at(n1, nc0, cell, comp, qx, qy, qz)]; };
+          auto M = [&](int comp) -> double { return metric[metric_at(n1, nc0, ncells, cell, comp, qx, qy, qz)]; };
           const double g00 = M(1), g01 = M(2), g11 = M(3), g02 = M(4), g12 = M(5), g22 = M(6);
           const double gg = a[0] * (g00 * b[0] + g01 * b[1] + g02 * b[2]) +
                             a[1] * (g01 * b[0] + g11 * b[1] + g12 * b[2]) +

@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void diagonal_kernel(AuxTables<Number> t, int 
         Number c = Number(0);
         if (active) {
           if (MAPPED) {
-            const Number m = metric[metric_at(N1, nc0, cell, comp[term], b, a, qz)];
+            const Number m = metric[metric_at(N1, nc0, ncells, cell, comp[term], b, a, qz)];
             c = term == 0 ? cm * m : (term >= 4 ? Number(2) : Number(1)) * kk[qz] * m;
           } else {
             const Number W = t.w[qz] * t.w[a] * t.w[b];
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(256) void metric_kernel(AuxTables<double> t, int n1
   B[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
   const double jxw = fabs(det) * t.w[qx] * t.w[qy] * t.w[qz];
   auto g = [&](int a, int b) { return jxw * (B[a][0] * B[b][0] + B[a][1] * B[b][1] + B[a][2] * B[b][2]); };
-  auto M = [&](int comp) -> Number & { return metric[metric_at(n1, nc0, cell, comp, qx, qy, qz)]; };
+  auto M = [&](int comp) -> Number & { return metric[metric_at(n1, nc0, ncells, cell, comp, qx, qy, qz)]; };
   M(0) = (Number)jxw;
   M(1) = (Number)g(0, 0);
   M(2) = (Number)g(0, 1);
@@ -707,7 +707,7 @@ __global__ __launch_bounds__(256) void scale_metric_kernel(const Number *__restr
     const int qx = q % n1, qy = (q / n1) % n1, qz = q / (n1 * n1);
     const Number k = kq[c * nq + q];
     for (int comp = 0; comp < 7; ++comp) {
-      const long g = metric_at(n1, nc0, c, comp, qx, qy, qz);
+      const long g = metric_at(n1, nc0, ncells, c, comp, qx, qy, qz);
       out[g] = comp == 0 ? metric[g] : k * metric[g];
     }
   }

@@ -442,8 +442,17 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
   };
   // the lane's first point in the arrays with ncomp values per point (point_data_at)
   auto point_data = [&](const auto &A, int ncomp, int cxb, int cy) {
-    const long pencil = cxb / kNX + (long)((A.nc[0] + kNX - 1) / kNX) * (cy + (long)A.nc[1] * min(cz, A.nc[2] - 1));
-    return A.metric + (pencil * ncomp * NQ + min(l, K)) * kNX + min(c, A.nc[0] - 1 - cxb);
+    const long row = cy + (long)A.nc[1] * min(cz, A.nc[2] - 1);
+    const int full = (unsigned)A.nc[0] / kNX;
+    long block = row * full + (unsigned)cxb / kNX;
+    int at = min(l, K) * kNX + c;
+    if (cxb + kNX > A.nc[0]) {
+      const long t = row * ((unsigned)A.nc[0] % kNX);
+      const int place = (int)(t % kNX) + min(c, A.nc[0] - 1 - cxb);
+      block = (long)A.nc[1] * A.nc[2] * full + t / kNX;
+      at = (place / kNX * ncomp * NQ + min(l, K)) * kNX + place % kNX;
+    }
+    return A.metric + block * (ncomp * NQ * kNX) + at;
   };
   int parity = 0;
   for (int cy = cy0; cy < cy_end; ++cy) {
@@ -678,7 +687,7 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
           Number gx[N1][N1], gy[N1][N1];
           sweep_x<N1, false, false>(P.D, v, gx);
           sweep_y<N1, false, false>(P.D, v, gy);
-          const Number *M = point_data(P, kMetricComps, cxb, cy);
+          const Number *M = point_data(A, kMetricComps, cxb, cy);
           const bool idle = N1 == 3 && row == 3;
 #pragma unroll
           for (int j = 0; j < N1; ++j)
@@ -1335,8 +1344,10 @@ void tangent_points_kernel(const TangentPoints<N1> X, const double *__restrict__
       }
   }
   const bool mine = cxb + c < P.nc[0] && cz < P.nc[2] && l <= K;
-  const long pencil = cxb / kNX + (long)px * (cy + (long)P.nc[1] * cz);
-  double *const out = td + (pencil * kTangentCoeffs * NQ + l) * kNX + c;
+  long block = (unsigned)cxb / kNX + (long)((unsigned)P.nc[0] / kNX) * (cy + (long)P.nc[1] * cz);
+  int place = c;
+  if (cxb + kNX > P.nc[0]) block = point_block(P.nc[0], cy + (long)P.nc[1] * min(cz, P.nc[2] - 1), (long)P.nc[1] * P.nc[2], cx, place);
+  double *const out = td + (block * kTangentCoeffs * NQ + l) * kNX + place;
   auto put = [&](int comp, int j, int i, double x) {
     if (mine) out[(comp * NQ + (N1 * j + i) * N1) * kNX] = x;
   };

@@ -178,24 +178,41 @@ struct OperatorData {
   }
 };
 
-// Where component comp (of ncomp) of quadrature point q = (qx, qy, qz) of a cell lies in the per-point
-// arrays the library makes itself (the metric, the tangent's coefficients). Q1..Q3: [pencil of 16 cells
-// along x][comp][qy][qx][qz][cell of the pencil], so that each load of the apply's wavefront
-// (lane = 16 qz + cell) is contiguous (mapped Q3 96^3 FP64 apply: 0.82 ms; 2.4 ms with [cell][comp][q], where
-// every lane reads its own line); Q4, whose kernels give a lane consecutive qx: [cell][comp][q].
-__host__ __device__ __forceinline__ long point_data_at(int n1, int nc0, long cell, int ncomp, int comp, int qx, int qy, int qz) {
+// The per-point arrays the library makes itself (the metric, the tangent's coefficients). Q1..Q3: blocks of 16
+// cells, [comp][qy][qx][qz][cell of the block], so that each load of the apply's wavefront (lane = 16 qz + cell) is
+// contiguous (mapped Q3 96^3 FP64 apply: 0.82 ms; 2.4 ms with [cell][comp][q], where every lane reads its
+// own line). A block is a pencil of 16 cells along x; the cells that a row has beyond its full pencils follow, row
+// after row, in blocks of their own, so that no more than one block has room left (a pencil padded to 16
+// cells per row takes 16 times the memory for one cell along x and 1.9 times for 17). Q4, whose kernels give a
+// lane consecutive qx: [cell][comp][q].
+// Block and place in it of cell cx of a row (row = cy + nc1 cz, of rows)
+__host__ __device__ __forceinline__ long point_block(int nc0, long row, long rows, int cx, int &place) {
+  const int full = nc0 / 16, rest = nc0 % 16;
+  if (cx < 16 * full) {
+    place = cx % 16;
+    return row * full + cx / 16;
+  }
+  const long t = row * rest + cx - 16 * full;
+  place = (int)(t % 16);
+  return rows * full + t / 16;
+}
+// Where component comp (of ncomp) of quadrature point q = (qx, qy, qz) of a cell (of n_cells) lies
+__host__ __device__ __forceinline__ long point_data_at(int n1, int nc0, long n_cells, long cell, int ncomp, int comp, int qx, int qy,
+                                                       int qz) {
   const int nq = n1 * n1 * n1;
   if (n1 == 5) return (cell * ncomp + comp) * nq + qx + n1 * (qy + n1 * qz);
-  const long row = cell / nc0, cx = cell - row * nc0, pencil = row * ((nc0 + 15) / 16) + cx / 16;
-  return ((pencil * ncomp + comp) * nq + (qy * n1 + qx) * n1 + qz) * 16 + cx % 16;
+  const long row = cell / nc0;
+  int place;
+  const long block = point_block(nc0, row, n_cells / nc0, (int)(cell - row * nc0), place);
+  return ((block * ncomp + comp) * nq + (qy * n1 + qx) * n1 + qz) * 16 + place;
 }
 inline size_t point_data_elems(int n1, const int *nc, int ncomp) {
-  const size_t cells_x = n1 == 5 ? nc[0] : (nc[0] + 15) / 16 * 16;
-  return cells_x * nc[1] * nc[2] * ncomp * n1 * n1 * n1;
+  const size_t cells = (size_t)nc[0] * nc[1] * nc[2];
+  return (n1 == 5 ? cells : (cells + 15) / 16 * 16) * ncomp * n1 * n1 * n1;
 }
 constexpr int kMetricComps = 7;
-__host__ __device__ __forceinline__ long metric_at(int n1, int nc0, long cell, int comp, int qx, int qy, int qz) {
-  return point_data_at(n1, nc0, cell, kMetricComps, comp, qx, qy, qz);
+__host__ __device__ __forceinline__ long metric_at(int n1, int nc0, long n_cells, long cell, int comp, int qx, int qy, int qz) {
+  return point_data_at(n1, nc0, n_cells, cell, kMetricComps, comp, qx, qy, qz);
 }
 inline size_t metric_elems(int n1, const int *nc) { return point_data_elems(n1, nc, kMetricComps); }
 

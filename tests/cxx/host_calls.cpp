@@ -2,7 +2,7 @@
 // precedence over the runtime's), allocates host memory for them and launches nothing. It prints what it is
 // told to do by its arguments and, in between, each call that matters to a caller:
 //   create DEGREE NX NY NZ PRECISION | device D | refuse BYTES (allocations of at least that many fail)
-//   tangent (of a material without transition, bound to a temperature)
+//   tangent (of a material without transition, bound to a temperature) | mapping
 //   vmult | vmult_f32 | vmult_noalloc          prints "alloc DEVICE BYTES", "launch BLOCKS" and "rc CODE"
 #include <cstdio>
 #include <cstdlib>
@@ -91,6 +91,8 @@ int main(int argc, char **argv) {
       int rc = mpdg_heat_op_set_tangent(op, &m, 0, velocity);
       if (rc == MPDG_OK) rc = mpdg_heat_op_bind_temperature(op, unused, unused, nullptr);
       std::printf("rc %d\n", rc);
+    } else if (what == "mapping") {
+      std::printf("rc %d\n", mpdg_heat_op_set_mapping(op, unused));
     } else if (what == "vmult") {
       std::printf("rc %d\n", mpdg_heat_op_vmult(op, unused, unused, nullptr));
     } else if (what == "vmult_f32") {

@@ -596,3 +596,21 @@ def test_first_apply_of_an_fp32_operator_can_be_captured(cuda, degree):
         torch.cuda.synchronize()
         assert torch.equal(replayed, y)
         assert rel_err(y.cpu().numpy(), orc.vmult(x.cpu().numpy().astype(np.float64))) < 1e-5
+
+
+# cells beyond a row's full pencils of 16 share blocks of the metric with the next rows' (1, 5, 11, 15 of them here)
+@pytest.mark.parametrize("degree,nc,mode", [(1, (5, 7, 9), "cell"), (1, (31, 3, 5), "qp"), (2, (1, 6, 5), "const"),
+                                            (2, (21, 5, 3), "law"), (3, (11, 3, 5), "qp"), (3, (17, 9, 2), "cell")])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_mapped_at_row_remainders(cuda, degree, nc, mode, precision):
+    torch = cuda
+    orc, gop, _ = make_pair(torch, degree, nc, mode=mode, mapped=0.05, precision=precision, seed=61)
+    x = torch.tensor(np.random.default_rng(62).uniform(-1.0, 1.0, orc.n_dofs),
+                     dtype=torch.float64 if precision == 0 else torch.float32, device="cuda")
+    y, d = torch.full_like(x, float("nan")), torch.empty_like(x)
+    gop.vmult(y, x)
+    gop.compute_diagonal(d)
+    torch.cuda.synchronize()
+    tol = 1e-12 if precision == 0 else 1e-5
+    assert rel_err(y.cpu().numpy(), orc.vmult(x.cpu().numpy().astype(np.float64))) < tol
+    assert rel_err(d.cpu().numpy(), orc.diagonal()) < tol

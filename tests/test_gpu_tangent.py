@@ -228,3 +228,20 @@ def test_tangent_golden_norm_sequences(cuda, case):
         heat.solve(dt)
         norms.append(op.l2_norm(heat.solution()))
     assert ["%.5e" % v for v in norms] == ["%.5e" % v for v in TANGENT_GOLDEN[case]]
+
+
+# cells beyond a row's full pencils of 16 share blocks of the coefficients with the next rows'
+@pytest.mark.parametrize("degree,nc", [(1, (5, 6, 7)), (2, (21, 2, 5)), (2, (47, 3, 3)), (3, (11, 5, 2))])
+def test_tangent_at_row_remainders(cuda, degree, nc):
+    torch = cuda
+    import meltpooldg_amd as M
+    orc, op, T, T_old, Td, Tod = pair(torch, M, degree, nc, tuple(0.1 * n for n in nc), 0b000010, True, (0.2, -0.4, 0.1))
+    src = np.random.default_rng(7).uniform(-1, 1, orc.n_dofs)
+    dst = torch.full((orc.n_dofs,), float("nan"), dtype=torch.float64, device="cuda")
+    op.vmult(dst, torch.tensor(src, device="cuda"))
+    ref = orc.vmult(src, threads=1)
+    assert np.linalg.norm(dst.cpu().numpy() - ref) <= 1e-12 * np.linalg.norm(ref)
+    d = torch.empty_like(dst)
+    op.compute_diagonal(d)
+    ref = orc.diagonal()
+    assert np.linalg.norm(d.cpu().numpy() - ref) <= 1e-12 * np.linalg.norm(ref)

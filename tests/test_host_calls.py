@@ -71,3 +71,18 @@ def test_noalloc_of_a_tangent_without_scratch_is_out_of_memory(host_calls, degre
     _, create, _, tangent, apply = host_calls("refuse", 64, "create", degree, 20, 9, 10, 0, "refuse", 2 ** 40, "tangent", "vmult_noalloc")
     assert create[1] == ["rc 0"] and lines(tangent, "rc") == ["rc 0"]
     assert apply[1] == ["rc -2"]
+
+
+# the metric (7 values per point) and the tangent's coefficients (8) take no room for cells that are not there,
+# but for one block of 16 cells
+@pytest.mark.parametrize("degree", [1, 2, 3, 4])
+@pytest.mark.parametrize("nc", [(1, 9, 7), (17, 5, 6), (16, 2, 3), (31, 3, 1)])
+def test_point_data_is_not_padded(host_calls, degree, nc):
+    points = (degree + 1) ** 3
+    cells = nc[0] * nc[1] * nc[2]
+    blocks = cells if degree == 4 else (cells + 15) // 16 * 16
+    for precision, item in ((0, 8), (1, 4)):
+        _, mapping = host_calls("create", degree, *nc, precision, "mapping")
+        assert lines(mapping, "alloc") == ["alloc 0 %d" % (item * 7 * points * blocks)]
+    _, tangent = host_calls("create", degree, *nc, 0, "tangent")
+    assert lines(tangent, "alloc")[0] == "alloc 0 %d" % (8 * 8 * points * blocks)
