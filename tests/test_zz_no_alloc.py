@@ -82,3 +82,26 @@ def test_noalloc_refuses_meshes_beyond_its_scratch(cuda):
     g32 = M.HeatDiffuseMultiPhaseOperator(2, (4, 4, 4), precision=M.FP32)
     rc = lib.mpdg_heat_op_vmult_noalloc(g32.h, C.c_void_p(y.data_ptr()), C.c_void_p(x.data_ptr()), None)
     assert rc == -1
+
+
+# Q4, whose scratch is the fixed per-GPU array (Q1..Q3: the operator's own): several columns in y and z, so that
+# every call leaves sums in the array for the next mesh's
+Q4_CASES = [dict(degree=4, nc=(9, 14, 11), mode="qp", dirichlet=0, mapped=None, seed=35),
+            dict(degree=4, nc=(5, 9, 7), mode="cell", dirichlet=0b010110, mapped=None, seed=36),
+            dict(degree=4, nc=(6, 13, 8), mode="const", dirichlet=0, mapped=0.05, seed=37)]
+
+
+def test_noalloc_q4_reuses_the_array(cuda):
+    torch = cuda
+    pairs = [make_pair(torch, c["degree"], c["nc"], mode=c["mode"], dirichlet=c["dirichlet"], mapped=c["mapped"],
+                       seed=c["seed"]) for c in Q4_CASES]
+    xs = [torch.tensor(np.random.default_rng(45 + i).uniform(-1.0, 1.0, p[0].n_dofs), device="cuda")
+          for i, p in enumerate(pairs)]
+    for i in (0, 1, 0, 2, 1, 2, 0):
+        orc, gop, _ = pairs[i]
+        y = _noalloc(torch, gop, xs[i])
+        ref = _vmult(torch, gop, xs[i])
+        torch.cuda.synchronize()
+        # vmult and vmult_noalloc run the same kernels; the sums of a column arrive in one order
+        assert torch.equal(y, ref)
+        assert rel_err(y.cpu().numpy(), orc.vmult(xs[i].cpu().numpy())) < 1e-12
