@@ -614,3 +614,44 @@ def test_mapped_at_row_remainders(cuda, degree, nc, mode, precision):
     tol = 1e-12 if precision == 0 else 1e-5
     assert rel_err(y.cpu().numpy(), orc.vmult(x.cpu().numpy().astype(np.float64))) < tol
     assert rel_err(d.cpu().numpy(), orc.diagonal()) < tol
+
+
+def nan_reach(degree, nc):
+    """DoF grid with True on the cells around the vertex (15, 2, 4) of the mesh, and the vertex's place (z, y, x)."""
+    nd = [degree * n + 1 for n in nc]
+    at = (degree * 4, degree * 2, degree * 15)
+    want = np.zeros((nd[2], nd[1], nd[0]), dtype=bool)
+    want[tuple(slice(a - degree, a + degree + 1) for a in at)] = True
+    return want, at
+
+
+# pencils of 8 cells (Q1, Q2 with 20 cells along x, 8 along z) and of 16, FP32, mapped cells
+@pytest.mark.parametrize("degree,nc,mode,precision,mapped",
+                         [(1, (20, 5, 16), "qp", 0, None), (2, (20, 5, 8), "const", 1, None), (2, (20, 5, 8), "law", 0, None),
+                          (1, (18, 5, 9), "cell", 1, None), (2, (18, 5, 9), "qp", 1, None), (3, (18, 5, 9), "qp", 1, None),
+                          (3, (18, 5, 9), "cell", 1, None), (3, (18, 5, 9), "const", 0, None), (1, (18, 5, 9), "const", 0, 0.05),
+                          (2, (18, 5, 9), "cell", 0, 0.05), (3, (18, 5, 9), "qp", 0, 0.05), (2, (21, 5, 9), "const", 1, 0.05),
+                          (3, (18, 5, 9), "const", 1, 0.05)])
+def test_a_nan_of_the_source_stays_in_its_cells(cuda, degree, nc, mode, precision, mapped):
+    torch = cuda
+    _, gop, _ = make_pair(torch, degree, nc, mode=mode, precision=precision, mapped=mapped, seed=81)
+    want, at = nan_reach(degree, nc)
+    x = torch.zeros(want.shape, dtype=torch.float64 if precision == 0 else torch.float32, device="cuda")
+    x[at] = float("nan")
+    y = torch.empty_like(x)
+    gop.vmult(y.view(-1), x.view(-1))
+    assert np.array_equal(torch.isnan(y).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("field", ["T", "T_old", "q"])
+@pytest.mark.parametrize("degree,mode", [(1, "law"), (2, "qp"), (2, "law"), (3, "cell"), (3, "law")])
+def test_a_nan_of_the_residual_stays_in_its_cells(cuda, degree, mode, field):
+    torch = cuda
+    nc = (18, 5, 9)
+    _, gop, data = make_pair(torch, degree, nc, mode=mode, seed=83)
+    want, at = nan_reach(degree, nc)
+    f = {name: torch.ones(want.shape, dtype=torch.float64, device="cuda") for name in ("T", "T_old", "q")}
+    f[field][at] = float("nan")
+    r = torch.zeros(want.size, dtype=torch.float64, device="cuda")
+    gop.create_rhs(r, f["T"].view(-1), f["T_old"].view(-1), f["q"].view(-1))
+    assert np.array_equal(torch.isnan(r).view(want.shape).cpu().numpy(), want)

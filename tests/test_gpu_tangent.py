@@ -245,3 +245,31 @@ def test_tangent_at_row_remainders(cuda, degree, nc):
     op.compute_diagonal(d)
     ref = orc.diagonal()
     assert np.linalg.norm(d.cpu().numpy() - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("field", [False, True])
+@pytest.mark.parametrize("degree", [1, 2, 3])
+def test_a_nan_stays_in_its_cells(cuda, degree, field):
+    """Of the source: in the apply; of the bound temperature: in the apply and the diagonal."""
+    torch = cuda
+    import meltpooldg_amd as M
+    from tests.test_gpu_operator import nan_reach
+    nc = (18, 5, 9)
+    want, at = nan_reach(degree, nc)
+    orc, op, T, T_old, Td, Tod = pair(torch, M, degree, nc, tuple(0.1 * n for n in nc), 0, True, (0.2, -0.4, 0.1))
+    if field:
+        v = torch.tensor([0.2, -0.4, 0.1], dtype=torch.float64, device="cuda").repeat_interleave(op.n_dofs)
+        op.set_velocity_field(v)
+        op.bind_temperature(Td, Tod)
+    x, y = torch.zeros(want.shape, dtype=torch.float64, device="cuda"), torch.empty(want.size, dtype=torch.float64, device="cuda")
+    x[at] = float("nan")
+    op.vmult(y, x.view(-1))
+    assert np.array_equal(torch.isnan(y).view(want.shape).cpu().numpy(), want)
+    x[at] = 0.0
+    Tn = Td.clone()
+    Tn.view(want.shape)[at] = float("nan")
+    op.bind_temperature(Tn, Tod)
+    op.vmult(y, x.view(-1))
+    assert np.array_equal(torch.isnan(y).view(want.shape).cpu().numpy(), want)
+    op.compute_diagonal(y)
+    assert np.array_equal(torch.isnan(y).view(want.shape).cpu().numpy(), want)
