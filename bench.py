@@ -42,7 +42,7 @@ HBM_PEAK_GBS = 8000.0
 # the summaries with the commands are under profiles/ (heat_apply_*, heat_brick_*). Counters need their own
 # profiler runs, so the bench reports the profiled figure for these workloads and null for others.
 PROFILED_TRAFFIC = {(3, 128, "qp", False): 2.225e+09, (4, 96, "qp", False): 2.354e+09,
-                    (4, 96, "law", False): 2.308e+09, (3, 96, "const", True): 3.694e+09}
+                    (4, 96, "law", False): 2.279e+09, (3, 96, "const", True): 3.694e+09}
 # learned predictor: after PAUSE[0] consecutive steps whose learned guess loses the guess check, the
 # network is not evaluated for PAUSE[1] steps, then tried again
 PAUSE = (2, 8)

@@ -197,7 +197,11 @@ __device__ __forceinline__ bool reduce_to_last_block(double (&v)[NQ], double *pa
   if (threadIdx.x == 0) {
     // Exchanges whose results are used: the increment is issued after they were performed, in the memory that
     // all XCDs share. (A device-scope release would write back the L2's dirty lines, those of the kernel's
-    // own vectors among them, at the end of every workgroup.)
+    // own vectors among them, at the end of every workgroup; the statistics kernel of the network keeps the
+    // release: it writes no vectors.) The order rests on the hardware, not on C++, whose relaxed operations on
+    // two objects have none: a returned exchange has been performed, the wait for its value precedes the
+    // increment (s_waitcnt vmcnt(0) in between), and the last workgroup's loads bypass its L2 (sc1) and are
+    // issued after its own increment returned.
     unsigned long long done = 0;
 #pragma unroll
     for (int q = 0; q < NQ; ++q)

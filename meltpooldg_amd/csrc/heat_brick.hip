@@ -17,21 +17,23 @@
 //     of table r, and the backward pair transposes y registers against lane rows with
 //     v_permlane32/16_swap. Conductivity per point: twelve sweeps (collocated gradients on the Gauss
 //     points). One conductivity per Cartesian cell: seven sweeps with 1D mass and stiffness matrices.
-//   * Sums over cells, in FP64 at every precision and in a fixed order: along y the top row of
-//     a cell stays in registers for the next step; along x the last column moves one lane up
-//     (DPP row_shr:1); along z the top plane goes through LDS to the next pencil (one workgroup
-//     barrier per step).
+//   * Sums over a brick's cells, in FP64 at every precision and in a fixed order: along y the top row
+//     of a cell goes through LDS to the next step; along x the last column moves one lane up (DPP
+//     row_shr:1), and through LDS to the next pencil; along z the top plane goes through LDS to the next
+//     pencil (one workgroup barrier per step). A brick's sums are rounded to the operator's type where they
+//     are stored: in FP32 a DoF that bricks share (a corner: eight of them) is a sum of rounded parts.
 //   * A brick stores its DoFs except its upper x, y, z planes; those are shared with the next
 //     brick, which owns them, and go to a scratch array per class (planes, edges, corners).
 //     brick_fixup_kernel adds the classes to dst in a fixed order: no atomics and no zeroed
 //     rows, and vmult is bitwise repeatable.
 //
-// What bounds it: at Q3 FP64 with k per point, HBM (2.22 GB moved of 1.99 GB that the apply cannot do
-// without, 863 VALU instructions per 64 lanes and step) -- Q3 128^3, whole vmult: 0.663 ms for the column
-// kernel with LDS transposes, scatter and atomics it replaces, 0.566 ms here; elsewhere the VALU (Q3 128^3,
-// constant k: FP64 0.62 -> 0.43 ms, FP32 0.42 -> 0.28 ms; Q3 75 x 62 x 49 FP32 83.8 -> 45.4 us; mapped Q3 96^3
-// FP64, bound by the stored metric, 1.08 -> 0.78 ms). Q1 and Q2 on Cartesian cells run heat_cells_kernel
-// below, one lane per cell; here they run mapped, as residual and as the full tangent.
+// What bounds it: at Q3 FP64 with k per point, the latency of its loads at two wavefronts per SIMD (Q3 128^3:
+// 1.66 GB read and 0.56 GB written, which streams of their own take 0.39 ms for, in 0.52 to 0.56 ms; VALU 39 %
+// busy, 863 VALU instructions per 64 lanes and step) -- whole vmult: 0.663 ms for the column kernel with LDS
+// transposes, scatter and atomics it replaces, 0.566 ms here; elsewhere the VALU (Q3 128^3, constant k: FP64
+// 0.62 -> 0.43 ms, FP32 0.42 -> 0.28 ms; Q3 75 x 62 x 49 FP32 83.8 -> 45.4 us). Mapped Q3 96^3 FP64: 1.08 -> 0.78
+// ms, near what reading the stored metric takes (0.60 ms with the vectors). Q1 and Q2 on Cartesian cells run
+// heat_cells_kernel below, one lane per cell; here they run mapped, as residual and as the full tangent.
 #include "tangent.hpp"
 
 namespace mpdg {
@@ -301,10 +303,12 @@ __device__ __forceinline__ void lds_fence() {
 constexpr int KAPPA_TANGENT = 4;   // the full Newton tangent's coefficients instead of a conductivity
 constexpr int TANGENT_DIAGONAL = 5;  // ... and its diagonal: no source is read
 
-// Wavefronts per SIMD the register allocation targets: as many as fit without spills (Q3 FP64 needs
-// 226 VGPRs with per-point conductivity and 168 with one per cell, Q3 FP32 129 and 116; mapped cells
-// hold three fluxes: 195 and 129). Fewer wavefronts were slower even where the next step's source was
-// loaded ahead, and with three or four the loads need no such registers.
+// Wavefronts per SIMD the register allocation targets: as many as fit with few or no spilled VGPRs (Q3 FP64:
+// 228 VGPRs with per-point conductivity; 168 with one per cell, 6 to 11 of them spilled, in the residual too; Q2's
+// residual with a law 16 spilled at three; mapped cells hold three fluxes: Q3 FP64 215, FP32 123). Fewer
+// wavefronts were slower even where the next step's source was loaded ahead, and with three or four the
+// loads need no such registers. The 1D tables and sizes exceed the scalar registers: Q2 and Q3 keep 50 to 126
+// of them in VGPR lanes.
 template <int N1, typename Number, bool MAPPED, int KMODE> struct BrickOccupancy { static constexpr int W = 4; };
 template <bool M, int KM> struct BrickOccupancy<3, double, M, KM> { static constexpr int W = 3; };
 template <bool M, int KM> struct BrickOccupancy<4, double, M, KM> { static constexpr int W = 2; };
@@ -394,7 +398,8 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
   const long zoff = sz * (K * min(cz, P.nc[2] - 1) + min(l, K));
 
   // constrained planes that touch the brick (a z plane would otherwise be tested for in every step of every
-  // brick: Q1 283 x 252 x 459 FP32 526 -> 443 us)
+  // brick: residual of Q1 128^3 with k per point 88 -> 79 us, Q3 48^3 64 -> 61 us, Q3 75 x 62 x 49 FP32 apply
+  // 46.0 -> 44.4 us)
   int bmask = P.dmask;
   if (cx0 > 0) bmask &= ~1;
   if (cx_end < P.nc[0]) bmask &= ~2;
@@ -518,6 +523,8 @@ void heat_brick_kernel(const BrickArgs<Number, N1> P, const Number *__restrict__
           for (int m = 0; m < NLD; ++m) kraw[m] = p[min((long)(64 * m + lane), left - 1)];
         }
       } else if (KMODE == KAPPA_QP) {
+        // (Q1 past the caches: residual of 160 x 170 x 150, whose k exceeds them, 134 -> 127 us; of 128^3, whose
+        // k a repeated call finds there, 72 -> 80 us)
         const Number *p = A.kappa_arr + cell * NQ + N1 * N1 * min(l, K);
 #pragma unroll
         for (int j = 0; j < N1; ++j)
@@ -1013,7 +1020,8 @@ __device__ __forceinline__ double from_lane(double x, int lane) {
 // A whole cell per lane: a wavefront (= workgroup) holds LX x 64 / LX cells (x, z) and marches along y, pencils of
 // LX cells side by side along x done one after the other. All sweeps are register-local: per 64 cells Q2
 // takes half the VALU instructions of the kernel above, whose lane rows hold four planes, and there is no
-// barrier. What bounds it: the VALU, at two or three wavefronts per SIMD (Q2 FP64: 230 registers). Against the
+// barrier. What bounds it: the VALU, at few wavefronts per SIMD (Q2 FP64: two with one k per cell, 235 registers;
+// one with k per point or a law, 320 and 346; Q2 FP32 two or three; Q1 FP64 two to four, FP32 four). Against the
 // kernel above with these degrees: Q2 100^3 k per point FP64 178 -> 140 us, FP32 126 -> 79 us (101 us for a
 // kernel with LDS transposes between the sweeps), with a law FP32 196 -> 118 us (136), Q2 64^3 one k per cell
 // FP32 29 -> 24 us, Q1 112 x 116 x 132 k per point FP32 47 -> 33 us (40). Mapped cells, the residual and the
@@ -1596,10 +1604,12 @@ int launch_brick_tangent_data_n1(const OperatorData<double> &op, double dt, cons
 }  // namespace
 
 // Long bricks share fewer planes and set their tables up less often; short ones give every CU work, and end
-// the launch evenly. Taken is the shape with the least modelled time, in steps of one CU: full rounds of the
-// workgroups that are resident at once, the rest (no faster than the latency of one workgroup, which shows
-// below `latency` per CU), start-up, and the sums of the shared planes (of the x planes, which are strided,
-// separately). Measured over 28 meshes and kernels: 1.6% above the best shape on average (at most 15%); about
+// the launch evenly. Taken is the shape with the least modelled time, in steps of one CU: full rounds of
+// `resident` workgroups per CU, the rest (no faster than the latency of one workgroup, which shows below
+// `latency` per CU), start-up, and the sums of the shared planes (of the x planes, which are strided,
+// separately). The constants are fitted to measured times, one set per degree for all its kernels: `resident` is
+// not what the compiler lets a CU hold (Q3 FP64 with k per point two workgroups, Q2 FP64 cells with k per point
+// four wavefronts). Measured over 28 meshes and kernels: 1.6% above the best shape on average (at most 15%); about
 // 2048 workgroups for every mesh: 5.7% (24%) (Q3 75 x 62 x 49 FP32 49.6 -> 45.4 us, mapped Q3 96^3 FP64
 // 809 -> 781 us, Q2 and Q3 64^3 and 128^3 the same shapes); one cell per lane: 24 meshes, 2.5% (9%). It depends
 // on the mesh only, so every apply of a mesh sums in the same order.

@@ -15,7 +15,7 @@ enum KappaMode { KAPPA_CONST = MPDG_KAPPA_CONST, KAPPA_QP = MPDG_KAPPA_QP, KAPPA
 enum LawId { LAW_TANH = MPDG_LAW_TANH, LAW_MUSHY = MPDG_LAW_MUSHY };
 
 // tanh |x| = -E / (E + 2) with E = e^y - 1 = 2^n (e^r - 1) + (2^n - 1), y = -2 |x|, r = y - n ln 2 (ln 2 in two
-// parts, e^r - 1 by its Taylor series on |r| <= ln 2 / 2): small x keep their relative accuracy, and the
+// parts after Cody and Waite, e^r - 1 by its Taylor series on |r| <= ln 2 / 2): small x keep their relative accuracy, and the
 // rounding errors of e^r - 1, E and E + 2 are carried into the quotient's correction. Largest error over 4M
 // arguments |x| <= 25, in units of 2^-53 (2^-24) of the result: 1.16 (FP32 1.4), the device library's 1.34
 // (2.33). The law is evaluated at every point of every apply, and the library's tanh and the division by

@@ -16,7 +16,7 @@
 // Coefficients a problem does not have (no velocity, no solidification) are neither written
 // nor read. Q1..Q3: the coefficients and the apply have the lane layout of heat_brick.hip, one launch each
 // and the sums of shared planes (bind and apply of Q2 70 x 50 x 33 with solidification and a constant
-// velocity: 195 us with eight coloured launches, 135 us so). The kernels below are for Q4 and for the residual: cell-local sum factorization with one
+// velocity: 195 us with eight coloured launches, 121 us so). The kernels below are for Q4 and for the residual: cell-local sum factorization with one
 // thread per line of the cell's N1^3 tensor (N1^2 threads per cell) and LDS transposes between
 // the directions. A block holds a segment of an x-row of cells; it loads and stores its DoFs as
 // N1^2 lines along x with consecutive lanes on consecutive addresses, sums the shared x-faces in

@@ -231,8 +231,9 @@ def test_robin_faces_and_flux_are_bitwise_repeatable(cuda):
             assert np.array_equal(a, b)
 
 
-# Meshes with 64 columns of chunks (a multiple of the 8 XCDs): the launch then gives each XCD
-# a contiguous range of columns, a path the smaller meshes above do not take.
+# Meshes with 64 columns of Q4 chunks (a multiple of the 8 XCDs): the launch then gives each XCD
+# a contiguous range of columns, a path the smaller meshes above do not take. Q1..Q3 give each XCD a
+# contiguous range of bricks on every mesh.
 XCD_CASES = [(1, (8, 32, 32), "const", 0, 0), (2, (14, 24, 16), "qp", 0, 0), (3, (8, 32, 16), "qp", 0b000101, 0),
              (4, (4, 32, 24), "law", 0, 0), (3, (8, 32, 16), "cell", 0, 1), (3, (8, 32, 16), "const", 0b100000, 1),
              (4, (12, 16, 16), "qp", 0, 1)]
@@ -308,9 +309,9 @@ def test_vmult_mapped_xcd_column_launch_matches_oracle(cuda, degree, nc, mode, p
     assert rel_err(y.cpu().numpy(), ref) < (1e-12 if precision == 0 else 1e-5)
 
 
-# Meshes longer than one chunk along x that are no multiple of it, with ragged y/z columns: the
-# x-face carried in LDS between chunks, for every chunk shape (FP64 Q3 8x4x2, FP32 Q3 16x2x2,
-# mapped Q3 16x2x2, FP64 Q4 4x4x3, FP32 Q4 12x2x2, FP64 Q2 14x3x2).
+# Meshes longer than one chunk along x that are no multiple of it, with ragged y/z columns: for Q4 the
+# x-face carried in LDS between chunks (FP64 4x4x3, FP32 12x2x2). Q2 and Q3 have several bricks of one
+# pencil along x here; the x plane that a brick's pencils carry is tested in test_gpu_bricks.py.
 WIDE_CASES = [(3, (19, 5, 3), "qp", 0, None), (3, (37, 5, 3), "const", 1, None), (3, (37, 5, 3), "qp", 1, None),
               (3, (37, 5, 3), "law", 1, None), (3, (35, 4, 5), "const", 0, 0.05), (3, (35, 4, 5), "qp", 0, 0.05),
               (3, (35, 4, 5), "const", 1, 0.05), (4, (9, 5, 4), "qp", 0, None), (4, (27, 3, 5), "const", 1, None),
@@ -438,7 +439,8 @@ def test_node_coordinates_match_the_oracle_mapping(cuda, degree, nc, amp):
 
 
 # edges of the apply's bricks: pencils of 16 cells along x (one, two, an odd number; ragged), 4 cells
-# along z (Q1: 8), one or several steps along y and pencils per brick, one brick in a direction
+# along z (Q1: 8), one brick in a direction. Nearly all have bricks of one pencil and one step along y; several
+# of either are tested in test_gpu_bricks.py
 BRICK_CASES = [(1, (1, 1, 1), "const", 0, 0), (1, (15, 2, 8), "cell", 0, 0b100001), (1, (17, 3, 9), "qp", 0, 0),
                (2, (16, 4, 4), "cell", 0, 0b001100), (2, (33, 5, 5), "qp", 1, 0), (2, (31, 6, 3), "law", 0, 0b010010),
                (3, (16, 3, 4), "qp", 0, 0), (3, (47, 2, 5), "cell", 1, 0b111111), (3, (1, 9, 7), "qp", 1, 0b000100),

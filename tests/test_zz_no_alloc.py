@@ -1,10 +1,10 @@
 """mpdg_heat_op_vmult_noalloc, the apply that allocates nothing, against mpdg_heat_op_vmult.
 
-Both are called through the C ABI (ctypes). The no-allocation variant runs the same kernels
-with the apply's scratch taken from a fixed per-GPU device array, so its result must equal
-vmult's bit for bit, and the oracle's to the 1e-12 bar of every FP64 apply. Two calls in a
-row, the second on a smaller mesh, then the first mesh again; a mesh beyond the array's
-maximum is refused before anything is launched.
+Both are called through the C ABI (ctypes). The no-allocation variant runs the same kernels, with the
+operator's own scratch for Q1..Q3 and a fixed per-GPU device array for Q4, so its result must equal
+vmult's bit for bit, and the oracle's to the 1e-12 bar of every FP64 apply. Calls alternate between
+meshes, so that one meets what another left in the array; a mesh beyond the fixed maximum is refused
+before anything is launched.
 """
 import ctypes as C
 
